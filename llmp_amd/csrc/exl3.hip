@@ -657,6 +657,10 @@ __global__ __launch_bounds__(kProductWaves * 64) void ProductKernel(const Produc
             Hadamard128(a, b, lane);
             a *= kHadamardScale;
             b *= kHadamardScale;
+            // Rounded to F32 here, as the input transform's launch rounds it: a product and a conversion that the
+            // compiler sees together become one instruction that rounds once, to F16.
+            LLMP_TIE(a);
+            LLMP_TIE(b);
             const uint32_t packed = FloatToHalfBits(a) | (FloatToHalfBits(b) << 16);
             LdsWrite4(LdsAddress(operand) + static_cast<uint32_t>(t * 256 + 4 * lane), packed);
             if (block == 0) *reinterpret_cast<uint32_t*>(a_had + static_cast<int64_t>(t) * k + at) = packed;

@@ -143,6 +143,22 @@ def test_linear_rows_are_independent_and_f16_output_rounds_once(device):
     assert np.array_equal(half.view(np.uint16), full.astype(np.float16).view(np.uint16))
 
 
+def test_a_rows_transformed_input_is_the_same_bits_alone(device):
+    """Up to four rows the product transforms its input itself: the same F32 roundings as the input transform's own
+    launch, on inputs where rounding once, straight to F16, gives another value."""
+    k, n, bits = 1024, 128, 4
+    trellis, suh, svh = synth.exl3_weights(k, n, bits, 84)
+    args = (dev(trellis, device), halves(suh, device), halves(svh, device), k, n, bits, ops.EXL3_3INST)
+    x = halves(synth.rng(5).standard_normal((16, k)).astype(np.float16), device)
+    keep = {}
+    full = ops.exl3_linear(*args, x, keep=keep)
+    together = keep["a_had"]
+    for r in range(16):
+        alone = ops.exl3_linear(*args, x[r:r + 1], keep=keep)
+        assert torch.equal(keep["a_had"][0].view(torch.int16), together[r].view(torch.int16)), r
+        assert torch.equal(alone[0].view(torch.int32), full[r].view(torch.int32)), r
+
+
 @pytest.mark.parametrize("m", [17, 40, 144])
 def test_linear_of_more_than_sixteen_rows_runs_in_passes(device, m):
     """The packed path is upstream's choice through 144 rows (src/kernels/exl3/validate.h:254-256 of the
