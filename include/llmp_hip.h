@@ -426,13 +426,14 @@ int llmp_hip_exl3_hadamard(const void* x, void* y, const void* scale, int rows, 
                            int input_scale, void* stream);
 
 /* The packed linear: LinearOperands of validate.h:118-131 and PackedGemvLinear / PackedGemmLinear of
- * src/kernels/exl3/linear.h:47-54, 1 to 65536 rows (validate.h:76) in passes of sixteen, each pass streaming
+ * src/kernels/exl3/linear.h:47-54, 1 to 65536 rows (validate.h:76) in passes of sixteen, or of up to 144 (80
+ * above five bits a value) where `scratch` has llmp_hip_exl3_linear_wide_scratch bytes, each pass streaming
  * the weights once (upstream's choice, validate.h:254-256, is this path through 144 rows and the
- * reconstruction above, which is not built: a caller with more rows pays a pass every sixteen). x (m x k F16)
+ * reconstruction above); the results are the same bits either way. x (m x k F16)
  * into y (m x n, F16 or F32); a_had is the caller's m x k F16 scratch for the transformed input, which the
  * launches write as they compute it. `scratch` (llmp_hip_exl3_linear_scratch bytes, 8-byte aligned: one pass's,
  * shared by the passes in stream order) takes the place of the reference's lock area: the K slices' partial
- * sums, added in slice order. Two launches a pass are queued (three above four rows: the input transform is
+ * sums, added in slice order (and, of the wide size, the transformed rows in the product's order). Two launches a pass are queued (three above four rows: the input transform is
  * then a launch of its own); a failure after the first is reported as a fault (negative). */
 typedef struct llmp_exl3_linear {
   llmp_exl3_weights weights;
@@ -443,6 +444,7 @@ typedef struct llmp_exl3_linear {
   int m;
 } llmp_exl3_linear;
 size_t llmp_hip_exl3_linear_scratch(const llmp_exl3_linear* op);
+size_t llmp_hip_exl3_linear_wide_scratch(const llmp_exl3_linear* op);
 int llmp_hip_exl3_linear(const llmp_exl3_linear* op, void* scratch, size_t scratch_bytes, void* stream);
 
 /* The same linear for callers that cannot allocate or bring a workspace (code under HIP graph capture, tight
@@ -486,8 +488,8 @@ int llmp_hip_exl3_linear_reconstructed(const llmp_exl3_linear* op, void* w, size
  * first linear's rows, then the second's); a_had is 2 x m x k F16 (validate.cc:257-260), each
  * linear's own transformed input. The reference's three pointer tables have no counterpart:
  * the launches carry the six addresses. Same launches as llmp_hip_exl3_linear, both linears in
- * each (one linear after the other where their codebooks differ), in the same passes of sixteen rows;
- * `scratch` is llmp_hip_exl3_multi_linear_scratch bytes. */
+ * each (one linear after the other where their codebooks differ), in the same passes;
+ * `scratch` is llmp_hip_exl3_multi_linear_scratch bytes, or the wide size for passes of more than sixteen rows. */
 typedef struct llmp_exl3_multi_linear {
   llmp_exl3_weights first;
   llmp_exl3_weights second;
@@ -498,6 +500,7 @@ typedef struct llmp_exl3_multi_linear {
   int m;
 } llmp_exl3_multi_linear;
 size_t llmp_hip_exl3_multi_linear_scratch(const llmp_exl3_multi_linear* op);
+size_t llmp_hip_exl3_multi_linear_wide_scratch(const llmp_exl3_multi_linear* op);
 int llmp_hip_exl3_multi_linear(const llmp_exl3_multi_linear* op, void* scratch, size_t scratch_bytes, void* stream);
 
 /* ---------------------------------------------------------------- llmp.decode.vector

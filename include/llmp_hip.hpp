@@ -340,7 +340,13 @@ inline std::size_t ScratchBytes(const LinearOperands& o) {
   const llmp_exl3_linear abi = ToAbi(o);
   return llmp_hip_exl3_linear_scratch(&abi);
 }
-// PackedGemvLinear / PackedGemmLinear of src/kernels/exl3/linear.h:47-54, 1 to 65536 rows in passes of sixteen.
+// The bytes with which more than sixteen rows go in passes of up to 144.
+inline std::size_t WideScratchBytes(const LinearOperands& o) {
+  const llmp_exl3_linear abi = ToAbi(o);
+  return llmp_hip_exl3_linear_wide_scratch(&abi);
+}
+// PackedGemvLinear / PackedGemmLinear of src/kernels/exl3/linear.h:47-54, 1 to 65536 rows in passes of sixteen
+// (up to 144 where the scratch has WideScratchBytes).
 // UpstreamPath of src/kernels/exl3/validate.h:254-256: the packed path through 144 rows (the reconstruction paths
 // it names above that are not built here; the packed path still takes those rows).
 enum class LinearPath : std::uint8_t { kPacked, kReconstruct, kReconstructFused };

@@ -162,6 +162,7 @@ SYMBOLS = {
     "llmp_hip_exl3_linear_reconstructed": (_int, [C.POINTER(Exl3Linear), _vp, C.c_size_t, _int, _int, _vp]),
     "llmp_hip_exl3_hadamard": (_int, [_vp, _vp, _vp, _int, _int, _int, _int, _vp]),
     "llmp_hip_exl3_linear_scratch": (C.c_size_t, [C.POINTER(Exl3Linear)]),
+    "llmp_hip_exl3_linear_wide_scratch": (C.c_size_t, [C.POINTER(Exl3Linear)]),
     "llmp_hip_exl3_linear": (_int, [C.POINTER(Exl3Linear), _vp, C.c_size_t, _vp]),
     "llmp_hip_exl3_linear_static": (_int, [C.POINTER(Exl3Linear), _vp]),
     "llmp_hip_exl3_linear_static_prepare": (_int, [C.POINTER(Exl3Linear)]),
@@ -177,6 +178,7 @@ SYMBOLS = {
     "llmp_hip_decode_matrix": (_int, [_int, C.POINTER(DecodeOperand), C.c_uint64, C.c_uint64, _vp, C.c_uint64,
                                       C.c_uint64, _vp, C.c_uint64, _int, _vp]),
     "llmp_hip_exl3_multi_linear_scratch": (C.c_size_t, [C.POINTER(Exl3MultiLinear)]),
+    "llmp_hip_exl3_multi_linear_wide_scratch": (C.c_size_t, [C.POINTER(Exl3MultiLinear)]),
     "llmp_hip_exl3_multi_linear": (_int, [C.POINTER(Exl3MultiLinear), _vp, C.c_size_t, _vp]),
 }
 

@@ -47,6 +47,7 @@ constexpr float kHadamardScale = 0.088388347648f;  // validate.h:64
 typedef __attribute__((address_space(3))) void* LdsPointer;
 typedef const __attribute__((address_space(1))) void* GlobalPointer;
 typedef _Float16 Half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 Half8 __attribute__((ext_vector_type(8)));
 typedef float V4f __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------ codebooks
@@ -241,14 +242,17 @@ __device__ __forceinline__ void Hadamard128Rows(float (&x)[8], const float (&sig
 // y = f(H(x * in_scale)) * r * out_scale over each 128 block of each row; grid (rows, columns
 // / 128), a wave a block. X / Y: 0 F16, 1 F32. `slices` partial inputs are added in order first.
 // One or two transforms a launch (grid z): a linear's, or the two of a gate/up pair.
+// An F16 result is stored a second time, in the order in which the product of many rows reads its operand (see
+// WideProductKernel), where `operand` is given.
 struct HadamardSides {
   const void* x[2];
   void* y[2];
   const uint16_t* in_scale[2];
   const uint16_t* out_scale[2];
+  uint32_t* operand[2];
 };
 inline HadamardSides OneSide(const void* x, void* y, const uint16_t* in_scale, const uint16_t* out_scale) {
-  return HadamardSides{{x, x}, {y, y}, {in_scale, in_scale}, {out_scale, out_scale}};
+  return HadamardSides{{x, x}, {y, y}, {in_scale, in_scale}, {out_scale, out_scale}, {nullptr, nullptr}};
 }
 
 template <int X, int Y>
@@ -292,7 +296,15 @@ __global__ __launch_bounds__(64) void HadamardKernel(const HadamardSides sides, 
     b *= HalfBitsToFloat(s >> 16);
   }
   if constexpr (Y == 0) {
-    *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(y) + at) = FloatToHalfBits(a) | (FloatToHalfBits(b) << 16);
+    const uint32_t packed = FloatToHalfBits(a) | (FloatToHalfBits(b) << 16);
+    *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(y) + at) = packed;
+    if (sides.operand[blockIdx.z] != nullptr) {
+      // Values c and c + 1 of 32 inputs: the K step of sixteen they are of, the lane group and the half of its four.
+      const int row = blockIdx.x, pair = c >> 5, step = (c >> 4) & 1, half = (c >> 3) & 1, g = (c & 7) >> 1;
+      const int tiles = (gridDim.x + 15) / 16;
+      const int64_t chunk = static_cast<int64_t>(pair) * tiles + (row >> 4);
+      sides.operand[blockIdx.z][(chunk * 64 + g * 16 + (row & 15)) * 4 + 2 * step + half] = packed;
+    }
   } else {
     *reinterpret_cast<float2*>(static_cast<float*>(y) + at) = make_float2(a, b);
   }
@@ -613,11 +625,12 @@ __global__ __launch_bounds__(kProductWaves * 64) void ProductKernel(const Produc
   const uint16_t* my_row = x + static_cast<int64_t>(min(p.n, m - 1)) * k + 2 * p.g;
 
   if (first < last) {
-    // The ring runs kRingDepth - 1 steps ahead of the words read, the words one step ahead of the decode. Every
-    // step asks for the same loads in the same order (the next step's two activation words, then a stage of the
-    // ring; with kFused the next block's activations in place of the words), so that a wait can count them.
+    // The ring runs kRingDepth - 1 steps ahead of the words read, the words one step ahead of the decode. Every pair of
+    // steps asks for the same loads in the same order (a stage of the ring a step, then the next pair's four activation
+    // words; with kFused the next block's activations in place of the words), so that a wait can count them.
     uint32_t words[2][8][kWords];
-    uint32_t xa[2] = {0, 0}, xb[2] = {0, 0};  // a step's activation words (unfused: from global memory)
+    uint2 even_w[8], even_x;                  // the pair's first step, decoded: one product takes both steps' K
+    uint32_t xq[4];                           // a pair of steps' activation words (unfused: from global memory)
     uint32_t held[kFusedRows + 1];             // the next block's scales and activations (fused)
     auto ask_block = [&](int step) {           // of K step `step`'s 128 block
       const int at = min(step >> 3, k / 128 - 1) * 128 + 2 * lane;
@@ -625,15 +638,16 @@ __global__ __launch_bounds__(kProductWaves * 64) void ProductKernel(const Produc
 #pragma unroll
       for (int t = 0; t < kFusedRows; ++t) held[1 + t] = GlobalLoad4(x + static_cast<int64_t>(min(t, m - 1)) * k + at);
     };
-    if constexpr (kFused) {
-      ask_block(first);
-    } else {
-      xa[0] = GlobalLoad4(my_row + first * 16);
-      xb[0] = GlobalLoad4(my_row + first * 16 + 8);
-    }
+    auto ask_pair = [&](int step) {
+      const uint16_t* at = my_row + min(step, last - 2) * 16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xq[i] = GlobalLoad4(at + 8 * i);
+    };
+    if constexpr (kFused) ask_block(first);
 #pragma unroll
     for (int s = 0; s < kRingDepth - 1; ++s) fetch(first + s);
-    LoadsWaited<kLoads*(kRingDepth - 2)>();
+    if constexpr (!kFused) ask_pair(first);  // (behind the stages, where a later pair's are: the waits count on it)
+    LoadsWaited<kLoads*(kRingDepth - 2) + (kFused ? 0 : 4)>();
     ask(first, words[0]);
     auto one = [&](int step, int parity) {
       uint32_t (&mine)[8][kWords] = words[parity];
@@ -675,41 +689,50 @@ __global__ __launch_bounds__(kProductWaves * 64) void ProductKernel(const Produc
         const uint32_t at = my_operand + static_cast<uint32_t>((step & 7) * 32);
         x01 = LdsRead4<0>(at);
         x89 = LdsRead4<16>(at);
-      } else {
-        xa[parity ^ 1] = GlobalLoad4(my_row + min(step + 1, last - 1) * 16);
-        xb[parity ^ 1] = GlobalLoad4(my_row + min(step + 1, last - 1) * 16 + 8);
       }
-      // The ring's next stage asked for; the stage after this step's has landed (and this step's activation
-      // words): its words asked for, and this step's words (asked for a step ago) decoded while those come.
+      // The ring's next stage asked for; the stage after this step's has landed (at the pair's second step, its
+      // activation words too, which were asked for ahead of the last two stages): its words asked for, and this step's
+      // words (asked for a step ago) decoded while those come.
       fetch(step + kRingDepth - 1);
-      LoadsWaited<kLoads*(kRingDepth - 2) + (kFused ? 0 : 2)>();
+      if (kFused || parity == 1) {
+        LoadsWaited<kLoads*(kRingDepth - 2)>();
+      } else {
+        LoadsWaited<kLoads*(kRingDepth - 2) + 4>();
+      }
       LdsWaited();
       landed(mine);
       if constexpr (kFused) {
         LLMP_TIE(x01);
         LLMP_TIE(x89);
-      } else {
-        LLMP_TIE(xa[parity]);
-        LLMP_TIE(xb[parity]);
-        x01 = xa[parity], x89 = xb[parity];
+      } else if (parity == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) LLMP_TIE(xq[i]);
+        x01 = xq[2], x89 = xq[3];
       }
       ask(step + 1, next);
-      if (p.n >= m) x01 = 0, x89 = 0;
-      Half4 xv;
-      xv[0] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(x01 & 0xFFFFu));
-      xv[1] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(x01 >> 16));
-      xv[2] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(x89 & 0xFFFFu));
-      xv[3] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(x89 >> 16));
+      // (A row of the operand past the tokens is the last token's again: its sums are never stored.)
+      if (!kFused && parity == 1) even_x = make_uint2(xq[0], xq[1]);
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
         const Half4 wv = DecodeWindows<CB, BITS>(windows, mine[t]);
-        // D[token][n] += sum_j xv[token][j] wv[j][n]: first operand rows are tokens.
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(xv, wv, acc[t], 0, 0, 0);
+        const uint2 packed = __builtin_bit_cast(uint2, wv);
+        if (parity == 0) {
+          even_w[t] = packed;
+          LLMP_TIE(even_w[t].x);  // decoded here: left to itself the compiler keeps the states till the pair's second step
+          LLMP_TIE(even_w[t].y);
+        } else {
+          // D[token][n] += sum_j x[token][j] w[j][n]: first operand rows are tokens.
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(Half8, make_uint4(even_x.x, even_x.y, x01, x89)),
+                                                          __builtin_bit_cast(Half8, make_uint4(even_w[t].x, even_w[t].y, packed.x, packed.y)),
+                                                          acc[t], 0, 0, 0);
+        }
       }
+      if (kFused && parity == 0) even_x = make_uint2(x01, x89);
+      if (!kFused && parity == 1) ask_pair(step + 1);
     };
-    for (int step = first; step < last; step += 2) {
+    for (int step = first; step < last; step += 2) {  // (a wave's steps are whole 128 blocks: eight steps each)
       one(step, 0);
-      if (step + 1 < last) one(step + 1, 1);
+      one(step + 1, 1);
     }
     LdsWaited();  // the words asked for past the end
     LoadsWaited<0>();
@@ -735,6 +758,168 @@ __global__ __launch_bounds__(kProductWaves * 64) void ProductKernel(const Produc
     const int tq = e >> 6, l = e & 63;
     const int row = 4 * (l >> 4) + (tq & 3);
     if (row < m) out[static_cast<int64_t>(row) * n + (tq >> 2) * 16 + (l & 15)] = total;
+  }
+}
+
+// The same product for up to 16 TILES rows a pass (17 rows and more), each weight decoded once for all of them. What
+// bounds it is the decode's vector operations, as in the product of sixteen rows; a further sixteen rows cost one
+// matrix instruction of 16 cycles for the 200 cycles in which two tiles are decoded, where a pass of their own costs
+// the whole decode again (the linear of 4096 x 14336, four bits, at 77 rows: 112 us in five passes, 41.7 in one).
+// Grid (n / 64, outer slices), eight waves a workgroup as there, each its own K range in the same order, so that a
+// row's sums are bit for bit those of the sixteen-row product. A wave takes 64 columns, not 128: sixteen sums a lane
+// for every sixteen rows, which leaves registers for 144 rows at two waves a SIMD. A step is 32 of K (two tiles of
+// each of four columns). The rows' operand comes from L2 in the order of the lanes (chunk (K / 32, rows / 16) of 64
+// lanes by eight values, written by the input transform): sixteen bytes a lane, a KB an instruction, where the rows
+// as they lie take four loads that touch sixteen lines each. It is asked for when the step before has used its
+// registers, a decode ahead of its use; the rows past m in its last chunk are never written and never stored.
+struct WideSides {
+  const uint8_t* trellis[2];
+  const uint8_t* operand[2];
+  float* partial[2];
+};
+constexpr int kWideTiles = 4;  // 16-column tiles a wave
+
+template <int CB, int BITS, int TILES>
+__global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const WideSides sides, int m, int n, int k,
+                                                                       int blocks_per_wave) {
+  constexpr int kTileBytes = BITS * 32;
+  constexpr int kStepBytes = kWideTiles * kTileBytes;     // sixteen of K
+  constexpr int kUnits = kStepBytes / 16;                 // 16-byte pieces of it
+  constexpr int kLoads = (2 * kUnits + 63) / 64;          // a stage is two of them, one after the other
+  constexpr int kStageBytes = kLoads * 1024;
+  constexpr int kRingBytes = kRingDepth * kStageBytes;
+  constexpr int kWords = 2 * Windows<BITS>::kCount;
+  const uint8_t* __restrict__ trellis = sides.trellis[blockIdx.z];
+  const uint8_t* __restrict__ rows = sides.operand[blockIdx.z];
+  float* __restrict__ partial = sides.partial[blockIdx.z];
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint8_t* ring = lds + wave * kRingBytes;
+  const int slice = blockIdx.y * kProductWaves + wave;
+  const int first = min(slice * blocks_per_wave, k / 128) * 4;  // in steps of 32
+  const int last = min((slice + 1) * blocks_per_wave, k / 128) * 4;
+  const Place p = PlaceOf(lane);
+  const Windows<BITS> windows = WindowsOf<BITS>(p.first);
+  const int64_t row_bytes = static_cast<int64_t>(n / 16) * kTileBytes;
+  const uint8_t* source = trellis + static_cast<int64_t>(blockIdx.x) * kStepBytes;
+  const uint32_t ring_at = LdsAddress(ring);
+  const int chunks = (m + 15) / 16;  // TILES or, of the last pass, fewer
+
+  auto fetch = [&](int step) {
+    const uint8_t* from = source + static_cast<int64_t>(2 * min(step, last - 1)) * row_bytes;
+    uint8_t* to = ring + (step % kRingDepth) * kStageBytes;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int unit = i * 64 + lane;
+      const int64_t at = unit < kUnits ? unit * 16 : row_bytes + (unit - kUnits) * 16;
+      if (unit < 2 * kUnits) {
+        __builtin_amdgcn_global_load_lds((GlobalPointer)(from + at), (LdsPointer)(to + i * 1024), 16, 0, 0);
+      }
+    }
+  };
+  auto ask = [&](int step, uint32_t (&words)[2 * kWideTiles][kWords]) {
+    const uint32_t stage = ring_at + static_cast<uint32_t>((step % kRingDepth) * kStageBytes);
+#pragma unroll
+    for (int w = 0; w < Windows<BITS>::kCount; ++w) {
+      const uint32_t high = stage + windows.w[w].high, low = stage + windows.w[w].low;
+      words[0][2 * w] = LdsRead4<0 * kTileBytes>(high), words[0][2 * w + 1] = LdsRead4<0 * kTileBytes>(low);
+      words[1][2 * w] = LdsRead4<1 * kTileBytes>(high), words[1][2 * w + 1] = LdsRead4<1 * kTileBytes>(low);
+      words[2][2 * w] = LdsRead4<2 * kTileBytes>(high), words[2][2 * w + 1] = LdsRead4<2 * kTileBytes>(low);
+      words[3][2 * w] = LdsRead4<3 * kTileBytes>(high), words[3][2 * w + 1] = LdsRead4<3 * kTileBytes>(low);
+      words[4][2 * w] = LdsRead4<4 * kTileBytes>(high), words[4][2 * w + 1] = LdsRead4<4 * kTileBytes>(low);
+      words[5][2 * w] = LdsRead4<5 * kTileBytes>(high), words[5][2 * w + 1] = LdsRead4<5 * kTileBytes>(low);
+      words[6][2 * w] = LdsRead4<6 * kTileBytes>(high), words[6][2 * w + 1] = LdsRead4<6 * kTileBytes>(low);
+      words[7][2 * w] = LdsRead4<7 * kTileBytes>(high), words[7][2 * w + 1] = LdsRead4<7 * kTileBytes>(low);
+    }
+  };
+
+  V4f acc[TILES][kWideTiles];
+#pragma unroll
+  for (int r = 0; r < TILES; ++r)
+#pragma unroll
+    for (int t = 0; t < kWideTiles; ++t) acc[r][t] = V4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+  if (first < last) {
+    uint32_t words[2][2 * kWideTiles][kWords];
+    U32x4 x[TILES];
+    auto ask_rows = [&](int step) {  // (a chunk past the pass's last is its last again: no load is skipped)
+      const uint8_t* at = rows + (static_cast<int64_t>(min(step, last - 1)) * chunks * 64 + lane) * 16;
+#pragma unroll
+      for (int r = 0; r < TILES; ++r) {
+        const uint8_t* from = at + min(r, chunks - 1) * 1024;
+        asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(x[r]) : "v"(from));
+      }
+    };
+#pragma unroll
+    for (int s = 0; s < kRingDepth - 1; ++s) fetch(first + s);
+    ask_rows(first);  // (behind the stages, where a later step's are: the waits count on it)
+    LoadsWaited<kLoads*(kRingDepth - 2) + TILES>();
+    ask(first, words[0]);
+    auto one = [&](int step, int parity) {
+      uint32_t (&mine)[2 * kWideTiles][kWords] = words[parity];
+      // Asked for since stage step + 1: stage step + 2, this step's rows, the stage asked for here.
+      fetch(step + kRingDepth - 1);
+      LoadsWaited<kLoads*(kRingDepth - 2) + TILES>();
+      LdsWaited();
+#pragma unroll
+      for (int t = 0; t < 2 * kWideTiles; ++t)
+#pragma unroll
+        for (int w = 0; w < kWords; ++w) LLMP_TIE(mine[t][w]);
+      ask(step + 1, words[parity ^ 1]);
+      Half8 wv[kWideTiles];
+#pragma unroll
+      for (int t = 0; t < kWideTiles; ++t) {
+        const Half4 even = DecodeWindows<CB, BITS>(windows, mine[t]);
+        const Half4 odd = DecodeWindows<CB, BITS>(windows, mine[kWideTiles + t]);
+        wv[t] = __builtin_shufflevector(even, odd, 0, 1, 2, 3, 4, 5, 6, 7);
+        LLMP_TIE(wv[t]);
+      }
+      LoadsWaited<kLoads>();  // the rows: only the stage asked for above may still be on its way
+#pragma unroll
+      for (int r = 0; r < TILES; ++r) LLMP_TIE(x[r]);
+#pragma unroll
+      for (int r = 0; r < TILES; ++r)
+#pragma unroll
+        for (int t = 0; t < kWideTiles; ++t)
+          acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(Half8, x[r]), wv[t], acc[r][t], 0, 0, 0);
+      ask_rows(step + 1);
+    };
+    for (int step = first; step < last; step += 2) {
+      one(step, 0);
+      one(step + 1, 1);
+    }
+    LdsWaited();
+    LoadsWaited<0>();
+  }
+
+  // The waves' sums in wave order through LDS, 32 rows at a time: [wave][row tile][4 t + q][lane].
+  float* sums = reinterpret_cast<float*>(lds);
+  float* out = partial + static_cast<int64_t>(blockIdx.y) * m * n + blockIdx.x * 64;
+#pragma unroll
+  for (int r0 = 0; r0 < TILES; r0 += 2) {
+    __syncthreads();
+#pragma unroll
+    for (int r = r0; r < r0 + 2 && r < TILES; ++r)
+#pragma unroll
+      for (int t = 0; t < kWideTiles; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sums[((wave * 2 + r - r0) * 16 + t * 4 + q) * 64 + lane] = acc[r][t][q];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int e = tid + j * (kProductWaves * 64);  // of 2 x 16 x 64
+      const int r = r0 + (e >> 10);
+      if (r < TILES) {
+        float total = sums[e];
+#pragma unroll
+        for (int w = 1; w < kProductWaves; ++w) total += sums[w * 2048 + e];
+        const int tq = (e >> 6) & 15, l = e & 63;
+        const int row = 16 * r + 4 * (l >> 4) + (tq & 3);
+        if (row < m) out[static_cast<int64_t>(row) * n + (tq >> 2) * 16 + (l & 15)] = total;
+      }
+    }
   }
 }
 
@@ -831,6 +1016,38 @@ void LaunchProduct(const llmp_exl3_weights& w, const ProductSides& sides, int co
   const dim3 grid(static_cast<unsigned>(w.n / 128), static_cast<unsigned>(slices), static_cast<unsigned>(count));
   hipLaunchKernelGGL((ProductKernel<CB, BITS, kFused>), grid, dim3(kProductWaves * 64), kLds, stream, sides, m, w.n, w.k,
                      per);
+}
+
+// The rows of a pass: sixteen through ProductKernel; through WideProductKernel, where the caller's scratch holds its
+// partial sums and its operand, up to 144 (80 above five bits a value, whose decode holds twice the words), shared
+// out evenly in whole tiles of sixteen.
+constexpr int kPassRows = 16;
+int PassRows(int m, int bits, bool wide) {
+  if (m <= kPassRows || !wide) return m < kPassRows ? m : kPassRows;
+  const int tiles = (m + 15) / 16, most = bits <= 5 ? 9 : 5;
+  const int passes = (tiles + most - 1) / most;
+  const int rows = (tiles + passes - 1) / passes * 16;
+  return m < rows ? m : rows;
+}
+// What a pass of `rows` rows of one linear needs: the K slices' partial sums, then the operand of more than sixteen rows.
+size_t PartialBytes(const llmp_exl3_weights& w, int rows) {
+  return static_cast<size_t>(SlicesFor(w.n, w.k)) * rows * w.n * sizeof(float);
+}
+size_t PassBytes(const llmp_exl3_weights& w, int rows) {
+  return PartialBytes(w, rows) + (rows > kPassRows ? static_cast<size_t>((rows + 15) / 16) * 16 * w.k * 2 : 0);
+}
+
+template <int CB, int BITS, int TILES>
+bool g_wide_sized = false;
+template <int CB, int BITS, int TILES>
+void LaunchWide(const llmp_exl3_weights& w, const WideSides& sides, int count, int m, int slices, hipStream_t stream) {
+  constexpr int kRing = kProductWaves * kRingDepth * ((2 * kWideTiles * BITS * 32 + 1023) / 1024) * 1024;
+  constexpr int kLds = kRing > kReduceBytes ? kRing : kReduceBytes;
+  if (!AllowLds(reinterpret_cast<const void*>(&WideProductKernel<CB, BITS, TILES>), kLds, &g_wide_sized<CB, BITS, TILES>)) return;
+  const int blocks = w.k / 128;
+  const int per = (blocks + slices * kProductWaves - 1) / (slices * kProductWaves);
+  const dim3 grid(static_cast<unsigned>(w.n / 64), static_cast<unsigned>(slices), static_cast<unsigned>(count));
+  hipLaunchKernelGGL((WideProductKernel<CB, BITS, TILES>), grid, dim3(kProductWaves * 64), kLds, stream, sides, m, w.n, w.k, per);
 }
 
 template <typename F>
@@ -945,7 +1162,7 @@ namespace {
 
 // `count` linears of the same shape, rate and codebook over one input: the transformed input
 // (a launch of its own above a few rows), the products in slices of K, the slices' sums
-// transformed. Linear i writes a_had[i], scratch[i] and y[i].
+// transformed. Linear i writes a_had[i], scratch[i] (PassBytes of m rows) and y[i].
 int LaunchLinears(const llmp_exl3_weights* const (&w)[2], int count, const void* x, void* const (&a_had)[2],
                   void* const (&y)[2], float* const (&scratch)[2], bool f32, int m, const char* what, hipStream_t s) {
   const llmp_exl3_weights& w0 = *w[0];
@@ -953,8 +1170,14 @@ int LaunchLinears(const llmp_exl3_weights* const (&w)[2], int count, const void*
   const bool fused = m <= kFusedRows;
   const auto* suh0 = static_cast<const uint16_t*>(w[0]->suh);
   const auto* suh1 = static_cast<const uint16_t*>(w[1]->suh);
+  const bool wide = m > kPassRows;
+  uint8_t* operand[2] = {nullptr, nullptr};
+  if (wide) {
+    for (int i = 0; i < 2; ++i) operand[i] = reinterpret_cast<uint8_t*>(scratch[i]) + PartialBytes(w0, m);
+  }
   if (!fused) {
-    const HadamardSides in{{x, x}, {a_had[0], a_had[1]}, {suh0, suh1}, {nullptr, nullptr}};
+    const HadamardSides in{{x, x}, {a_had[0], a_had[1]}, {suh0, suh1}, {nullptr, nullptr},
+                           {reinterpret_cast<uint32_t*>(operand[0]), reinterpret_cast<uint32_t*>(operand[1])}};
     hipLaunchKernelGGL((HadamardKernel<0, 0>),
                        dim3(static_cast<unsigned>(m), static_cast<unsigned>(w0.k / 128), static_cast<unsigned>(count)),
                        dim3(64), 0, s, in, w0.k, 1, int64_t{0});
@@ -970,7 +1193,16 @@ int LaunchLinears(const llmp_exl3_weights* const (&w)[2], int count, const void*
   }
   Dispatch(w0.codebook, w0.bits, [&](auto cb, auto bits) {
     constexpr int kCb = decltype(cb)::value, kBits = decltype(bits)::value;
-    if (fused) {
+    if (wide) {
+      const WideSides over{{sides.trellis[0], sides.trellis[1]}, {operand[0], operand[1]}, {scratch[0], scratch[1]}};
+      if (m <= 32) {
+        LaunchWide<kCb, kBits, 2>(w0, over, count, m, slices, s);
+      } else if (m <= 80) {
+        LaunchWide<kCb, kBits, 5>(w0, over, count, m, slices, s);
+      } else if constexpr (kBits <= 5) {
+        LaunchWide<kCb, kBits, 9>(w0, over, count, m, slices, s);
+      }
+    } else if (fused) {
       LaunchProduct<kCb, kBits, true>(w0, sides, count, m, slices, s);
     } else {
       LaunchProduct<kCb, kBits, false>(w0, sides, count, m, slices, s);
@@ -982,7 +1214,8 @@ int LaunchLinears(const llmp_exl3_weights* const (&w)[2], int count, const void*
   const HadamardSides out{{scratch[0], scratch[1]},
                           {y[0], y[1]},
                           {nullptr, nullptr},
-                          {static_cast<const uint16_t*>(w[0]->svh), static_cast<const uint16_t*>(w[1]->svh)}};
+                          {static_cast<const uint16_t*>(w[0]->svh), static_cast<const uint16_t*>(w[1]->svh)},
+                          {nullptr, nullptr}};
   if (f32) {
     hipLaunchKernelGGL((HadamardKernel<1, 1>), grid, dim3(64), 0, s, out, w0.n, slices, stride);
   } else {
@@ -996,15 +1229,18 @@ int LaunchLinears(const llmp_exl3_weights* const (&w)[2], int count, const void*
 }  // namespace
 }  // namespace llmp_hip
 
-// The rows of one pass of the packed product (the matrix instruction's sixteen); more rows take more passes,
-// each streaming the weights again (src/kernels/exl3/validate.h:76: a launch takes 1 to 65536 rows).
-constexpr int kPassRows = 16;
+// More rows than one pass's take more passes, each streaming the weights again (src/kernels/exl3/validate.h:76: a
+// launch takes 1 to 65536 rows).
 constexpr int kMostRows = 1 << 16;
 
 extern "C" size_t llmp_hip_exl3_linear_scratch(const llmp_exl3_linear* op) {
   if (op == nullptr || op->m <= 0 || op->weights.k <= 0 || op->weights.n <= 0) return 0;
-  const int pass = op->m < kPassRows ? op->m : kPassRows;  // the passes share the area
-  return static_cast<size_t>(SlicesFor(op->weights.n, op->weights.k)) * pass * op->weights.n * sizeof(float);
+  return PassBytes(op->weights, PassRows(op->m, op->weights.bits, false));  // the passes share the area
+}
+
+extern "C" size_t llmp_hip_exl3_linear_wide_scratch(const llmp_exl3_linear* op) {
+  if (op == nullptr || op->m <= 0 || op->weights.k <= 0 || op->weights.n <= 0) return 0;
+  return PassBytes(op->weights, PassRows(op->m, op->weights.bits, true));
 }
 
 namespace llmp_hip {
@@ -1023,6 +1259,8 @@ int LinearOver(const llmp_exl3_linear* op, void* area, size_t area_bytes, hipStr
   if ((reinterpret_cast<uintptr_t>(op->x) | reinterpret_cast<uintptr_t>(op->a_had) |
        reinterpret_cast<uintptr_t>(op->y) | reinterpret_cast<uintptr_t>(area)) % 8 != 0)
     return Refuse(1, "exl3.linear: operands not 8-byte aligned");
+  const bool wide = area_bytes >= llmp_hip_exl3_linear_wide_scratch(op);
+  const int pass = PassRows(op->m, op->weights.bits, wide);
   {
     // validate.cc:120-126: what the launches write (a_had, y, the partial sums in place of the lock area) meets
     // nothing they read and not one another.
@@ -1030,7 +1268,7 @@ int LinearOver(const llmp_exl3_linear* op, void* area, size_t area_bytes, hipStr
     const Range x{"x", reinterpret_cast<uintptr_t>(op->x), m * op->weights.k * 2};
     const Range a_had{"a_had", reinterpret_cast<uintptr_t>(op->a_had), m * op->weights.k * 2};
     const Range y{"y", reinterpret_cast<uintptr_t>(op->y), m * op->weights.n * (op->f32 ? 4 : 2)};
-    const Range partials{"the scratch", reinterpret_cast<uintptr_t>(area), llmp_hip_exl3_linear_scratch(op)};
+    const Range partials{"the scratch", reinterpret_cast<uintptr_t>(area), PassBytes(op->weights, pass)};
     const llmp_exl3_weights& w = op->weights;
     if (const int bad = Disjoint("exl3.linear", a_had, {x, y, TrellisRange(w), SuhRange(w), SvhRange(w), partials}); bad != 0) return bad;
     if (const int bad = Disjoint("exl3.linear", y, {x, TrellisRange(w), SuhRange(w), SvhRange(w), partials}); bad != 0) return bad;
@@ -1038,9 +1276,9 @@ int LinearOver(const llmp_exl3_linear* op, void* area, size_t area_bytes, hipStr
   }
   const llmp_exl3_weights* const w[2] = {&op->weights, &op->weights};
   float* const partial[2] = {static_cast<float*>(area), static_cast<float*>(area)};
-  // Sixteen rows a pass, the passes in stream order over the one area of partial sums.
-  for (int row = 0; row < op->m; row += kPassRows) {
-    const int rows = op->m - row < kPassRows ? op->m - row : kPassRows;
+  // The passes in stream order over the one area.
+  for (int row = 0; row < op->m; row += pass) {
+    const int rows = op->m - row < pass ? op->m - row : pass;
     const size_t in = static_cast<size_t>(row) * op->weights.k * 2;
     const size_t out = static_cast<size_t>(row) * op->weights.n * (op->f32 ? 4 : 2);
     void* const a_had[2] = {static_cast<uint8_t*>(op->a_had) + in, static_cast<uint8_t*>(op->a_had) + in};
@@ -1198,8 +1436,12 @@ extern "C" int llmp_hip_exl3_linear_reconstructed(const llmp_exl3_linear* op, vo
 
 extern "C" size_t llmp_hip_exl3_multi_linear_scratch(const llmp_exl3_multi_linear* op) {
   if (op == nullptr || op->m <= 0 || op->first.k <= 0 || op->first.n <= 0) return 0;
-  const int pass = op->m < kPassRows ? op->m : kPassRows;  // the passes share the area
-  return 2 * static_cast<size_t>(SlicesFor(op->first.n, op->first.k)) * pass * op->first.n * sizeof(float);
+  return 2 * PassBytes(op->first, PassRows(op->m, op->first.bits, false));  // the passes share the area
+}
+
+extern "C" size_t llmp_hip_exl3_multi_linear_wide_scratch(const llmp_exl3_multi_linear* op) {
+  if (op == nullptr || op->m <= 0 || op->first.k <= 0 || op->first.n <= 0) return 0;
+  return 2 * PassBytes(op->first, PassRows(op->m, op->first.bits, true));
 }
 
 extern "C" int llmp_hip_exl3_multi_linear(const llmp_exl3_multi_linear* op, void* scratch, size_t scratch_bytes,
@@ -1218,13 +1460,15 @@ extern "C" int llmp_hip_exl3_multi_linear(const llmp_exl3_multi_linear* op, void
   if ((reinterpret_cast<uintptr_t>(op->x) | reinterpret_cast<uintptr_t>(op->a_had) |
        reinterpret_cast<uintptr_t>(op->y) | reinterpret_cast<uintptr_t>(scratch)) % 8 != 0)
     return Refuse(1, "exl3.multi_linear: operands not 8-byte aligned");
+  const bool wide = scratch_bytes >= llmp_hip_exl3_multi_linear_wide_scratch(op);
+  const int pass = PassRows(op->m, op->first.bits, wide);
   {
     // validate.cc:310-323: a_had, y and the partial sums meet nothing the launches read and not one another.
     const size_t rows = static_cast<size_t>(op->m);
     const Range x{"x", reinterpret_cast<uintptr_t>(op->x), rows * op->first.k * 2};
     const Range a_had{"a_had", reinterpret_cast<uintptr_t>(op->a_had), 2 * rows * op->first.k * 2};
     const Range y{"y", reinterpret_cast<uintptr_t>(op->y), 2 * rows * op->first.n * (op->f32 ? 4 : 2)};
-    const Range area{"the scratch", reinterpret_cast<uintptr_t>(scratch), llmp_hip_exl3_multi_linear_scratch(op)};
+    const Range area{"the scratch", reinterpret_cast<uintptr_t>(scratch), 2 * PassBytes(op->first, pass)};
     for (const llmp_exl3_weights* w : {&op->first, &op->second}) {
       for (const Range& written : {a_had, y, area}) {
         if (const int bad = Disjoint("exl3.multi_linear", written, {TrellisRange(*w), SuhRange(*w), SvhRange(*w)}); bad != 0)
@@ -1239,13 +1483,13 @@ extern "C" int llmp_hip_exl3_multi_linear(const llmp_exl3_multi_linear* op, void
   const int m = op->m, k = op->first.k, n = op->first.n;
   const size_t element = op->f32 ? 4 : 2;
   float* const part = static_cast<float*>(scratch);
-  const size_t part_floats = static_cast<size_t>(SlicesFor(n, k)) * (m < kPassRows ? m : kPassRows) * n;
+  const size_t part_floats = PassBytes(op->first, pass) / sizeof(float);
   const llmp_exl3_weights* const w[2] = {&op->first, &op->second};
   float* const partial[2] = {part, part + part_floats};
   bool queued = false;
-  // Sixteen rows a pass, the passes in stream order over the one area of partial sums.
-  for (int row = 0; row < m; row += kPassRows) {
-    const int rows = m - row < kPassRows ? m - row : kPassRows;
+  // The passes in stream order over the one area.
+  for (int row = 0; row < m; row += pass) {
+    const int rows = m - row < pass ? m - row : pass;
     const uint8_t* x = static_cast<const uint8_t*>(op->x) + static_cast<size_t>(row) * k * 2;
     void* const a_had[2] = {static_cast<uint16_t*>(op->a_had) + static_cast<size_t>(row) * k,
                             static_cast<uint16_t*>(op->a_had) + (static_cast<size_t>(m) + row) * k};

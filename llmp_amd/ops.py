@@ -463,7 +463,7 @@ def exl3_hadamard(x, scale, input_scale=True):
 
 
 def exl3_linear(trellis, suh, svh, k, n, bits, codebook, x, f32=True, keep=None):
-    """x float16 [m, k] through the EXL3 linear (sixteen rows a pass): [m, n] float32 or float16.
+    """x float16 [m, k] through the EXL3 linear (up to 144 rows a pass): [m, n] float32 or float16.
     `keep`, a dict, receives the transformed input a_had."""
     lib = _lib.load()
     m = x.shape[0]
@@ -472,7 +472,7 @@ def exl3_linear(trellis, suh, svh, k, n, bits, codebook, x, f32=True, keep=None)
     a_had = torch.empty((m, k), dtype=torch.float16, device=x.device)
     y = torch.empty((m, n), dtype=torch.float32 if f32 else torch.float16, device=x.device)
     op.x, op.a_had, op.y, op.f32, op.m = x.data_ptr(), a_had.data_ptr(), y.data_ptr(), int(f32), m
-    need = lib.llmp_hip_exl3_linear_scratch(C.byref(op))
+    need = lib.llmp_hip_exl3_linear_wide_scratch(C.byref(op))
     scratch = torch.empty(max(need, 8), dtype=torch.uint8, device=x.device)
     _lib.check(lib.llmp_hip_exl3_linear(C.byref(op), _ptr(scratch), need, _stream()))
     if keep is not None:
@@ -522,7 +522,7 @@ def exl3_linear_static_prepare(trellis, suh, svh, k, n, bits, codebook):
 
 
 def exl3_multi_linear(first, second, x, f32=True, keep=None):
-    """exl3.multi_linear: x float16 [m, k] (sixteen rows a pass) through a gate and an up linear of the same k, n and
+    """exl3.multi_linear: x float16 [m, k] (up to 144 rows a pass) through a gate and an up linear of the same k, n and
     rate: [2, m, n]. `first` and `second` are (trellis, suh, svh, k, n, bits, codebook); `keep`, a dict,
     receives the two transformed inputs a_had [2, m, k]."""
     lib = _lib.load()
@@ -534,7 +534,7 @@ def exl3_multi_linear(first, second, x, f32=True, keep=None):
     a_had = torch.empty((2, m, k), dtype=torch.float16, device=x.device)
     y = torch.empty((2, m, n), dtype=torch.float32 if f32 else torch.float16, device=x.device)
     op.x, op.a_had, op.y, op.f32, op.m = x.data_ptr(), a_had.data_ptr(), y.data_ptr(), int(f32), m
-    need = lib.llmp_hip_exl3_multi_linear_scratch(C.byref(op))
+    need = lib.llmp_hip_exl3_multi_linear_wide_scratch(C.byref(op))
     scratch = torch.empty(max(need, 8), dtype=torch.uint8, device=x.device)
     _lib.check(lib.llmp_hip_exl3_multi_linear(C.byref(op), _ptr(scratch), need, _stream()))
     if keep is not None:

@@ -189,6 +189,41 @@ def test_linear_of_more_than_sixteen_rows_runs_in_passes(device, m):
         assert np.array_equal(both[1].view(np.uint32), alone.view(np.uint32))
 
 
+@pytest.mark.parametrize("m,k,n,bits,codebook", [
+    (17, 128, 128, 4, ops.EXL3_3INST),     # one 128 block: seven of the eight waves have no K
+    (32, 1152, 384, 1, ops.EXL3_MCG), (33, 1024, 128, 2, ops.EXL3_MUL1), (80, 2176, 256, 3, ops.EXL3_3INST),
+    (81, 1024, 256, 4, ops.EXL3_MUL1), (144, 1152, 128, 5, ops.EXL3_MCG),
+    (81, 1024, 256, 6, ops.EXL3_3INST),    # two passes above five bits
+    (145, 512, 256, 4, ops.EXL3_3INST),    # two passes, the second short of its tiles
+    (290, 256, 128, 8, ops.EXL3_MUL1)])
+def test_wide_passes_are_the_sixteen_row_passes_bit_for_bit(device, m, k, n, bits, codebook):
+    """Passes of up to 144 rows (the scratch's wide size) against the linear's passes of sixteen (its least size)."""
+    trellis, suh, svh = synth.exl3_weights(k, n, bits, 80 + bits)
+    args = (dev(trellis, device), halves(suh, device), halves(svh, device), k, n, bits, codebook)
+    x = halves(synth.rng(81 + m).standard_normal((m, k)).astype(np.float16), device)
+    keep = {}
+    got = ops.exl3_linear(*args, x, keep=keep)
+    lib = ops._lib.load()
+    op = ops.Exl3Linear()
+    op.weights = ops._exl3_weights(*args)
+    a_had, y = torch.empty_like(x), torch.empty_like(got)
+    op.x, op.a_had, op.y, op.f32, op.m = x.data_ptr(), a_had.data_ptr(), y.data_ptr(), 1, m
+    least, wide = lib.llmp_hip_exl3_linear_scratch(C.byref(op)), lib.llmp_hip_exl3_linear_wide_scratch(C.byref(op))
+    assert least < wide
+    scratch = torch.full((wide,), 0xFF, dtype=torch.uint8, device=device)  # NaNs where a pass does not write
+    stream = torch.cuda.current_stream().cuda_stream
+    ops._lib.check(lib.llmp_hip_exl3_linear(C.byref(op), scratch.data_ptr(), wide - 1, stream))  # short of wide: sixteen a pass
+    assert torch.equal(y.view(torch.int32), got.view(torch.int32))
+    assert torch.equal(a_had.view(torch.int16), keep["a_had"].view(torch.int16))
+    y.zero_()
+    scratch.fill_(0xFF)
+    ops._lib.check(lib.llmp_hip_exl3_linear(C.byref(op), scratch.data_ptr(), wide, stream))
+    assert torch.equal(y.view(torch.int32), got.view(torch.int32))
+    both = ops.exl3_multi_linear(args, args, x)
+    assert torch.equal(both[0].view(torch.int32), got.view(torch.int32))
+    assert torch.equal(both[1].view(torch.int32), got.view(torch.int32))
+
+
 @pytest.mark.parametrize("m,k,n,bits,codebook", [(200, 1024, 512, 4, ops.EXL3_3INST), (300, 256, 384, 3, ops.EXL3_MCG),
                                                  (1, 128, 128, 5, ops.EXL3_MUL1), (130, 128, 32768 + 256, 2, ops.EXL3_3INST)])
 @pytest.mark.parametrize("fused", [True, False])
