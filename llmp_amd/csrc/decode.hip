@@ -13,6 +13,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "llmp_hip.h"
 
@@ -617,6 +619,17 @@ __device__ __forceinline__ uint32_t ToElement(float v) {
   }
 }
 
+// Two of them, the first in the low half. BF16: one instruction for both.
+template <bool kHalf>
+__device__ __forceinline__ uint32_t ToElements(float low, float high) {
+  if constexpr (kHalf) {
+    return ToElement<true>(low) | (ToElement<true>(high) << 16);
+  } else {
+    typedef __bf16 Bf2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((Float2{low, high}), Bf2));
+  }
+}
+
 // G: groups of 16 outputs a wave; M: groups of 16 input rows (a workgroup takes 64 G outputs by 16 M input rows).
 // Decoding a segment costs some sixty vector instructions whatever M is, so the large tile is what
 // lets the matrix cores, not the decoding, set the pace; the small one is for products with few tiles, where
@@ -942,6 +955,320 @@ void LaunchMatrixShared(const DecodeArgs& a, dim3 grid, uint32_t rows, hipStream
   static bool sized = false;  // more than 64 KB of dynamic LDS must be asked for once
   if (!AllowLds(reinterpret_cast<const void*>(&DecodeMatrixSharedKernel<D, MR>), 2 * SharedStageBytes(MR), &sized)) return;
   hipLaunchKernelGGL((DecodeMatrixSharedKernel<D, MR>), grid, dim3(512), 2 * SharedStageBytes(MR), stream, a, rows);
+}
+
+// The product over laid-out inputs: a launch of its own rounds the inputs to the matrix element once and lays them out as
+// the matrix instruction's first operands (a tile of 16 rows by a chunk of 64 values is 2 KB: both halves of K, a lane's
+// 16 bytes after its neighbour's), so the product reads them into registers as they lie, one coalesced load an operand,
+// and only the weights' decode is left on the vector pipe.
+constexpr int kPanelOutputs = 128;
+struct PanelArgs {
+  DecodeArgs a;
+  const uint8_t* inputs;
+  uint32_t rows, row_tiles, tiles_m, tiles, tiles_a_xcd;
+};
+
+template <bool kHalf>
+__global__ __launch_bounds__(256) void DecodeMatrixInputsKernel(const float* __restrict__ x, uint64_t stride, uint32_t rows,
+                                                                uint32_t k, uint32_t chunks, uint32_t pieces, uint8_t* __restrict__ to) {
+  const uint32_t piece = blockIdx.x * 256u + threadIdx.x;  // a lane of a tile's chunk
+  if (piece >= pieces) return;
+  const uint32_t lane = piece & 63u, unit = piece >> 6, tile = unit / chunks, chunk = unit - tile * chunks;
+  const uint32_t row = tile * 16u + (lane & 15u), column = chunk * 64u + (lane >> 4) * 16u;
+  U32x4 out[2] = {U32x4{0, 0, 0, 0}, U32x4{0, 0, 0, 0}};
+  if (row < rows && column < k) {  // k is a multiple of 16
+    const float4* from = reinterpret_cast<const float4*>(x + row * stride + column);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float4 v = from[i];
+      out[i >> 1][(i & 1) * 2] = ToElements<kHalf>(v.x, v.y);
+      out[i >> 1][(i & 1) * 2 + 1] = ToElements<kHalf>(v.z, v.w);
+    }
+  }
+  U32x4* place = reinterpret_cast<U32x4*>(to + static_cast<uint64_t>(unit) * 2048u) + lane;
+  place[0] = out[0], place[64] = out[1];
+}
+
+// A segment on its way, its scale in its own type and its bytes and halves packed: held as the 32-bit values they widen
+// to, the compiler carries the narrow load around the loop and widens it at the loop's top, which waits for a load just
+// asked for.
+template <int D>
+struct HeldSegment {
+  static constexpr bool kBytes = D == LLMP_DECODER_NVFP4_INTERLEAVED, kHalves = D == LLMP_DECODER_Q8_0_BLOCKS;
+  using Scale = std::conditional_t<kHalves, uint16_t,
+                                   std::conditional_t<D == LLMP_DECODER_NVFP4_GGML_BLOCKS || D == LLMP_DECODER_AFFINE_SPLIT, uint32_t, uint8_t>>;
+  uint32_t code[8];
+  Scale scale;
+  uint32_t extra;
+  __device__ __forceinline__ void Hold(const RawSegment& r) {
+    if constexpr (kBytes) {
+      code[0] = r.a[0] | (r.a[1] << 8) | (r.a[2] << 16) | (r.a[3] << 24);
+      code[1] = r.b[0] | (r.b[1] << 8) | (r.b[2] << 16) | (r.b[3] << 24);
+    } else if constexpr (kHalves) {
+      code[0] = r.a[0] | (r.a[1] << 16), code[1] = r.a[2] | (r.a[3] << 16);
+      code[2] = r.b[0] | (r.b[1] << 16), code[3] = r.b[2] | (r.b[3] << 16);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) code[i] = r.a[i], code[4 + i] = r.b[i];
+    }
+    scale = static_cast<Scale>(r.scale), extra = r.extra;
+  }
+  // As it is, or (past a row's last) zeros, in every encoding the value 0.
+  __device__ __forceinline__ RawSegment Raw(bool live) const {
+    uint32_t c[8];
+#pragma unroll
+    for (int i = 0; i < (kBytes ? 2 : kHalves ? 4 : 8); ++i) c[i] = live ? code[i] : 0u;
+    RawSegment r;
+    if constexpr (kBytes) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r.a[i] = (c[0] >> (8 * i)) & 0xFFu, r.b[i] = (c[1] >> (8 * i)) & 0xFFu;
+    } else if constexpr (kHalves) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r.a[i] = (c[i / 2] >> (16 * (i & 1))) & 0xFFFFu, r.b[i] = (c[2 + i / 2] >> (16 * (i & 1))) & 0xFFFFu;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r.a[i] = c[i], r.b[i] = c[4 + i];
+    }
+    r.scale = live ? scale : 0u, r.extra = live ? extra : 0u;
+    return r;
+  }
+};
+
+__device__ __forceinline__ uint32_t LdsAddress(const void* p) { return static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p)); }
+
+// A workgroup of four waves takes 32 MT input rows by 128 outputs, a wave (rows' half w / 2, outputs' half w % 2) 16 MT
+// rows by 64 outputs: one wave a SIMD, so nothing but its own schedule covers what it waits for. The inputs go to LDS by
+// global_load_lds, three chunks ahead in four stages; a thread's two of a chunk's 512 segments are asked for four chunks
+// ahead, and decoded into the stage after the next one's (three) among the products. A half chunk's operands are read
+// while the half before multiplies. What bounds it: a chunk costs 0.42 us (waits, the decode's 90 vector instructions,
+// LDS) and 0.07 us a row tile (eight products at 16 cycles); what does not depend on K is 10 us a round of workgroups
+// (the first loads, 17 MB of sums stored at the end). 4096 -> 14336 at 300 rows: 64 us with the launch before, 113 with
+// the tiles of 256 by 128 below it, which convert the inputs 56 times and wait for a chunk's loads in every chunk; 64
+// rows 38 us against 54, 1,024 rows 208 against 235 (NVFP4).
+template <int D, int MT>
+__global__ __launch_bounds__(256, 2) void DecodeMatrixPanelKernel(const PanelArgs p) {
+  constexpr bool kHalf = D == LLMP_DECODER_F16_DENSE || D == LLMP_DECODER_Q8_0_BLOCKS;
+  constexpr int kStageBytes = kPanelOutputs * kMatrixRowBytes;
+  constexpr int R = 4;  // chunks of weights on their way
+  constexpr int kInputBytes = MT * 4096, kInputStages = 4;
+  extern __shared__ __attribute__((aligned(16))) uint8_t stages[];  // four of inputs, three of weights
+  const DecodeArgs& a = p.a;
+  // An XCD's workgroups (every eighth) are consecutive tiles, the row tiles of the same outputs next to each other: they
+  // read the same weights through one L2.
+  const uint32_t at = (blockIdx.x & 7u) * p.tiles_a_xcd + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= p.tiles_a_xcd || at >= p.tiles) return;
+  const uint32_t tile_n = at / p.tiles_m, tile_m = at - tile_n * p.tiles_m;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, q = lane >> 4;
+  const uint32_t out0 = tile_n * kPanelOutputs, t0 = tile_m * (32 * MT) + (wave >> 1) * (16 * MT);
+  const uint32_t out_half = (wave & 1) * 64;
+  const uint32_t segs = a.w.k / 16u, chunks = (segs + 3u) / 4u;
+  Float4 acc[4][MT];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[g][m] = Float4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  // The inputs' stage: the workgroup's 2 MT tiles as they lie, MT of the 4 MT pieces of 1 KB a wave, loaded to LDS without
+  // passing through registers. A tile past the last reads the last's and is not stored.
+  const uint8_t* from[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const uint32_t piece = wave * MT + i;
+    from[i] = p.inputs + static_cast<uint64_t>(min(tile_m * (2 * MT) + piece / 2, p.row_tiles - 1)) * chunks * 2048u + (piece & 1u) * 1024u;
+  }
+  const uint32_t inputs_at = LdsAddress(stages);
+  uint8_t* const weight_stages = stages + kInputStages * kInputBytes;
+  HeldSegment<D> raw[R][2];
+  auto load_input = [&](uint32_t chunk, int i) {
+    const uint32_t offset = min(chunk, chunks - 1) * 2048u + lane * 16u;
+    const uint32_t to = inputs_at + (chunk & 3u) * kInputBytes + wave * (MT * 1024) + i * 1024;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(from[i]) : "memory");
+  };
+  auto read_input = [&](uint32_t chunk, int j, int m) {
+    return *reinterpret_cast<const U32x4*>(stages + (chunk & 3u) * kInputBytes + (wave >> 1) * (MT * 2048) + m * 2048 + j * 1024 + lane * 16);
+  };
+  auto load_weights = [&](uint32_t chunk, HeldSegment<D> (&to)[2]) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const uint32_t e = tid + u * 256;
+      to[u].Hold(FetchSegment<D>(a.w, a.first + min(out0 + (e >> 2), a.outputs - 1), min(chunk * 4u + (e & 3u), segs - 1)));
+    }
+  };
+  // One of the thread's two segments of a chunk, decoded into the chunk's stage.
+  auto stage_weights = [&](uint32_t chunk, uint8_t* stage, const HeldSegment<D>& set, int u) {
+    const uint32_t e = tid + u * 256;
+    const uint32_t seg = chunk * 4u + (e & 3u);
+    float v[16], s;
+    DecodeSegment<D>(a.w, min(seg, segs - 1), set.Raw(seg < segs), v, s);
+    U32x4 half[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) half[j][i] = ToElements<kHalf>(v[8 * j + 2 * i] * s, v[8 * j + 2 * i + 1] * s);
+    }
+    U32x4* to = reinterpret_cast<U32x4*>(stage + (e >> 2) * kMatrixRowBytes + (e & 3u) * 32u);
+    to[0] = half[0], to[1] = half[1];
+  };
+  auto read_weight = [&](const uint8_t* stage, int j, int g) {
+    return reinterpret_cast<const U32x4*>(stage + (out_half + 16 * g + n) * kMatrixRowBytes + q * 32)[j];
+  };
+  // A half of a chunk: its products, and between them, one after four, the reads of the next half's operands (a read is
+  // 1 KB of LDS's 128 bytes a cycle and the other three waves read too: read all at once they hold the products back)
+  // and, of the first half, the loads of the inputs three chunks ahead; the thread's segment is decoded among them.
+  auto half = [&](const U32x4 (&x)[MT], const U32x4 (&b)[4], U32x4 (&x_next)[MT], U32x4 (&b_next)[4], const uint8_t* stage_next,
+                  uint32_t chunk_next, int j_next, auto&& load, auto&& decode) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      x_next[m] = read_input(chunk_next, j_next, m);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if (g * MT / 4 == m) b_next[g] = read_weight(stage_next, j_next, g);
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if constexpr (kHalf) {
+          typedef _Float16 Half8 __attribute__((ext_vector_type(8)));
+          acc[g][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(Half8, x[m]), __builtin_bit_cast(Half8, b[g]),
+                                                             acc[g][m], 0, 0, 0);
+        } else {
+          typedef __bf16 Bf8 __attribute__((ext_vector_type(8)));
+          acc[g][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(Bf8, x[m]), __builtin_bit_cast(Bf8, b[g]),
+                                                              acc[g][m], 0, 0, 0);
+        }
+      }
+      load(m);
+    }
+    decode();
+#pragma unroll
+    for (int i = 0; i < 4 * MT; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, MT >= 4 ? 3 : 6, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  uint8_t* now = weight_stages;  // this chunk's stage, the next's and the one after's
+  uint8_t* next = weight_stages + kStageBytes;
+  uint8_t* after = weight_stages + 2 * kStageBytes;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) load_input(0, i), load_input(1, i), load_input(2, i);
+#pragma unroll
+  for (int s = 0; s < R; ++s) load_weights(s, raw[s]);
+  stage_weights(0, now, raw[0][0], 0), stage_weights(0, now, raw[0][1], 1);
+  load_weights(R, raw[0]);
+  stage_weights(1, next, raw[1][0], 0), stage_weights(1, next, raw[1][1], 1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  load_weights(R + 1, raw[1]);
+  __syncthreads();
+  U32x4 b[2][4], x[2][MT];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) b[0][g] = read_weight(now, 0, g);
+#pragma unroll
+  for (int m = 0; m < MT; ++m) x[0][m] = read_input(0, 0, m);
+  auto step = [&](uint32_t chunk, auto slot) {
+    constexpr int P = decltype(slot)::value;
+    // The next chunk's inputs, asked for two steps ago, are here: younger are the inputs asked for a step ago and the
+    // weights of both steps, at least two loads a segment.
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MT + 8) : "memory");
+    // One barrier a chunk: the next chunk's stages are complete, and the readers of those that are written here (the
+    // last chunk's) are done.
+    __syncthreads();
+    half(x[0], b[0], x[1], b[1], now, chunk, 1, [&](int i) { load_input(chunk + 3, i); },
+         [&] { stage_weights(chunk + 2, after, raw[(P + 2) % R][0], 0); });
+    half(x[1], b[1], x[0], b[0], next, chunk + 1, 0, [](int) {}, [&] { stage_weights(chunk + 2, after, raw[(P + 2) % R][1], 1); });
+    load_weights(chunk + 2 + R, raw[(P + 2) % R]);
+    __builtin_amdgcn_sched_barrier(0);
+    uint8_t* const last = now;
+    now = next, next = after, after = last;
+  };
+  uint32_t chunk = 0;
+  for (; chunk + 4 <= chunks; chunk += 4) {  // every wave: the same count of barriers
+    step(chunk, std::integral_constant<int, 0>{});
+    step(chunk + 1, std::integral_constant<int, 1>{});
+    step(chunk + 2, std::integral_constant<int, 2>{});
+    step(chunk + 3, std::integral_constant<int, 3>{});
+  }
+  if (chunk < chunks) step(chunk, std::integral_constant<int, 0>{});
+  if (chunk + 1 < chunks) step(chunk + 1, std::integral_constant<int, 1>{});
+  if (chunk + 2 < chunks) step(chunk + 2, std::integral_constant<int, 2>{});
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing lands in LDS after the workgroup
+  // acc[g][m][i] = D[input row 16 m + 4 q + i][output 16 g + n].
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const uint32_t out = out0 + out_half + 16 * g + n;
+    if (out < a.outputs) {
+      const float scale = a.w.tensor_scale != nullptr ? a.w.tensor_scale[(a.first + out) / a.w.rows_per_scale] : 1.0f;
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t t = t0 + 16 * m + 4 * q + i;
+          if (t < p.rows) a.y[t * a.y_stride + out] = acc[g][m][i] * scale;
+        }
+      }
+    }
+  }
+}
+
+template <int D>
+void LaunchPanel(const DecodeArgs& a, uint32_t rows, int mt, uint8_t* scratch, hipStream_t stream) {
+  constexpr bool kHalf = D == LLMP_DECODER_F16_DENSE || D == LLMP_DECODER_Q8_0_BLOCKS;
+  PanelArgs p;
+  p.a = a, p.inputs = scratch, p.rows = rows, p.row_tiles = (rows + 15u) / 16u;
+  p.tiles_m = (rows + 32u * mt - 1) / (32u * mt);
+  p.tiles = p.tiles_m * ((a.outputs + kPanelOutputs - 1) / kPanelOutputs);
+  p.tiles_a_xcd = (p.tiles + 7) / 8;
+  const uint32_t chunks = (a.w.k + 63u) / 64u, pieces = p.row_tiles * chunks * 64u;
+  hipLaunchKernelGGL((DecodeMatrixInputsKernel<kHalf>), dim3((pieces + 255u) / 256u), dim3(256), 0, stream, a.x, a.x_stride, rows,
+                     a.w.k, chunks, pieces, scratch);
+  const dim3 grid(8 * p.tiles_a_xcd);
+  const auto launch = [&](auto tiles) {
+    constexpr int MT = decltype(tiles)::value;
+    constexpr int kLds = 4 * MT * 4096 + 3 * kPanelOutputs * kMatrixRowBytes;
+    static bool sized = false;  // more than 64 KB of dynamic LDS must be asked for once
+    if (!AllowLds(reinterpret_cast<const void*>(&DecodeMatrixPanelKernel<D, MT>), kLds, &sized)) return;
+    hipLaunchKernelGGL((DecodeMatrixPanelKernel<D, MT>), grid, dim3(256), kLds, stream, p);
+  };
+  switch (mt) {
+    case 1: launch(std::integral_constant<int, 1>{}); break;
+    case 2: launch(std::integral_constant<int, 2>{}); break;
+    case 3: launch(std::integral_constant<int, 3>{}); break;
+    case 4: launch(std::integral_constant<int, 4>{}); break;
+    default: launch(std::integral_constant<int, 5>{}); break;
+  }
+}
+
+// The tiles of the form that converts its inputs itself: 256 outputs by 128 input rows where those still give every other
+// CU a workgroup (else 64 by 64), by 256 rows where the inputs have them and the tiles still give every CU one.
+struct MatrixTiles {
+  bool wide, tall;
+};
+MatrixTiles TilesOf(uint64_t outputs, uint64_t rows) {
+  const int cus = llmp_hip_compute_units();
+  const uint64_t units = static_cast<uint64_t>(cus > 0 ? cus : 256);
+  const bool wide = 2 * ((outputs + 255) / 256 * ((rows + 127) / 128)) >= units;
+  return {wide, wide && rows >= 256 && (outputs + 255) / 256 * ((rows + 255) / 256) >= units};
+}
+
+// The row tiles a wave of the laid-out form: the fewest microseconds by its kernel's costs (10 us a round of workgroups,
+// 0.42 us a chunk and 0.07 us a chunk and tile; LDS holds two workgroups of one tile, one of more, which side by side
+// take 0.6 us a chunk). 4096 -> 14336 with one to five: 300 rows 141, 121, 92, 102, 65 us, 64 rows 38, 45, 49, 53, 58,
+// 1,024 rows 489, 308, 234, 208, 233.
+int PanelTiles(uint64_t outputs, uint64_t rows, uint32_t k) {
+  const int cus = llmp_hip_compute_units();
+  const uint64_t units = static_cast<uint64_t>(cus > 0 ? cus : 256), chunks = (k + 63ull) / 64ull;
+  uint64_t best = ~uint64_t{0};
+  int tiles = 1;
+  for (int mt = 1; mt <= 5; ++mt) {
+    const uint64_t groups = (outputs + kPanelOutputs - 1) / kPanelOutputs * ((rows + 32 * mt - 1) / (32 * mt));
+    const uint64_t paired = mt == 1 && groups > units ? 2 : 1;
+    const uint64_t cost = (groups + paired * units - 1) / (paired * units) * (1000 + chunks * (paired == 2 ? 60 : 42 + 7 * mt));
+    if (cost < best) best = cost, tiles = mt;
+  }
+  return tiles;
 }
 
 size_t DecodeLds(int tokens, uint32_t k) { return static_cast<size_t>(tokens) * (k / 16u) * kSegmentStride; }
@@ -1272,9 +1599,26 @@ extern "C" int llmp_hip_decode_grouped(int decoder, const llmp_decode_operand* e
   return LaunchStatus("decode.grouped");
 }
 
+extern "C" size_t llmp_hip_decode_matrix_scratch(const llmp_decode_operand* w, uint64_t outputs, uint64_t rows) {
+  if (w == nullptr || outputs == 0 || rows == 0 || rows > 65535ull * 64ull || w->k == 0 || w->k > (1u << 26)) return 0;
+  const MatrixTiles t = TilesOf(outputs, rows);
+  // The inputs' launch and the start and end of a round are paid back by the chunks. Measured at 1,024 and 2,048 values of
+  // K, the old form against this one: tiles of 64 by 64 13.0-17.6 us against 14.0-18.3 and 24.6-26.7 against 21.8-24.4;
+  // of 256 by 128 36.6 against 32.2 (26.7 both at 512); of 256 by 256 77 against 92 (235 against 208 at 4,096).
+  const uint64_t chunks = (w->k + 63ull) / 64ull;
+  if (chunks < (t.tall ? 36u : t.wide ? 12u : 24u)) return 0;
+  return (rows + 15) / 16 * chunks * 2048;
+}
+
 extern "C" int llmp_hip_decode_matrix(int decoder, const llmp_decode_operand* w, uint64_t first, uint64_t outputs,
                                       const float* x, uint64_t rows, uint64_t x_stride, float* y, uint64_t y_stride,
                                       int path, void* stream) {
+  return llmp_hip_decode_matrix_staged(decoder, w, first, outputs, x, rows, x_stride, y, y_stride, path, nullptr, 0, stream);
+}
+
+extern "C" int llmp_hip_decode_matrix_staged(int decoder, const llmp_decode_operand* w, uint64_t first, uint64_t outputs,
+                                             const float* x, uint64_t rows, uint64_t x_stride, float* y, uint64_t y_stride,
+                                             int path, void* scratch, size_t scratch_bytes, void* stream) {
   BeginLaunches();
   if (const int bad = CheckOperand("decode.matrix", decoder, w, first, outputs); bad != 0) return bad;
   if (x == nullptr || y == nullptr) return Refuse(1, "decode.matrix: null operand");
@@ -1290,15 +1634,34 @@ extern "C" int llmp_hip_decode_matrix(int decoder, const llmp_decode_operand* w,
   a.first = static_cast<uint32_t>(first);
   a.outputs = static_cast<uint32_t>(outputs);
   a.x = x, a.x_stride = x_stride, a.y = y, a.y_stride = y_stride;
-  // Tiles of 256 outputs by 128 input rows where those still give every other CU a workgroup; else 64 by 64.
-  const int cus = llmp_hip_compute_units();
-  const uint64_t units = static_cast<uint64_t>(cus > 0 ? cus : 256);
-  const bool wide = 2 * ((outputs + 255) / 256 * ((rows + 127) / 128)) >= units;
-  // Tiles of 256 input rows where the inputs have them and the tiles still give every CU one.
-  const bool tall = wide && rows >= 256 && (outputs + 255) / 256 * ((rows + 255) / 256) >= units;
+  const MatrixTiles t = TilesOf(outputs, rows);
+  const bool wide = t.wide, tall = t.tall;
+  const auto s = static_cast<hipStream_t>(stream);
+  const size_t staged = scratch == nullptr ? 0 : llmp_hip_decode_matrix_scratch(w, outputs, rows);
+  if (staged > 0 && scratch_bytes >= staged) {
+    if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0) return Refuse(1, "decode.matrix: scratch is 16-byte aligned");
+    const int tiles = PanelTiles(outputs, rows, w->k);
+    switch (decoder) {
+#define LLMP_DECODER(ID) \
+  case ID: LaunchPanel<ID>(a, static_cast<uint32_t>(rows), tiles, static_cast<uint8_t*>(scratch), s); break;
+      LLMP_DECODER(LLMP_DECODER_BF16_DENSE)
+      LLMP_DECODER(LLMP_DECODER_F16_DENSE)
+      LLMP_DECODER(LLMP_DECODER_Q8_0_BLOCKS)
+      LLMP_DECODER(LLMP_DECODER_NVFP4_SPLIT)
+      LLMP_DECODER(LLMP_DECODER_NVFP4_ATOMS)
+      LLMP_DECODER(LLMP_DECODER_NVFP4_INTERLEAVED)
+      LLMP_DECODER(LLMP_DECODER_NVFP4_GGML_BLOCKS)
+      LLMP_DECODER(LLMP_DECODER_MXFP8_SPLIT)
+      LLMP_DECODER(LLMP_DECODER_MXFP8_ATOMS)
+      LLMP_DECODER(LLMP_DECODER_MXFP4_SPLIT)
+      LLMP_DECODER(LLMP_DECODER_MXFP4_ATOMS)
+      LLMP_DECODER(LLMP_DECODER_AFFINE_SPLIT)
+#undef LLMP_DECODER
+    }
+    return LaunchStatus("decode.matrix");
+  }
   const uint64_t per = wide ? 256 : 64, tile = tall ? 256 : wide ? 128 : 64;
   const dim3 grid(static_cast<unsigned>((outputs + per - 1) / per), static_cast<unsigned>((rows + tile - 1) / tile));
-  const auto s = static_cast<hipStream_t>(stream);
   switch (decoder) {
 #define LLMP_DECODER(ID)                                                                                          \
   case ID:                                                                                                        \

@@ -627,6 +627,8 @@ def decode_matrix(decoder, weight, x, first=0, outputs=None, path=0, out=None):
     outputs = weight["data"].shape[0] - first if outputs is None else outputs
     rows = x.shape[0]
     y = torch.empty((rows, outputs), dtype=torch.float32, device=x.device) if out is None else out
-    _lib.check(lib.llmp_hip_decode_matrix(decoder, C.byref(op), first, outputs, _ptr(x), rows, x.stride(0), _ptr(y),
-                                          y.stride(0), path, _stream()))
+    size = lib.llmp_hip_decode_matrix_scratch(C.byref(op), outputs, rows) if outputs > 0 else 0
+    scratch = torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
+    _lib.check(lib.llmp_hip_decode_matrix_staged(decoder, C.byref(op), first, outputs, _ptr(x), rows, x.stride(0), _ptr(y),
+                                                 y.stride(0), path, _ptr(scratch) if size else None, size, _stream()))
     return y

@@ -2,13 +2,15 @@
 1 to 16 input rows, row windows, strides, tensor scales, undefined block scales. Float outputs to
 a maximum relative error of 1e-3 (the accumulation order is the only difference: both sides
 decode every value exactly)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import oracle
 from conftest import rel_close
-from llmp_amd import ops, synth
+from llmp_amd import _lib, ops, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -319,6 +321,31 @@ def test_matrix_tall_tiles_match_oracle(device, decoder):
     want = oracle.decode_matrix(decoder, w, x, first=7, outputs=4100, threads=oracle.max_threads())
     got = ops.decode_matrix(decoder, wd, torch.from_numpy(x).to(device), first=7, outputs=4100).cpu().numpy()
     ok, worst = rel_close(got, want, 1e-3)
+    assert ok, (oracle.DECODERS[decoder], worst)
+
+
+@pytest.mark.parametrize("decoder", list(range(12)))
+def test_matrix_laid_out_inputs_are_the_same_bits(device, decoder):
+    """The two-launch form (inputs laid out first) against the one launch, whose operands, and their order in the sums, it
+    shares: one to five row tiles a wave, partial tiles of rows, outputs and K; then few outputs against the oracle."""
+    n, k = 14300, 1568 if decoder in (0, 1, 3, 5, 11) else 1664 if decoder in (8, 10) else 1600
+    w = synth.affine_weight(n, k, 900, bits=8, group=32, scale="bf16") if decoder == 11 else \
+        synth.decode_weight(decoder, n, k, 900 + decoder, tensor_scales=4)
+    wd = {key: (torch.from_numpy(np.ascontiguousarray(v)).to(device) if isinstance(v, np.ndarray) else v)
+          for key, v in w.items() if key != "plain"}
+    x = torch.from_numpy(synth.activations(300, k, 901)).to(device)
+    lib, op = _lib.load(), ops._decode_operand(wd)
+    for rows in (17, 128, 190, 250, 300):
+        scratch = lib.llmp_hip_decode_matrix_scratch(ctypes.byref(op), 14290, rows)
+        assert scratch == (rows + 15) // 16 * 2048 * ((k + 63) // 64)
+        want = torch.empty((rows, 14290), dtype=torch.float32, device=device)
+        _lib.check(lib.llmp_hip_decode_matrix(decoder, ctypes.byref(op), 7, 14290, x.data_ptr(), rows, k, want.data_ptr(),
+                                              14290, 0, None))
+        torch.cuda.synchronize()
+        got = ops.decode_matrix(decoder, wd, x[:rows], first=7, outputs=14290)
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), rows
+    want = oracle.decode_matrix(decoder, w, x[:33].cpu().numpy(), first=7, outputs=139, threads=oracle.max_threads())
+    ok, worst = rel_close(ops.decode_matrix(decoder, wd, x[:33], first=7, outputs=139).cpu().numpy(), want, 1e-3)
     assert ok, (oracle.DECODERS[decoder], worst)
 
 
