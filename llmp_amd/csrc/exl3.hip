@@ -211,34 +211,6 @@ __device__ __forceinline__ void Hadamard128(float& a, float& b, int lane) {
   }
 }
 
-// The same transform of four vectors a wave, one a row of sixteen lanes: lane l of a row holds elements l + 16 e,
-// e = 0 .. 7. (The transform does not change when the bits of its index are permuted on both sides.) The three index
-// bits that e holds are butterflies within the lane, the four that l holds exchanges within the row, which are
-// data-parallel moves: nothing passes through LDS, and a value costs twelve operations where the wave-wide form
-// takes over twenty. `sign[b]`: -1 where bit b of l is set, else 1.
-__device__ __forceinline__ void Hadamard128Rows(float (&x)[8], const float (&sign)[4]) {
-#pragma clang fp contract(off)
-#pragma unroll
-  for (int bit = 1; bit < 8; bit <<= 1) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      if ((e & bit) == 0) {
-        const float sum = x[e] + x[e | bit];
-        x[e | bit] = x[e] - x[e | bit];
-        x[e] = sum;
-      }
-    }
-  }
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float other = ShflXor(x[e], 1 << b);
-      x[e] = __builtin_fmaf(x[e], sign[b], other);
-    }
-  }
-}
-
 // y = f(H(x * in_scale)) * r * out_scale over each 128 block of each row; grid (rows, columns
 // / 128), a wave a block. X / Y: 0 F16, 1 F32. `slices` partial inputs are added in order first.
 // One or two transforms a launch (grid z): a linear's, or the two of a gate/up pair.
@@ -312,33 +284,19 @@ __global__ __launch_bounds__(64) void HadamardKernel(const HadamardSides sides, 
 
 // ------------------------------------------------------- reconstruct, transformed
 
-// Columns [column, column + columns) of the weights themselves, W = diag(suh) H What H diag(svh) / 128 with H the
-// 128-point transform over each block of 128 inputs and of 128 outputs, into w[k][columns] F16 (the reference's
-// reconstruct_had_kernel, launch.cc:440-448; the definition decode.h:37-43). A workgroup of four waves a block of 128
-// inputs by 128 outputs; LDS 128 x 129 floats. The rotated values are decoded into
-// LDS (exact), every column is transformed along the inputs and every row along the outputs in F32 (four vectors a
-// wave at a time, Hadamard128Rows), and the block is rounded to F16 once, after the scales: the reference's kernel
-// rounds every butterfly to F16.
+// Columns [column, column + columns) of the rotated weights transposed, w[columns][k]: a column's inputs together, which is
+// how the product below reads its second operand (both operands' rows along K). A workgroup of four waves a block of 128
+// inputs by 128 outputs, turned by way of LDS, 128 x 129 floats.
 constexpr int kHadBlockPitch = 129;
 constexpr int kHadBlockLds = 128 * kHadBlockPitch * 4;
 
-// kTransform false: the rotated values as they are (the reconstruction without the transforms, through the same
-// block). kTransposed: w[columns][k] instead, a column's inputs together, which is how the product below reads its
-// second operand (both operands' rows along K).
-template <int CB, int BITS, bool kTransform, bool kTransposed>
-__global__ __launch_bounds__(256) void ReconstructHadKernel(const uint32_t* __restrict__ trellis,
-                                                           const uint16_t* __restrict__ suh,
-                                                           const uint16_t* __restrict__ svh,
-                                                           uint16_t* __restrict__ w, int n, int k, int column, int columns) {
-#pragma clang fp contract(off)
+template <int CB, int BITS>
+__global__ __launch_bounds__(256) void ReconstructTransposedKernel(const uint32_t* __restrict__ trellis,
+                                                                  uint16_t* __restrict__ w, int n, int k, int column, int columns) {
   extern __shared__ __attribute__((aligned(16))) float had_block[];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const Place p = PlaceOf(lane);
-  const int l16 = lane & 15, row4 = lane >> 4;
-  float sign[4];
-#pragma unroll
-  for (int b = 0; b < 4; ++b) sign[b] = (l16 >> b) & 1 ? -1.0f : 1.0f;
   // Sixteen of a block's 64 tiles a wave. A lane's four states lie within three consecutive words of a tile's
   // stream, the same three in every tile: they are asked for from all sixteen tiles before the first is decoded (a
   // tile after the other, each decode would wait for its own loads), and a workgroup goes through its blocks (every
@@ -381,52 +339,192 @@ __global__ __launch_bounds__(256) void ReconstructHadKernel(const uint32_t* __re
   // (A block past the last is the last again: no load under a branch.)
   ask(min(block + static_cast<int>(gridDim.x), blocks - 1));
   __syncthreads();
-  if constexpr (kTransform) {
-    // Along the inputs: a wave 32 columns, four at a time, one a row of sixteen lanes (Hadamard128Rows).
-    for (int j = wave * 32 + row4; j < wave * 32 + 32; j += 4) {
-      float x[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = had_block[(l16 + 16 * e) * kHadBlockPitch + j];
-      Hadamard128Rows(x, sign);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) had_block[(l16 + 16 * e) * kHadBlockPitch + j] = x[e];
-    }
-    __syncthreads();
-    // Along the outputs, then the scales: a wave 32 rows.
-    float sv[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sv[e] = HalfBitsToFloat(svh[column + c0 + l16 + 16 * e]) * (1.0f / 128.0f);
-    for (int i = wave * 32 + row4; i < wave * 32 + 32; i += 4) {
-      float x[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = had_block[i * kHadBlockPitch + l16 + 16 * e];
-      Hadamard128Rows(x, sign);
-      const float su = HalfBitsToFloat(suh[k0 + i]);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) had_block[i * kHadBlockPitch + l16 + 16 * e] = x[e] * (su * sv[e]);
-    }
-    __syncthreads();
-  }
-  // Sixteen bytes a thread: a row (a column, transposed) is sixteen threads' worth.
+  // Sixteen bytes a thread: a column is sixteen threads' worth.
   const int part = threadIdx.x & 15;
   for (int i = threadIdx.x >> 4; i < 128; i += 16) {
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      v[e] = kTransposed ? had_block[(part * 8 + e) * kHadBlockPitch + i] : had_block[i * kHadBlockPitch + part * 8 + e];
+      v[e] = had_block[(part * 8 + e) * kHadBlockPitch + i];
     }
     U32x4 out;
     out.x = FloatToHalfBits(v[0]) | (FloatToHalfBits(v[1]) << 16);
     out.y = FloatToHalfBits(v[2]) | (FloatToHalfBits(v[3]) << 16);
     out.z = FloatToHalfBits(v[4]) | (FloatToHalfBits(v[5]) << 16);
     out.w = FloatToHalfBits(v[6]) | (FloatToHalfBits(v[7]) << 16);
-    if constexpr (kTransposed) {
-      *reinterpret_cast<U32x4*>(w + static_cast<int64_t>(c0 + i) * k + k0 + part * 8) = out;
-    } else {
-      *reinterpret_cast<U32x4*>(w + static_cast<int64_t>(k0 + i) * columns + c0 + part * 8) = out;
-    }
+    *reinterpret_cast<U32x4*>(w + static_cast<int64_t>(c0 + i) * k + k0 + part * 8) = out;
   }
   __syncthreads();  // the block's readers, before the next is decoded into it
+  }
+}
+
+// Columns [column, column + columns) of the weights themselves, W = diag(suh) H What H diag(svh) / 128 with H the
+// 128-point transform over each block of 128 inputs and of 128 outputs, as F16 (the reference's
+// reconstruct_had_kernel, launch.cc:440-448; the definition decode.h:37-43), rounded to F16 once, after the scales: the
+// reference's kernel rounds every butterfly to F16.
+// Both transforms are on the matrix cores: a workgroup a block of 128 inputs by 128 outputs, a wave 32 of the inputs'
+// indices. H128 is H8 x H16 over an index 16 a + r; its entries +-1 are exact in F16, as the rotated values are. A lane's
+// four decoded values of a tile are a 16x16x16 operand as they lie, two tiles of K one of 16x16x32 (a wave decodes a quarter
+// of the tiles for all four, by way of LDS): along the inputs, four products a tile of 16 outputs by 16 indices. The sums
+// come out as a lane's four outputs of one index, the next operand's layout: split into three F16, each the remainder of
+// those before it (nothing of an F32 sum is left out), they are the halves of K of two products with H16 along the
+// outputs; H8 along them is three additions a value. The indices are dealt to the rows so that a lane ends with eight
+// consecutive ones, sixteen bytes of a column. Against F64 a result's error is the one rounding to F16: 2.07e-4 over two
+// to six bits and the three codebooks, in every one of them at most the F32 butterflies'.
+// Bound by vector issue (decode 1,800 instructions a block and lane, split 2,000, additions 800, scales and rounding 800),
+// 3.5 blocks a SIMD at 4096 x 14336, and 117 MB written (23 us at a copy's rate): 59 us there, where the transforms as
+// butterflies in F32 by data-parallel moves and LDS, 42 operations a value, took 104. A wave a block with all its sums in
+// registers (one wave a SIMD) took 74: nothing ran under its waits.
+// kTransposed: w[columns][k], a column's inputs together. Else w[k][columns], the rows turned by way of LDS.
+constexpr int kTurnPitch = 264;  // bytes from a row of 128 outputs to the next: four rows eight apart in different banks
+template <int CB, int BITS, bool kTransposed>
+__global__ __launch_bounds__(256, 3) void ReconstructHadKernel(const uint32_t* __restrict__ trellis,
+                                                              const uint16_t* __restrict__ suh,
+                                                              const uint16_t* __restrict__ svh,
+                                                              uint16_t* __restrict__ w, int n, int k, int column, int columns) {
+#pragma clang fp contract(off)
+  typedef _Float16 Half8 __attribute__((ext_vector_type(8)));
+  typedef float Float4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int blocks_k = k / 128;
+  const int c0 = (static_cast<int>(blockIdx.x) / blocks_k) * 128, k0 = (static_cast<int>(blockIdx.x) % blocks_k) * 128;
+  const Place p = PlaceOf(lane);
+  constexpr int kWords = BITS * 8, kHeld = BITS <= 5 ? 2 : 3;  // a lane's states lie within so many words of a tile
+  const int word0 = (((p.first + 1) * BITS + 256 * BITS - 16) >> 5) % kWords;
+  const uint32_t* tiles = trellis + (static_cast<int64_t>(k0 / 16) * (n / 16) + (column + c0) / 16) * kWords;
+  uint32_t at[kHeld];
+#pragma unroll
+  for (int i = 0; i < kHeld; ++i) at[i] = (word0 + i) % kWords;
+  // Two of the block's eight columns of tiles a wave, into LDS as the operands they are: [column][two tiles][lane].
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kTransposed ? 32 * 1024 : 4 * 32 * kTurnPitch];
+  uint32_t words[16][kHeld];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const uint32_t* tile = tiles + (static_cast<int64_t>(u & 7) * (n / 16) + 2 * wave + (u >> 3)) * kWords;
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i) words[u][i] = tile[at[i]];
+  }
+#pragma unroll
+  for (int pair = 0; pair < 8; ++pair) {
+    Half8 two;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const uint32_t(&held)[kHeld] = words[2 * pair + u];
+      const Half4 v = DecodeFour<CB, BITS>(p.first, [&](int i) {
+        const int d = (i - word0 + kWords) % kWords;
+        return d == 0 ? held[0] : (kHeld == 2 || d == 1) ? held[1] : held[kHeld - 1];
+      });
+#pragma unroll
+      for (int j = 0; j < 4; ++j) two[4 * u + j] = v[j];
+    }
+    *reinterpret_cast<Half8*>(lds + ((8 * wave + pair) * 64 + lane) * 16) = two;
+  }
+  // H's operands. Along the inputs, for rows m = lane % 16 of index 32 wave + 8 (m / 4) + 4 b + m % 4: the signs of the
+  // tile's sixteen and of the pair's two (and, for an odd count of common bits of the wave's and the pair's numbers, the
+  // other sign); along the outputs H16, once for each half of the split.
+  Half8 along_inputs[2][4], along_outputs;
+  U32x4 flipped[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t flip = __popc(wave & q) & 1 ? 0x80008000u : 0u;
+    flipped[q] = U32x4{flip, flip, flip, flip};
+  }
+  const int m = lane & 15;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int index = 8 * ((m >> 2) & 1) + 4 * b + (m & 3);
+      const int odd = __popc(RowOf(p.g, j & 3) & index) + (j >> 2) * (m >> 3);
+      along_inputs[b][0][j] = static_cast<_Float16>(odd & 1 ? -1.0f : 1.0f);
+    }
+    const int odd = __popc((4 * p.g + (j & 3)) & m) & 1;
+    along_outputs[j] = static_cast<_Float16>(odd ? -1.0f : 1.0f);
+  }
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+#pragma unroll
+    for (int q = 1; q < 4; ++q)
+      along_inputs[b][q] = __builtin_bit_cast(Half8, __builtin_bit_cast(U32x4, along_inputs[b][0]) ^ flipped[q]);
+  }
+  __syncthreads();
+  Float4 sums[2][8];  // [the inputs' 32: which half of a lane's eight][outputs' tile]
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    Float4 first[2] = {Float4{0.0f, 0.0f, 0.0f, 0.0f}, Float4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const Half8 rotated = *reinterpret_cast<const Half8*>(lds + ((4 * t + q) * 64 + lane) * 16);
+#pragma unroll
+      for (int b = 0; b < 2; ++b) first[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rotated, along_inputs[b][q], first[b], 0, 0, 0);
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      Half8 split, rest;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const _Float16 high = static_cast<_Float16>(first[b][r]);
+        const float below = first[b][r] - static_cast<float>(high);
+        const _Float16 middle = static_cast<_Float16>(below);
+        split[r] = high, split[4 + r] = middle;
+        rest[r] = static_cast<_Float16>(below - static_cast<float>(middle)), rest[4 + r] = static_cast<_Float16>(0.0f);
+      }
+      const Float4 low = __builtin_amdgcn_mfma_f32_16x16x32_f16(rest, along_outputs, Float4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+      sums[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(split, along_outputs, low, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+#pragma unroll
+    for (int bit = 1; bit < 8; bit <<= 1) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        if ((t & bit) == 0) {
+          const Float4 x = sums[b][t], y = sums[b][t | bit];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sums[b][t][r] = x[r] + y[r], sums[b][t | bit][r] = x[r] - y[r];
+        }
+      }
+    }
+  }
+  if constexpr (!kTransposed) __syncthreads();  // the operands' readers, before rows are turned there
+  uint8_t* const mine = lds + wave * (32 * kTurnPitch);
+  uint16_t* const out = w + static_cast<int64_t>(c0 + m) * k + k0 + 32 * wave + 8 * p.g;
+  float sv[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sv[e] = HalfBitsToFloat(svh[column + c0 + 16 * e + m]) * (1.0f / 128.0f);
+  const uint2* four = reinterpret_cast<const uint2*>(suh + k0 + 32 * wave + 8 * p.g);  // 8-byte aligned
+  const U32x4 scales = U32x4{four[0].x, four[0].y, four[1].x, four[1].y};
+  float su[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) su[e] = HalfBitsToFloat(e & 1 ? scales[e / 2] >> 16 : scales[e / 2] & 0xFFFFu);
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    U32x4 packed;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float low = sums[e >> 1][t][2 * (e & 1)] * (su[2 * e] * sv[t]);
+      const float high = sums[e >> 1][t][2 * (e & 1) + 1] * (su[2 * e + 1] * sv[t]);
+      packed[e] = FloatToHalfBits(low) | (FloatToHalfBits(high) << 16);
+    }
+    if constexpr (kTransposed) {
+      *reinterpret_cast<U32x4*>(out + static_cast<int64_t>(16 * t) * k) = packed;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        *reinterpret_cast<uint16_t*>(mine + (8 * p.g + e) * kTurnPitch + (16 * t + m) * 2) = static_cast<uint16_t>(packed[e / 2] >> (16 * (e & 1)));
+    }
+  }
+  if constexpr (!kTransposed) {  // a wave's own rows: its accesses of LDS are in order
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int row = 4 * u + (lane >> 4);
+      const uint2* part = reinterpret_cast<const uint2*>(mine + row * kTurnPitch + (lane & 15) * 16);
+      const uint2 low = part[0], high = part[1];
+      *reinterpret_cast<U32x4*>(w + static_cast<int64_t>(k0 + 32 * wave + row) * columns + c0 + (lane & 15) * 8) = U32x4{low.x, low.y, high.x, high.y};
+    }
   }
 }
 
@@ -975,20 +1073,27 @@ void LaunchReconstruct(const llmp_exl3_weights& w, void* out, int column, int co
                      static_cast<const uint32_t*>(w.trellis), static_cast<uint16_t*>(out), w.n, w.k, column, columns);
 }
 
-template <int CB, int BITS, bool kTransform, bool kTransposed>
-bool g_reconstruct_had_sized = false;
-template <int CB, int BITS, bool kTransform, bool kTransposed>
+template <int CB, int BITS, bool kTransposed>
 void LaunchReconstructHad(const llmp_exl3_weights& w, void* out, int column, int columns, hipStream_t stream) {
-  if (!AllowLds(reinterpret_cast<const void*>(&ReconstructHadKernel<CB, BITS, kTransform, kTransposed>), kHadBlockLds,
-                &g_reconstruct_had_sized<CB, BITS, kTransform, kTransposed>))
+  const int blocks = (columns / 128) * (w.k / 128);
+  hipLaunchKernelGGL((ReconstructHadKernel<CB, BITS, kTransposed>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
+                     static_cast<const uint32_t*>(w.trellis), static_cast<const uint16_t*>(w.suh),
+                     static_cast<const uint16_t*>(w.svh), static_cast<uint16_t*>(out), w.n, w.k, column, columns);
+}
+
+template <int CB, int BITS>
+bool g_reconstruct_transposed_sized = false;
+template <int CB, int BITS>
+void LaunchReconstructTransposed(const llmp_exl3_weights& w, void* out, int column, int columns, hipStream_t stream) {
+  if (!AllowLds(reinterpret_cast<const void*>(&ReconstructTransposedKernel<CB, BITS>), kHadBlockLds,
+                &g_reconstruct_transposed_sized<CB, BITS>))
     return;
   // Two workgroups a compute unit are resident (LDS): that many go through the blocks.
   const int blocks = (columns / 128) * (w.k / 128);
   const int cus = llmp_hip_compute_units() > 0 ? llmp_hip_compute_units() : 256;
   const dim3 grid(static_cast<unsigned>(blocks < 2 * cus ? blocks : 2 * cus));
-  hipLaunchKernelGGL((ReconstructHadKernel<CB, BITS, kTransform, kTransposed>), grid, dim3(256), kHadBlockLds, stream,
-                     static_cast<const uint32_t*>(w.trellis), static_cast<const uint16_t*>(w.suh),
-                     static_cast<const uint16_t*>(w.svh), static_cast<uint16_t*>(out), w.n, w.k, column, columns);
+  hipLaunchKernelGGL((ReconstructTransposedKernel<CB, BITS>), grid, dim3(256), kHadBlockLds, stream,
+                     static_cast<const uint32_t*>(w.trellis), static_cast<uint16_t*>(out), w.n, w.k, column, columns);
 }
 
 template <int BITS>
@@ -1118,7 +1223,7 @@ extern "C" int llmp_hip_exl3_reconstruct_fused(const llmp_exl3_weights* weights,
       bad != 0)
     return bad;
   Dispatch(weights->codebook, weights->bits, [&](auto cb, auto bits) {
-    LaunchReconstructHad<decltype(cb)::value, decltype(bits)::value, true, false>(*weights, w, column, columns,
+    LaunchReconstructHad<decltype(cb)::value, decltype(bits)::value, false>(*weights, w, column, columns,
                                                                                   static_cast<hipStream_t>(stream));
   });
   return LaunchStatus("exl3.reconstruct_fused");
@@ -1413,9 +1518,9 @@ extern "C" int llmp_hip_exl3_linear_reconstructed(const llmp_exl3_linear* op, vo
     // The slice's weights, a column's inputs together (the product reads both operands along K).
     llmp_hip::Dispatch(weights.codebook, weights.bits, [&](auto cb, auto bits) {
       if (fused) {
-        llmp_hip::LaunchReconstructHad<decltype(cb)::value, decltype(bits)::value, true, true>(weights, w, column, columns, s);
+        llmp_hip::LaunchReconstructHad<decltype(cb)::value, decltype(bits)::value, true>(weights, w, column, columns, s);
       } else {
-        llmp_hip::LaunchReconstructHad<decltype(cb)::value, decltype(bits)::value, false, true>(weights, w, column, columns, s);
+        llmp_hip::LaunchReconstructTransposed<decltype(cb)::value, decltype(bits)::value>(weights, w, column, columns, s);
       }
     });
     void* y_at = op->f32 ? static_cast<void*>(static_cast<float*>(op->y) + column) : static_cast<void*>(static_cast<uint16_t*>(op->y) + column);
