@@ -1042,7 +1042,7 @@ __device__ __forceinline__ uint32_t LdsAddress(const void* p) { return static_ca
 // ahead, and decoded into the stage after the next one's (three) among the products. A half chunk's operands are read
 // while the half before multiplies. What bounds it: a chunk costs 0.42 us (waits, the decode's 90 vector instructions,
 // LDS) and 0.07 us a row tile (eight products at 16 cycles); what does not depend on K is 10 us a round of workgroups
-// (the first loads, 17 MB of sums stored at the end). 4096 -> 14336 at 300 rows: 64 us with the launch before, 113 with
+// (the first loads, 17 MB of sums stored at the end). 4096 -> 14336 at 300 rows: 60 us with the launch before, 113 with
 // the tiles of 256 by 128 below it, which convert the inputs 56 times and wait for a chunk's loads in every chunk; 64
 // rows 38 us against 54, 1,024 rows 208 against 235 (NVFP4).
 template <int D, int MT>
@@ -1131,11 +1131,11 @@ __global__ __launch_bounds__(256, 2) void DecodeMatrixPanelKernel(const PanelArg
       for (int g = 0; g < 4; ++g) {
         if constexpr (kHalf) {
           typedef _Float16 Half8 __attribute__((ext_vector_type(8)));
-          acc[g][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(Half8, x[m]), __builtin_bit_cast(Half8, b[g]),
+          acc[g][m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(Half8, b[g]), __builtin_bit_cast(Half8, x[m]),
                                                              acc[g][m], 0, 0, 0);
         } else {
           typedef __bf16 Bf8 __attribute__((ext_vector_type(8)));
-          acc[g][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(Bf8, x[m]), __builtin_bit_cast(Bf8, b[g]),
+          acc[g][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(Bf8, b[g]), __builtin_bit_cast(Bf8, x[m]),
                                                               acc[g][m], 0, 0, 0);
         }
       }
@@ -1195,18 +1195,30 @@ __global__ __launch_bounds__(256, 2) void DecodeMatrixPanelKernel(const PanelArg
   if (chunk + 1 < chunks) step(chunk + 1, std::integral_constant<int, 1>{});
   if (chunk + 2 < chunks) step(chunk + 2, std::integral_constant<int, 2>{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing lands in LDS after the workgroup
-  // acc[g][m][i] = D[input row 16 m + 4 q + i][output 16 g + n].
+  // acc[g][m][i] = D[output 16 g + 4 q + i][input row 16 m + n]: a lane's four sums are consecutive outputs of one row,
+  // stored together where the rows' places allow it (one by one, a lane's 80 stores were 4.7 us of the 64.5 of 300 rows).
+  const bool together = reinterpret_cast<uintptr_t>(a.y) % 16 == 0 && a.y_stride % 4 == 0;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const uint32_t out = out0 + out_half + 16 * g + n;
-    if (out < a.outputs) {
-      const float scale = a.w.tensor_scale != nullptr ? a.w.tensor_scale[(a.first + out) / a.w.rows_per_scale] : 1.0f;
+    const uint32_t out = out0 + out_half + 16 * g + 4 * q;
+    float scale[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+    if (a.w.tensor_scale != nullptr) {
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
+      for (int i = 0; i < 4; ++i) scale[i] = a.w.tensor_scale[(a.first + min(out + i, a.outputs - 1)) / a.w.rows_per_scale];
+    }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t t = t0 + 16 * m + 4 * q + i;
-          if (t < p.rows) a.y[t * a.y_stride + out] = acc[g][m][i] * scale;
+    for (int m = 0; m < MT; ++m) {
+      const uint32_t t = t0 + 16 * m + n;
+      if (t < p.rows) {
+        float* to = a.y + t * a.y_stride + out;
+        if (together && out + 4 <= a.outputs) {
+          *reinterpret_cast<float4*>(to) =
+              make_float4(acc[g][m][0] * scale[0], acc[g][m][1] * scale[1], acc[g][m][2] * scale[2], acc[g][m][3] * scale[3]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            if (out + i < a.outputs) to[i] = acc[g][m][i] * scale[i];
+          }
         }
       }
     }
@@ -1255,8 +1267,8 @@ MatrixTiles TilesOf(uint64_t outputs, uint64_t rows) {
 
 // The row tiles a wave of the laid-out form: the fewest microseconds by its kernel's costs (10 us a round of workgroups,
 // 0.42 us a chunk and 0.07 us a chunk and tile; LDS holds two workgroups of one tile, one of more, which side by side
-// take 0.6 us a chunk). 4096 -> 14336 with one to five: 300 rows 141, 121, 92, 102, 65 us, 64 rows 38, 45, 49, 53, 58,
-// 1,024 rows 489, 308, 234, 208, 233.
+// take 0.6 us a chunk). 4096 -> 14336 with one to five, before the sums were stored four at a time: 300 rows 141, 121, 92,
+// 102, 65 us, 64 rows 38, 45, 49, 53, 58, 1,024 rows 489, 308, 234, 208, 233.
 int PanelTiles(uint64_t outputs, uint64_t rows, uint32_t k) {
   const int cus = llmp_hip_compute_units();
   const uint64_t units = static_cast<uint64_t>(cus > 0 ? cus : 256), chunks = (k + 63ull) / 64ull;

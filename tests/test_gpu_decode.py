@@ -335,14 +335,15 @@ def test_matrix_laid_out_inputs_are_the_same_bits(device, decoder):
           for key, v in w.items() if key != "plain"}
     x = torch.from_numpy(synth.activations(300, k, 901)).to(device)
     lib, op = _lib.load(), ops._decode_operand(wd)
-    for rows in (17, 128, 190, 250, 300):
-        scratch = lib.llmp_hip_decode_matrix_scratch(ctypes.byref(op), 14290, rows)
+    # (Rows of 14,288 outputs take their sums four at a time, of 14,290 one by one.)
+    for rows, outputs in ((17, 14288), (128, 14290), (190, 14288), (250, 14290), (300, 14288)):
+        scratch = lib.llmp_hip_decode_matrix_scratch(ctypes.byref(op), outputs, rows)
         assert scratch == (rows + 15) // 16 * 2048 * ((k + 63) // 64)
-        want = torch.empty((rows, 14290), dtype=torch.float32, device=device)
-        _lib.check(lib.llmp_hip_decode_matrix(decoder, ctypes.byref(op), 7, 14290, x.data_ptr(), rows, k, want.data_ptr(),
-                                              14290, 0, None))
+        want = torch.empty((rows, outputs), dtype=torch.float32, device=device)
+        _lib.check(lib.llmp_hip_decode_matrix(decoder, ctypes.byref(op), 7, outputs, x.data_ptr(), rows, k, want.data_ptr(),
+                                              outputs, 0, None))
         torch.cuda.synchronize()
-        got = ops.decode_matrix(decoder, wd, x[:rows], first=7, outputs=14290)
+        got = ops.decode_matrix(decoder, wd, x[:rows], first=7, outputs=outputs)
         assert torch.equal(got.view(torch.int32), want.view(torch.int32)), rows
     want = oracle.decode_matrix(decoder, w, x[:33].cpu().numpy(), first=7, outputs=139, threads=oracle.max_threads())
     ok, worst = rel_close(ops.decode_matrix(decoder, wd, x[:33], first=7, outputs=139).cpu().numpy(), want, 1e-3)
