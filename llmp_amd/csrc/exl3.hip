@@ -1143,12 +1143,10 @@ size_t PassBytes(const llmp_exl3_weights& w, int rows) {
 }
 
 template <int CB, int BITS, int TILES>
-bool g_wide_sized = false;
-template <int CB, int BITS, int TILES>
 void LaunchWide(const llmp_exl3_weights& w, const WideSides& sides, int count, int m, int slices, hipStream_t stream) {
   constexpr int kRing = kProductWaves * kRingDepth * ((2 * kWideTiles * BITS * 32 + 1023) / 1024) * 1024;
   constexpr int kLds = kRing > kReduceBytes ? kRing : kReduceBytes;
-  if (!AllowLds(reinterpret_cast<const void*>(&WideProductKernel<CB, BITS, TILES>), kLds, &g_wide_sized<CB, BITS, TILES>)) return;
+  static_assert(kLds <= 64 * 1024, "more must be asked for, ahead of a capture too (llmp_hip_exl3_linear_static_prepare)");
   const int blocks = w.k / 128;
   const int per = (blocks + slices * kProductWaves - 1) / (slices * kProductWaves);
   const dim3 grid(static_cast<unsigned>(w.n / 64), static_cast<unsigned>(slices), static_cast<unsigned>(count));

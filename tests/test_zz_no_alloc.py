@@ -91,6 +91,34 @@ def test_static_scratch_linear_captured_in_a_graph_replays_bit_for_bit(device):
         assert torch.equal(y.view(torch.int32), want.view(torch.int32))
 
 
+def test_static_linear_of_more_than_sixteen_rows_captured_unrun(device):
+    """Prepared and never run before the capture: 32 rows of a linear whose wide passes fit the static array (the capture
+    meets launches only), replayed twice with eager work between."""
+    bits, codebook, k, n, m = 5, ops.EXL3_MCG, 1024, 512, 32
+    trellis, suh, svh = synth.exl3_weights(k, n, bits, 98)
+    weights = (dev(trellis, device), halves(suh, device), halves(svh, device), k, n, bits, codebook)
+    op = _lib.Exl3Linear()
+    op.weights, op.m = ops._exl3_weights(*weights), m
+    assert _lib.load().llmp_hip_exl3_linear_wide_scratch(C.byref(op)) <= 4 << 20
+    ops.exl3_linear_static_prepare(*weights)
+    x = torch.zeros((m, k), dtype=torch.float16, device=device)
+    a_had = torch.zeros((m, k), dtype=torch.float16, device=device)
+    y = torch.zeros((m, n), dtype=torch.float32, device=device)
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side, capture_error_mode="thread_local"):
+        ops.exl3_linear_static(*weights, x, a_had, y)
+    for seed in (99, 100):
+        fresh = halves(synth.rng(seed).standard_normal((m, k)).astype(np.float16), device)
+        x.copy_(fresh)
+        want = ops.exl3_linear(*weights, fresh, f32=True)  # eager work between the replays
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int32), want.view(torch.int32))
+
+
 def test_static_scratch_linear_refuses_what_exceeds_its_array(device):
     lib = _lib.load()
     op = _lib.Exl3Linear()
