@@ -1060,6 +1060,12 @@ int Disjoint(const char* what, const Range& written, std::initializer_list<Range
   }
   return 0;
 }
+bool Meets(const Range& area, std::initializer_list<Range> others) {
+  for (const Range& other : others) {
+    if (Overlap(area, other)) return true;
+  }
+  return false;
+}
 Range TrellisRange(const llmp_exl3_weights& w) {
   return {"the trellis", reinterpret_cast<uintptr_t>(w.trellis), static_cast<size_t>(w.k) * w.n * w.bits / 8};
 }
@@ -1362,17 +1368,21 @@ int LinearOver(const llmp_exl3_linear* op, void* area, size_t area_bytes, hipStr
   if ((reinterpret_cast<uintptr_t>(op->x) | reinterpret_cast<uintptr_t>(op->a_had) |
        reinterpret_cast<uintptr_t>(op->y) | reinterpret_cast<uintptr_t>(area)) % 8 != 0)
     return Refuse(1, "exl3.linear: operands not 8-byte aligned");
-  const bool wide = area_bytes >= llmp_hip_exl3_linear_wide_scratch(op);
-  const int pass = PassRows(op->m, op->weights.bits, wide);
+  int pass;
   {
     // validate.cc:120-126: what the launches write (a_had, y, the partial sums in place of the lock area) meets
     // nothing they read and not one another.
+    const llmp_exl3_weights& w = op->weights;
     const size_t m = static_cast<size_t>(op->m);
     const Range x{"x", reinterpret_cast<uintptr_t>(op->x), m * op->weights.k * 2};
     const Range a_had{"a_had", reinterpret_cast<uintptr_t>(op->a_had), m * op->weights.k * 2};
     const Range y{"y", reinterpret_cast<uintptr_t>(op->y), m * op->weights.n * (op->f32 ? 4 : 2)};
+    // The wide passes' part of the area may hold an operand (a caller's one arena): then passes of sixteen.
+    const size_t wide_bytes = llmp_hip_exl3_linear_wide_scratch(op);
+    const bool wide = area_bytes >= wide_bytes && !Meets({"the scratch", reinterpret_cast<uintptr_t>(area), wide_bytes},
+                                                         {x, a_had, y, TrellisRange(w), SuhRange(w), SvhRange(w)});
+    pass = PassRows(op->m, w.bits, wide);
     const Range partials{"the scratch", reinterpret_cast<uintptr_t>(area), PassBytes(op->weights, pass)};
-    const llmp_exl3_weights& w = op->weights;
     if (const int bad = Disjoint("exl3.linear", a_had, {x, y, TrellisRange(w), SuhRange(w), SvhRange(w), partials}); bad != 0) return bad;
     if (const int bad = Disjoint("exl3.linear", y, {x, TrellisRange(w), SuhRange(w), SvhRange(w), partials}); bad != 0) return bad;
     if (const int bad = Disjoint("exl3.linear", partials, {x, TrellisRange(w), SuhRange(w), SvhRange(w)}); bad != 0) return bad;
@@ -1563,14 +1573,20 @@ extern "C" int llmp_hip_exl3_multi_linear(const llmp_exl3_multi_linear* op, void
   if ((reinterpret_cast<uintptr_t>(op->x) | reinterpret_cast<uintptr_t>(op->a_had) |
        reinterpret_cast<uintptr_t>(op->y) | reinterpret_cast<uintptr_t>(scratch)) % 8 != 0)
     return Refuse(1, "exl3.multi_linear: operands not 8-byte aligned");
-  const bool wide = scratch_bytes >= llmp_hip_exl3_multi_linear_wide_scratch(op);
-  const int pass = PassRows(op->m, op->first.bits, wide);
+  int pass;
   {
     // validate.cc:310-323: a_had, y and the partial sums meet nothing the launches read and not one another.
     const size_t rows = static_cast<size_t>(op->m);
     const Range x{"x", reinterpret_cast<uintptr_t>(op->x), rows * op->first.k * 2};
     const Range a_had{"a_had", reinterpret_cast<uintptr_t>(op->a_had), 2 * rows * op->first.k * 2};
     const Range y{"y", reinterpret_cast<uintptr_t>(op->y), 2 * rows * op->first.n * (op->f32 ? 4 : 2)};
+    // The wide passes' part of the scratch may hold an operand (a caller's one arena): then passes of sixteen.
+    const size_t wide_bytes = llmp_hip_exl3_multi_linear_wide_scratch(op);
+    const bool wide =
+        scratch_bytes >= wide_bytes && !Meets({"the scratch", reinterpret_cast<uintptr_t>(scratch), wide_bytes},
+                                              {x, a_had, y, TrellisRange(op->first), SuhRange(op->first), SvhRange(op->first),
+                                               TrellisRange(op->second), SuhRange(op->second), SvhRange(op->second)});
+    pass = PassRows(op->m, op->first.bits, wide);
     const Range area{"the scratch", reinterpret_cast<uintptr_t>(scratch), 2 * PassBytes(op->first, pass)};
     for (const llmp_exl3_weights* w : {&op->first, &op->second}) {
       for (const Range& written : {a_had, y, area}) {
