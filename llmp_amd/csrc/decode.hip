@@ -1407,6 +1407,36 @@ int CheckOperand(const char* what, int decoder, const llmp_decode_operand* w, ui
   return 0;
 }
 
+// What the laid-out form's scratch meets of the operands that its launches read and write, or null: written there, an
+// operand would be gone before it is read. The rows [first, first + outputs) of the weight count, not all of it.
+const char* ScratchMeets(int decoder, const DecodeArgs& a, uint64_t rows, const void* scratch, size_t bytes) {
+  const uintptr_t from = reinterpret_cast<uintptr_t>(scratch);
+  auto meets = [&](const void* base, uint64_t begin, uint64_t end) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(base);
+    return base != nullptr && at + begin < from + bytes && from < at + end;
+  };
+  const llmp_decode_operand& w = a.w;
+  const uint64_t first = a.first, last = first + a.outputs;
+  if (meets(a.x, 0, ((rows - 1) * a.x_stride + w.k) * 4)) return "x";
+  if (meets(a.y, 0, ((rows - 1) * a.y_stride + a.outputs) * 4)) return "y";
+  if (meets(w.data, first * w.row_bytes, last * w.row_bytes)) return "the weight";
+  if (w.tensor_scale != nullptr && meets(w.tensor_scale, first / w.rows_per_scale * 4, ((last - 1) / w.rows_per_scale + 1) * 4))
+    return "the tensor scales";
+  if (decoder == LLMP_DECODER_AFFINE_SPLIT) {
+    if (meets(w.scales, first * w.scale_row_bytes, last * w.scale_row_bytes)) return "the scales";
+    const uint64_t zeros = (static_cast<uint64_t>(w.k / w.group) * w.bits + 7) / 8;
+    const uint64_t bias_row = (w.scale_type & 0x80u) != 0 ? zeros : w.scale_row_bytes;
+    if (meets(w.biases, first * bias_row, last * bias_row)) return "the biases";
+  } else if (SplitScales(decoder)) {
+    const bool nvfp4 = decoder == LLMP_DECODER_NVFP4_SPLIT || decoder == LLMP_DECODER_NVFP4_ATOMS;
+    const bool atoms = decoder == LLMP_DECODER_NVFP4_ATOMS || decoder == LLMP_DECODER_MXFP8_ATOMS || decoder == LLMP_DECODER_MXFP4_ATOMS;
+    const uint64_t blocks = w.k / (nvfp4 ? 16u : 32u);
+    if (meets(w.scales, (atoms ? first / 128 * 128 : first) * blocks, (atoms ? (last + 127) / 128 * 128 : last) * blocks))
+      return "the scales";
+  }
+  return nullptr;
+}
+
 // The launches of a product whose operands have been checked: four input rows a pass, or
 // fewer of a long row.
 int LaunchProduct(const char* what, int decoder, bool glu, DecodeArgs& a, uint64_t rows, hipStream_t s, int up_decoder = -1) {
@@ -1669,6 +1699,8 @@ extern "C" int llmp_hip_decode_matrix_staged(int decoder, const llmp_decode_oper
   const size_t staged = scratch == nullptr ? 0 : llmp_hip_decode_matrix_scratch(w, outputs, rows);
   if (staged > 0 && scratch_bytes >= staged) {
     if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0) return Refuse(1, "decode.matrix: scratch is 16-byte aligned");
+    if (const char* what = ScratchMeets(decoder, a, rows, scratch, staged); what != nullptr)
+      return Refuse(1, "decode.matrix: the scratch overlaps %s", what);
     const int tiles = PanelTiles(outputs, rows, w->k);
     switch (decoder) {
 #define LLMP_DECODER(ID) \

@@ -276,6 +276,40 @@ def test_decode_matrix_refuses_bad_operands():
     assert run(rows=0) > 0 and run(decoder=12) > 0 and run(first=60) > 0 and run(x=0x4004) > 0 and run(x_stride=100) > 0
 
 
+@pytest.mark.parametrize("decoder", range(12))
+def test_decode_matrix_refuses_scratch_over_its_operands(decoder):
+    """The laid-out form writes its scratch before it reads the weight, and reads it while it writes y: a scratch that holds the
+    first or the last byte of x, of y, or of the used rows of the weight, its scales, biases or tensor scales is refused."""
+    lib = _lib.load()
+    k, first, outputs, rows, total = 2048, 130, 4000, 1000, 4300
+    blocks = k // (16 if decoder in (3, 4, 5, 6) else 32)
+    w = _lib.DecodeOperand()
+    w.data, w.k, w.rows, w.rows_per_scale, w.row_bytes = 0x10000000, k, total, 100, 4096
+    w.tensor_scale = 0x30000000
+    spans = {"x": (0x50000000, 0x50000000 + ((rows - 1) * 2052 + k) * 4),
+             "y": (0x60000000, 0x60000000 + ((rows - 1) * 5000 + outputs) * 4),
+             "the weight": (0x10000000 + first * 4096, 0x10000000 + (first + outputs) * 4096),
+             "the tensor scales": (0x30000000 + 4, 0x30000000 + 42 * 4)}
+    if decoder == 11:
+        w.group, w.bits, w.scale_type, w.scale_row_bytes, w.biases = 32, 4, 1, 128, 0x40000000
+        w.scales = 0x20000000
+        spans["the scales"] = (0x20000000 + first * 128, 0x20000000 + (first + outputs) * 128)
+        spans["the biases"] = (0x40000000 + first * 128, 0x40000000 + (first + outputs) * 128)
+    elif decoder in (3, 7, 9):
+        w.scales = 0x20000000
+        spans["the scales"] = (0x20000000 + first * blocks, 0x20000000 + (first + outputs) * blocks)
+    elif decoder in (4, 8, 10):
+        w.scales = 0x20000000
+        spans["the scales"] = (0x20000000 + 128 * blocks, 0x20000000 + (first + outputs + 127) // 128 * 128 * blocks)
+    size = lib.llmp_hip_decode_matrix_scratch(C.byref(w), outputs, rows)
+    assert size > 0
+    for name, (begin, end) in spans.items():
+        for scratch in (begin // 16 * 16 - size + 16, (end - 1) // 16 * 16):
+            assert lib.llmp_hip_decode_matrix_staged(decoder, C.byref(w), first, outputs, 0x50000000, rows, 2052, 0x60000000,
+                                                     5000, 0, scratch, size, None) > 0, name
+            assert lib.llmp_hip_last_error().endswith(b"the scratch overlaps " + name.encode())
+
+
 def test_grouped_store_refusals_queue_nothing():
     lib = _lib.load()
     table = (_lib.SetRowsStore * 2)()
