@@ -580,10 +580,10 @@ int llmp_hip_decode_grouped(int decoder, const llmp_decode_operand* experts, uin
 int llmp_hip_decode_matrix(int decoder, const llmp_decode_operand* weight, uint64_t first, uint64_t outputs, const float* x,
                            uint64_t rows, uint64_t x_stride, float* y, uint64_t y_stride, int path, void* stream);
 
-/* The same product in two launches where that is faster (llmp_hip_decode_matrix_scratch says how many bytes of scratch it
- * then takes, and 0 where one launch is used): the first rounds the inputs to the matrix element and lays them out in the
- * scratch (16-byte aligned, the call's own until its work has run; those bytes meet no operand). The same bits; with less
- * scratch, or null, the one launch. */
+/* The same product in two launches where that is faster for the encoding and the sizes: the first rounds the inputs to the
+ * matrix element and lays them out in the scratch (16-byte aligned, the call's own until its work has run; its bytes meet no
+ * operand). llmp_hip_decode_matrix_scratch says how many bytes the two launches take, and 0 where one launch is faster
+ * whatever the encoding. The same bits either way; with less scratch, or null, the one launch. */
 size_t llmp_hip_decode_matrix_scratch(const llmp_decode_operand* weight, uint64_t outputs, uint64_t rows);
 int llmp_hip_decode_matrix_staged(int decoder, const llmp_decode_operand* weight, uint64_t first, uint64_t outputs,
                                   const float* x, uint64_t rows, uint64_t x_stride, float* y, uint64_t y_stride, int path,

@@ -1282,22 +1282,61 @@ MatrixTiles TilesOf(uint64_t outputs, uint64_t rows) {
   return {wide, wide && rows >= 256 && (outputs + 255) / 256 * ((rows + 255) / 256) >= units};
 }
 
-// The row tiles a wave of the laid-out form: the fewest microseconds by its kernel's costs (10 us a round of workgroups,
-// 0.42 us a chunk and 0.07 us a chunk and tile; LDS holds two workgroups of one tile, one of more, which side by side
-// take 0.6 us a chunk). 4096 -> 14336 with one to five, before the sums were stored four at a time: 300 rows 141, 121, 92,
-// 102, 65 us, 64 rows 38, 45, 49, 53, 58, 1,024 rows 489, 308, 234, 208, 233.
-int PanelTiles(uint64_t outputs, uint64_t rows, uint32_t k) {
+// The row tiles a wave of the laid-out form, and the rounds of workgroups that they make: the fewest microseconds by its
+// kernel's costs (10 us a round of workgroups, 0.42 us a chunk and 0.07 us a chunk and tile; LDS holds two workgroups of one
+// tile, one of more, which side by side take 0.6 us a chunk). NVFP4 4096 -> 14336 with one to five, before the sums were
+// stored four at a time: 300 rows 141, 121, 92, 102, 65 us, 64 rows 38, 45, 49, 53, 58, 1,024 rows 489, 308, 234, 208, 233.
+struct PanelShape {
+  int tiles;
+  uint64_t rounds;
+  bool paired;
+};
+PanelShape PanelTiles(uint64_t outputs, uint64_t rows, uint32_t k) {
   const int cus = llmp_hip_compute_units();
   const uint64_t units = static_cast<uint64_t>(cus > 0 ? cus : 256), chunks = (k + 63ull) / 64ull;
   uint64_t best = ~uint64_t{0};
-  int tiles = 1;
+  PanelShape shape{1, 1, false};
   for (int mt = 1; mt <= 5; ++mt) {
     const uint64_t groups = (outputs + kPanelOutputs - 1) / kPanelOutputs * ((rows + 32 * mt - 1) / (32 * mt));
     const uint64_t paired = mt == 1 && groups > units ? 2 : 1;
-    const uint64_t cost = (groups + paired * units - 1) / (paired * units) * (1000 + chunks * (paired == 2 ? 60 : 42 + 7 * mt));
-    if (cost < best) best = cost, tiles = mt;
+    const uint64_t rounds = (groups + paired * units - 1) / (paired * units);
+    const uint64_t cost = rounds * (1000 + chunks * (paired == 2 ? 60 : 42 + 7 * mt));
+    if (cost < best) best = cost, shape = {mt, rounds, paired == 2};
   }
-  return tiles;
+  return shape;
+}
+
+// Whether the laid-out form is the faster one: both forms' microseconds by what was measured. The one launch takes a round of
+// its workgroups for every CU's worth of tiles of 256 by 128 or 256, and of its small tiles, several of which share a CU, a
+// time with their number once there is more than one a CU; this form a round of its own tiles. So a product whose last round
+// of large tiles is full stays with the one launch (NVFP4 4096 -> 8192 at 2,048 rows: 197 us against 243), and where most of
+// that round is idle this form is up to 2.6 times faster (4096 -> 14336 at 200 rows: 134 against 52). Three kinds of
+// encoding differ enough to have costs of their own: 16-bit values, whose loads are what the small tiles wait for; the other
+// nine; and affine, whose loads lie under branches, so that this form waits for each where it is asked for. Over 8,097
+// products (twelve encodings, 1,024 to 14,336 outputs, K from 768, 17 to 4,096 rows) the choice by these costs is 0.3 %
+// from the better form's time in the mean, and 23 are more than 7 % slower than the other form, none more than 13 %; this
+// form wherever K has 12, 24 or 36 chunks (by the tiles) was 2.3 % and 877, the affine ones up to twice as slow.
+bool PanelPays(int decoder, uint64_t outputs, uint64_t rows, uint32_t k) {
+  const int cus = llmp_hip_compute_units();
+  const uint64_t units = static_cast<uint64_t>(cus > 0 ? cus : 256);
+  const double chunks = static_cast<double>((k + 63ull) / 64ull);
+  const bool affine = decoder == LLMP_DECODER_AFFINE_SPLIT;
+  const bool plain = decoder == LLMP_DECODER_BF16_DENSE || decoder == LLMP_DECODER_F16_DENSE;
+  const MatrixTiles t = TilesOf(outputs, rows);
+  double one;
+  if (t.wide) {
+    const uint64_t tile = t.tall ? 256 : 128;
+    const double rounds = static_cast<double>(((outputs + 255) / 256 * ((rows + tile - 1) / tile) + units - 1) / units);
+    one = rounds * (t.tall ? (affine ? 30.0 + 4.6 * chunks : 17.3 + 2.58 * chunks) : (affine ? 8.5 + 3.5 * chunks : 9.2 + 1.73 * chunks));
+  } else {
+    const double share = static_cast<double>((outputs + 63) / 64 * ((rows + 63) / 64)) / static_cast<double>(units);  // tiles a CU
+    const double more = share > 1.0 ? share : 1.0;
+    one = affine ? 4.0 + chunks * (0.95 + 0.4 * more) : 2.4 + chunks * more * (plain ? (rows <= 32 ? 0.62 : 0.88) : 0.72);
+  }
+  const PanelShape p = PanelTiles(outputs, rows, k);
+  const double chunk = affine ? (p.paired ? 2.2 : 1.55 + 0.13 * p.tiles) : (p.paired ? 0.85 : 0.31 + 0.09 * p.tiles);
+  const double laid_out = affine ? 4.0 + p.rounds * (8.3 + chunks * chunk) : 4.6 + p.rounds * (7.4 + chunks * chunk);
+  return laid_out <= one;
 }
 
 size_t DecodeLds(int tokens, uint32_t k) { return static_cast<size_t>(tokens) * (k / 16u) * kSegmentStride; }
@@ -1661,9 +1700,7 @@ extern "C" int llmp_hip_decode_grouped(int decoder, const llmp_decode_operand* e
 extern "C" size_t llmp_hip_decode_matrix_scratch(const llmp_decode_operand* w, uint64_t outputs, uint64_t rows) {
   if (w == nullptr || outputs == 0 || rows == 0 || rows > 65535ull * 64ull || w->k == 0 || w->k > (1u << 26)) return 0;
   const MatrixTiles t = TilesOf(outputs, rows);
-  // The inputs' launch and the start and end of a round are paid back by the chunks. Measured at 1,024 and 2,048 values of
-  // K, the old form against this one: tiles of 64 by 64 13.0-17.6 us against 14.0-18.3 and 24.6-26.7 against 21.8-24.4;
-  // of 256 by 128 36.6 against 32.2 (26.7 both at 512); of 256 by 256 77 against 92 (235 against 208 at 4,096).
+  // Below these no encoding is faster with it (PanelPays, which knows the encoding, decides above them).
   const uint64_t chunks = (w->k + 63ull) / 64ull;
   if (chunks < (t.tall ? 36u : t.wide ? 12u : 24u)) return 0;
   return (rows + 15) / 16 * chunks * 2048;
@@ -1697,11 +1734,11 @@ extern "C" int llmp_hip_decode_matrix_staged(int decoder, const llmp_decode_oper
   const bool wide = t.wide, tall = t.tall;
   const auto s = static_cast<hipStream_t>(stream);
   const size_t staged = scratch == nullptr ? 0 : llmp_hip_decode_matrix_scratch(w, outputs, rows);
-  if (staged > 0 && scratch_bytes >= staged) {
+  if (staged > 0 && scratch_bytes >= staged && PanelPays(decoder, outputs, rows, w->k)) {
     if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0) return Refuse(1, "decode.matrix: scratch is 16-byte aligned");
     if (const char* what = ScratchMeets(decoder, a, rows, scratch, staged); what != nullptr)
       return Refuse(1, "decode.matrix: the scratch overlaps %s", what);
-    const int tiles = PanelTiles(outputs, rows, w->k);
+    const int tiles = PanelTiles(outputs, rows, w->k).tiles;
     switch (decoder) {
 #define LLMP_DECODER(ID) \
   case ID: LaunchPanel<ID>(a, static_cast<uint32_t>(rows), tiles, static_cast<uint8_t*>(scratch), s); break;

@@ -353,26 +353,37 @@ def test_matrix_laid_out_inputs_are_the_same_bits(device, decoder):
 @pytest.mark.parametrize("decoder", list(range(12)))
 def test_matrix_laid_out_inputs_at_three_and_no_chunks_past_the_loop(device, decoder):
     """The two-launch form's loop takes four chunks of 64 at a time: K with three chunks left over (the last one whole or
-    partial, as the encoding's blocks allow) and with none, against the one launch bit for bit, one to five row tiles a wave;
-    an infinity and a NaN in the inputs stay in their rows."""
-    n, outputs = 14300, 14288
+    partial, as the encoding's blocks allow; two where they make the count even) and with none, against the one launch bit for
+    bit, one to five row tiles a wave. The scratch shows that the form ran; an infinity and a NaN in the inputs stay in their
+    rows."""
+    n, outputs = 4096, 32700
     lib = _lib.load()
     whole = decoder in (8, 10)  # blocks of 128: an even count of chunks
     for k in (1664,) if whole else (1728 if decoder in (4, 6) else 1712 if decoder in (0, 1, 3, 5) else 1696, 1792):
-        w = synth.affine_weight(n, k, 950, bits=4, group=32, scale="f16") if decoder == 11 else \
+        w = synth.affine_weight(n, k, 950, bits=4, group=32, scale="f16", tensor_scales=4) if decoder == 11 else \
             synth.decode_weight(decoder, n, k, 950 + decoder, tensor_scales=4)
-        wd = {key: (torch.from_numpy(np.ascontiguousarray(v)).to(device) if isinstance(v, np.ndarray) else v)
-              for key, v in w.items() if key != "plain"}
+        wd = {}
+        for key, v in w.items():
+            if isinstance(v, np.ndarray):  # eight times the rows (whole scale atoms)
+                v = torch.from_numpy(np.ascontiguousarray(v)).to(device)
+                v = v.repeat(8, *[1] * (v.dim() - 1))
+            if key != "plain":
+                wd[key] = v
         op = ops._decode_operand(wd)
-        x = torch.from_numpy(synth.activations(300, k, 951)).to(device)
+        x = torch.from_numpy(synth.activations(150, k, 951)).to(device)
         x[3, 5], x[9, k - 1] = float("inf"), float("nan")
-        for rows in (17, 128, 190, 250, 300):
-            assert lib.llmp_hip_decode_matrix_scratch(ctypes.byref(op), outputs, rows) > 0
+        for rows in (20, 50, 80, 120, 150):
+            size = lib.llmp_hip_decode_matrix_scratch(ctypes.byref(op), outputs, rows)
+            assert size == (rows + 15) // 16 * 2048 * ((k + 63) // 64)
             want = torch.empty((rows, outputs), dtype=torch.float32, device=device)
             _lib.check(lib.llmp_hip_decode_matrix(decoder, ctypes.byref(op), 7, outputs, x.data_ptr(), rows, k, want.data_ptr(),
                                                   outputs, 0, None))
+            scratch = torch.full((size,), 0xA5, dtype=torch.uint8, device=device)
+            got = torch.empty_like(want)
+            _lib.check(lib.llmp_hip_decode_matrix_staged(decoder, ctypes.byref(op), 7, outputs, x.data_ptr(), rows, k,
+                                                         got.data_ptr(), outputs, 0, scratch.data_ptr(), size, None))
             torch.cuda.synchronize()
-            got = ops.decode_matrix(decoder, wd, x[:rows], first=7, outputs=outputs)
+            assert not bool((scratch[:1024] == 0xA5).all())
             finite = torch.isfinite(want)
             assert finite.sum() == (rows - 2) * outputs
             assert torch.equal(finite, torch.isfinite(got)), (k, rows)

@@ -1,7 +1,8 @@
-"""What the EXL3 linears ask the HIP runtime for. The runtime's calls are counted by tests/host/counted_runtime.cc; no GPU, and
-the operands are addresses that nothing reads. llmp_hip_exl3_linear_static after llmp_hip_exl3_linear_static_prepare:
-launches and nothing else, whatever the rows (include/llmp_hip.h: a capture may refuse any other call). The linears over a
-scratch larger than they need: which passes they take."""
+"""What the EXL3 linears and the stored encodings' matrix product ask the HIP runtime for. The runtime's calls are counted by
+tests/host/counted_runtime.cc; no GPU, and the operands are addresses that nothing reads. The matrix product: which of its
+forms it takes. llmp_hip_exl3_linear_static after llmp_hip_exl3_linear_static_prepare: launches and nothing else, whatever
+the rows (include/llmp_hip.h: a capture may refuse any other call). The linears over a scratch larger than they need: which
+passes they take."""
 import os
 import subprocess
 import sys
@@ -79,6 +80,35 @@ for make, name in ((linear, "linear"), (multi, "multi_linear")):
         assert b"overlaps" in lib.llmp_hip_last_error()
 """
 
+# (encoding, K, outputs, rows, launches): on both sides of the choice between the matrix product's one launch and its two, by
+# the times of both on the device (256 compute units, which the library also takes where it cannot ask).
+MATRIX = """
+def launched(decoder, k, outputs, rows):
+    w = _lib.DecodeOperand()
+    w.data, w.scales, w.k, w.rows, w.rows_per_scale, w.row_bytes = 0x10000000, 0x8000000000, k, outputs, outputs, 2 * k
+    if decoder == 11:
+        w.group, w.bits, w.scale_type, w.scale_row_bytes = 32, 4, 1, k // 16
+    size = lib.llmp_hip_decode_matrix_scratch(C.byref(w), outputs, rows)
+    before = launches.value
+    _lib.check(lib.llmp_hip_decode_matrix_staged(decoder, C.byref(w), 0, outputs, 0x9000000000, rows, k, 0xA000000000, outputs, 0,
+                                                 0xB000000000, size, None))
+    return launches.value - before
+
+for case in CASES:
+    assert launched(*case[:4]) == case[4], case
+"""
+
+CASES = [
+    (3, 4096, 14336, 300, 2), (3, 1024, 14336, 300, 2), (3, 4096, 14336, 200, 2), (9, 4096, 4096, 1024, 2), (0, 768, 8192, 400, 2),
+    (3, 4096, 4096, 17, 2), (7, 4096, 14336, 1024, 2), (0, 4096, 2048, 64, 2),
+    # A full round of tiles of 256 by 256 or, at a short K, of 256 by 128.
+    (3, 4096, 8192, 2048, 1), (1, 4096, 8192, 2048, 1), (0, 1024, 14336, 512, 1), (7, 768, 4096, 2048, 1),
+    # Small tiles, one a compute unit, and a short K.
+    (2, 1536, 2048, 17, 1), (9, 1536, 2048, 300, 1), (0, 1536, 14336, 17, 1),
+    # Affine: only where the one launch leaves much of its round idle.
+    (11, 4096, 14336, 17, 1), (11, 4096, 14336, 512, 1), (11, 4096, 14336, 2048, 1), (11, 2048, 2048, 300, 1),
+    (11, 4096, 14336, 300, 2), (11, 4096, 4096, 1024, 2)]
+
 
 def run(tmp_path, program):
     shared = os.path.join(tmp_path, "counted_runtime.so")
@@ -94,3 +124,7 @@ def test_a_prepared_static_linear_asks_for_nothing_but_launches(tmp_path):
 
 def test_an_arena_that_holds_operands_behind_the_least_scratch_is_accepted(tmp_path):
     run(tmp_path, ARENA)
+
+
+def test_the_matrix_product_takes_the_faster_form(tmp_path):
+    run(tmp_path, MATRIX.replace("CASES", repr(CASES)))
