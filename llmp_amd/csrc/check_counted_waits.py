@@ -7,6 +7,10 @@ their way; a branch goes both ways, except over an empty execution mask, which n
 decode.hip, the matrix product over laid-out inputs: inputs go to LDS three chunks ahead, a barrier a chunk. At a barrier
 only those asked for since the barrier before may be on their way (at the first, and at the end, none).
 
+exl3.hip, the packed products: words and activations are loaded into registers by instructions, from LDS and from memory.
+From such a load to the wait that covers it, past the loop too, no instruction may name a register that it writes: the
+compiler takes them for written, copies them, and gives those that nothing reads to other values.
+
 Needs hipcc, no GPU. Run by the library's build (__graft_entry__.build) and by tests/test_counted_waits.py;
 `python check_counted_waits.py` runs it alone."""
 import os
@@ -119,6 +123,49 @@ def check_panel(name, body):
     follow(body, (True, ()), step)
 
 
+def registers(code):
+    """The vector registers an instruction names."""
+    named = set()
+    for a, b in re.findall(r"\bv\[(\d+):(\d+)\]", code):
+        named.update(range(int(a), int(b) + 1))
+    named.update(int(v) for v in re.findall(r"\bv(\d+)\b", code))
+    return frozenset(named)
+
+
+def check_registers(name, body):
+    """Raises AssertionError where an instruction names a register that a load written by hand has yet to write."""
+    assert "scratch_" not in body, f"{name}: spills"
+    nothing = frozenset()
+
+    def step(code, own, state):
+        memory, lds = state  # oldest first: the registers that each operation on its way writes (of loads written by hand)
+        touched = registers(code) & nothing.union(*memory, *lds) if memory or lds else nothing
+        assert not touched, f"{name}: `{code}` names v{sorted(touched)} while a load to it is on its way"
+        if code.startswith("ds_"):
+            lds += (registers(code.split(",")[0]) if own and code.startswith("ds_read") else nothing,)
+        elif code.startswith("s_load"):
+            lds += (nothing,)
+        elif MEMORY.match(code):
+            to_register = own and re.match(r"global_load_dword(x[234])?\s", code)
+            memory += (registers(code.split(",")[0]) if to_register else nothing,)
+        elif code.startswith("s_waitcnt"):
+            left = re.search(r"vmcnt\((\d+)\)", code)
+            if left:
+                memory = after_wait(memory, int(left.group(1)))
+            left = re.search(r"lgkmcnt\((\d+)\)", code)
+            if left:
+                lds = after_wait(lds, int(left.group(1)))
+        elif code.startswith("s_endpgm"):
+            assert not any(memory) and not any(lds), f"{name}: a load to a register on its way at the end"
+        while memory and not memory[0]:
+            memory = memory[1:]
+        while lds and not lds[0]:
+            lds = lds[1:]
+        return memory, lds
+
+    follow(body, ((), ()), step)
+
+
 def check():
     """The number of kernels followed; raises AssertionError (or the compiler's error) where a count does not hold."""
     kernels = 0
@@ -126,7 +173,12 @@ def check():
         check_panel(name, body)
         kernels += 1
     assert kernels >= 5, f"only {kernels} kernels of the matrix product over laid-out inputs were found"
-    return kernels
+    products = 0
+    for name, body in kernels_of(assembly_of("exl3.hip"), "WideProductKernel|13ProductKernel"):
+        check_registers(name, body)
+        products += 1
+    assert products >= 48, f"only {products} packed products were found"
+    return kernels + products
 
 
 if __name__ == "__main__":

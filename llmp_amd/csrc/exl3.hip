@@ -832,8 +832,17 @@ __global__ __launch_bounds__(kProductWaves * 64) void ProductKernel(const Produc
       one(step, 0);
       one(step + 1, 1);
     }
-    LdsWaited();  // the words asked for past the end
+    // What was asked for past the end lands before its registers and LDS are anything else's: tied, they are in use till then.
+    LdsWaited();
+    landed(words[0]);
     LoadsWaited<0>();
+    if constexpr (kFused) {
+#pragma unroll
+      for (int i = 0; i <= kFusedRows; ++i) LLMP_TIE(held[i]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) LLMP_TIE(xq[i]);
+    }
   }
 
   // The waves' sums through LDS (over the rings, which every wave has left), added in wave
@@ -933,6 +942,13 @@ __global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const Wi
     }
   };
 
+  auto landed = [&](uint32_t (&words)[2 * kWideTiles][kWords]) {
+#pragma unroll
+    for (int t = 0; t < 2 * kWideTiles; ++t)
+#pragma unroll
+      for (int w = 0; w < kWords; ++w) LLMP_TIE(words[t][w]);
+  };
+
   V4f acc[TILES][kWideTiles];
 #pragma unroll
   for (int r = 0; r < TILES; ++r)
@@ -961,10 +977,7 @@ __global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const Wi
       fetch(step + kRingDepth - 1);
       LoadsWaited<kLoads*(kRingDepth - 2) + TILES>();
       LdsWaited();
-#pragma unroll
-      for (int t = 0; t < 2 * kWideTiles; ++t)
-#pragma unroll
-        for (int w = 0; w < kWords; ++w) LLMP_TIE(mine[t][w]);
+      landed(mine);
       ask(step + 1, words[parity ^ 1]);
       Half8 wv[kWideTiles];
 #pragma unroll
@@ -988,8 +1001,12 @@ __global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const Wi
       one(step, 0);
       one(step + 1, 1);
     }
+    // (As in the product of sixteen rows: nothing asked for past the end is left on its way to a register.)
     LdsWaited();
+    landed(words[0]);
     LoadsWaited<0>();
+#pragma unroll
+    for (int r = 0; r < TILES; ++r) LLMP_TIE(x[r]);
   }
 
   // The waves' sums in wave order through LDS, 32 rows at a time: [wave][row tile][4 t + q][lane].

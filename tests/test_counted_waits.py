@@ -19,7 +19,7 @@ def module():
 
 
 def test_counted_waits_hold_on_every_path(module):
-    assert module.check() >= 5
+    assert module.check() >= 53
 
 
 @pytest.mark.parametrize("left,weights,holds", [(9, 4, True), (9, 3, False), (1, 0, True)])
@@ -34,3 +34,17 @@ def test_a_wait_that_counts_loads_that_are_not_there_is_found(module, left, weig
     else:
         with pytest.raises(AssertionError, match="loads to LDS may still"):
             module.check_panel("kernel", body)
+
+
+@pytest.mark.parametrize("between,holds", [("v_add_f32_e32 v5, v1, v2", True), ("v_mov_b32_e32 v8, v1", False),
+                                           ("v_mov_b32_e32 v1, v7", False), ("ds_read_b32 v7, v2", False)])
+def test_a_register_named_while_a_load_to_it_is_on_its_way_is_found(module, between, holds):
+    """Past the loop, two loads whose results nothing reads any more, before the waits that close it."""
+    body = "\n".join(
+        [".LBB0_1:", "\ts_waitcnt vmcnt(0) lgkmcnt(0)", "\t;;#ASMSTART", "\tglobal_load_dwordx2 v[7:8], v[2:3], off",
+         "\t;;#ASMEND", "\ts_cbranch_scc1 .LBB0_1", "\t" + between, "\ts_waitcnt vmcnt(0)", "\ts_endpgm"])
+    if holds:
+        module.check_registers("kernel", body)
+    else:
+        with pytest.raises(AssertionError, match="on its way"):
+            module.check_registers("kernel", body)
