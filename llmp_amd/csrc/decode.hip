@@ -1085,7 +1085,7 @@ __global__ __launch_bounds__(256, 2) void DecodeMatrixPanelKernel(const PanelArg
   auto load_input = [&](uint32_t chunk, int i) {
     const uint32_t offset = min(chunk, chunks - 1) * 2048u + lane * 16u;
     const uint32_t to = inputs_at + (chunk & 3u) * kInputBytes + wave * (MT * 1024) + i * 1024;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(from[i]) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(offset), "s"(from[i]) : "memory", "m0");
   };
   auto read_input = [&](uint32_t chunk, int j, int m) {
     return *reinterpret_cast<const U32x4*>(stages + (chunk & 3u) * kInputBytes + (wave >> 1) * (MT * 2048) + m * 2048 + j * 1024 + lane * 16);
