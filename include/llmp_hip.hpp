@@ -345,14 +345,14 @@ inline std::size_t WideScratchBytes(const LinearOperands& o) {
   const llmp_exl3_linear abi = ToAbi(o);
   return llmp_hip_exl3_linear_wide_scratch(&abi);
 }
-// PackedGemvLinear / PackedGemmLinear of src/kernels/exl3/linear.h:47-54, 1 to 65536 rows in passes of sixteen
-// (up to 144 where the scratch has WideScratchBytes).
-// UpstreamPath of src/kernels/exl3/validate.h:254-256: the packed path through 144 rows (the reconstruction paths
-// it names above that are not built here; the packed path still takes those rows).
+// UpstreamPath of src/kernels/exl3/validate.h:254-256: the packed path through 144 rows, the reconstruction paths above
+// (llmp_hip_exl3_linear_reconstructed; the packed path takes those rows too).
 enum class LinearPath : std::uint8_t { kPacked, kReconstruct, kReconstructFused };
 constexpr LinearPath UpstreamPath(int rows) {
   return rows >= 1024 ? LinearPath::kReconstructFused : rows > 144 ? LinearPath::kReconstruct : LinearPath::kPacked;
 }
+// PackedGemvLinear / PackedGemmLinear of src/kernels/exl3/linear.h:47-54, 1 to 65536 rows in passes of sixteen
+// (up to 144 where the scratch has WideScratchBytes).
 inline KernelFailure PackedLinear(const LinearOperands& o, void* scratch, std::size_t scratch_bytes, void* stream) {
   const llmp_exl3_linear abi = ToAbi(o);
   return FromStatus(llmp_hip_exl3_linear(&abi, scratch, scratch_bytes, stream));
@@ -386,6 +386,10 @@ inline llmp_exl3_multi_linear ToAbi(const MultiLinearOperands& o) {
 inline std::size_t ScratchBytes(const MultiLinearOperands& o) {
   const llmp_exl3_multi_linear abi = ToAbi(o);
   return llmp_hip_exl3_multi_linear_scratch(&abi);
+}
+inline std::size_t WideScratchBytes(const MultiLinearOperands& o) {
+  const llmp_exl3_multi_linear abi = ToAbi(o);
+  return llmp_hip_exl3_multi_linear_wide_scratch(&abi);
 }
 // MultiLinear of src/kernels/exl3/linear.h:51-53.
 inline KernelFailure MultiLinear(const MultiLinearOperands& o, void* scratch, std::size_t scratch_bytes, void* stream) {
@@ -543,11 +547,11 @@ inline std::vector<Implementation> Implementations() {
   }
   // EXL3 (exl3/implementations.h:8-31): the packed paths and the reconstruction paths.
   add("exl3.linear.gemv", "quant_linear", {"exl3"}, {1, 8, 128, 128}, Rung::kOnChipDecode, kBf16Mma, {"llmp_hip_exl3_linear"},
-      "trellis tiles as the second operand of a 16 x 16 x 16 F16 matrix instruction");
+      "pairs of trellis tiles as the second operand of a 16 x 16 x 32 F16 matrix instruction");
   add("exl3.linear.gemm", "quant_linear", {"exl3"}, {1, 65536, 128, 128}, Rung::kOnChipDecode, kBf16Mma, {"llmp_hip_exl3_linear"},
-      "the same launches in passes of sixteen rows");
+      "the same launches in passes of sixteen rows, of up to 144 with WideScratchBytes");
   add("exl3.multi_linear.mgemm", "quant_multi_linear", {"exl3"}, {1, 65536, 128, 128}, Rung::kOnChipDecode, kBf16Mma,
-      {"llmp_hip_exl3_multi_linear"}, "gate and up in grid z, passes of sixteen rows");
+      {"llmp_hip_exl3_multi_linear"}, "gate and up in grid z, the same passes");
   // (Upstream's choice of path by rows, UpstreamPath above; the entry point itself takes any number from one.)
   add("exl3.linear.reconstruct", "quant_linear", {"exl3"}, {145, 65536, 128, 128}, Rung::kBf16Decode, kBf16Mma,
       {"llmp_hip_exl3_linear_reconstructed"}, "input transform, rotated weights to F16 and an F16 product a slice, output transform");

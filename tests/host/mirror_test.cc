@@ -140,7 +140,12 @@ void HostChecks() {
   EXPECT(!hipk::LastError().empty());
   hipk::exl3::MultiLinearOperands multi;
   EXPECT(hipk::exl3::MultiLinear(multi, nullptr, 0, nullptr) == hipk::KernelFailure::kRejected);
-  EXPECT(hipk::exl3::ScratchBytes(multi) == 0);
+  EXPECT(hipk::exl3::ScratchBytes(multi) == 0 && hipk::exl3::WideScratchBytes(multi) == 0);
+  // Two linears of 77 rows, each with the wide passes' scratch of one.
+  linear.weights.k = 512, linear.weights.n = 256, linear.weights.bits = 4, linear.m = 77;
+  multi.first = multi.second = linear.weights, multi.m = 77;
+  EXPECT(hipk::exl3::WideScratchBytes(linear) > hipk::exl3::ScratchBytes(linear));
+  EXPECT(hipk::exl3::WideScratchBytes(multi) == 2 * hipk::exl3::WideScratchBytes(linear));
 }
 
 // The registry's entries (include/llmp_hip.hpp, namespace execution) against the names the reference's planner and
