@@ -13,6 +13,7 @@ compiler takes them for written, copies them, and gives those that nothing reads
 
 Needs hipcc, no GPU. Run by the library's build (__graft_entry__.build) and by tests/test_counted_waits.py;
 `python check_counted_waits.py` runs it alone."""
+import functools
 import os
 import re
 import shutil
@@ -27,6 +28,7 @@ MEMORY = re.compile(r"(global|buffer|flat|scratch)_(load|store|atomic)")
 BRANCH = re.compile(r"s_(cbranch_\w+|branch)\s+(\S+)")
 
 
+@functools.lru_cache(maxsize=None)
 def assembly_of(source):
     """The compiler's gfx950 assembly of a source of this folder, with the library's flags."""
     with tempfile.TemporaryDirectory() as tmp:

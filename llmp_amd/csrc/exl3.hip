@@ -297,15 +297,15 @@ __global__ __launch_bounds__(256) void ReconstructTransposedKernel(const uint32_
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const Place p = PlaceOf(lane);
-  // Sixteen of a block's 64 tiles a wave. A lane's four states lie within three consecutive words of a tile's
-  // stream, the same three in every tile: they are asked for from all sixteen tiles before the first is decoded (a
+  // Sixteen of a block's 64 tiles a wave. A lane's four states lie within two (above five bits three) consecutive words
+  // of a tile's stream, the same in every tile: they are asked for from all sixteen tiles before the first is decoded (a
   // tile after the other, each decode would wait for its own loads), and a workgroup goes through its blocks (every
-  // gridDim.x-th, columns fastest) with the next block's words asked for ahead of this block's transforms.
-  constexpr int kWords = BITS * 8;
+  // gridDim.x-th, columns fastest) with the next block's words asked for ahead of this block's way out.
+  constexpr int kWords = BITS * 8, kHeld = BITS <= 5 ? 2 : 3;
   const int word0 = (((p.first + 1) * BITS + 256 * BITS - 16) >> 5) % kWords;
   const int blocks_n = columns / 128;
   const int blocks = blocks_n * (k / 128);
-  uint32_t words[16][3];
+  uint32_t words[16][kHeld];
   auto ask = [&](int block) {
     const int k_at = (block / blocks_n) * 128, c_at = (block % blocks_n) * 128;
 #pragma unroll
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256) void ReconstructTransposedKernel(const uint32_
       const uint32_t* tile =
           trellis + (static_cast<int64_t>(k_at / 16 + kt) * (n / 16) + (column + c_at) / 16 + nt) * kWords;
 #pragma unroll
-      for (int i = 0; i < 3; ++i) words[u][i] = tile[(word0 + i) % kWords];
+      for (int i = 0; i < kHeld; ++i) words[u][i] = tile[(word0 + i) % kWords];
     }
   };
   if (static_cast<int>(blockIdx.x) < blocks) ask(blockIdx.x);
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256) void ReconstructTransposedKernel(const uint32_
     const int kt = t >> 3, nt = t & 7;
     const Half4 v = DecodeFour<CB, BITS>(p.first, [&](int i) {
       const int d = (i - word0 + kWords) % kWords;
-      return d == 0 ? words[u][0] : d == 1 ? words[u][1] : words[u][2];
+      return d == 0 ? words[u][0] : (kHeld == 2 || d == 1) ? words[u][1] : words[u][kHeld - 1];
     });
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
