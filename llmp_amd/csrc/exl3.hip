@@ -214,8 +214,9 @@ __device__ __forceinline__ void Hadamard128(float& a, float& b, int lane) {
 // y = f(H(x * in_scale)) * r * out_scale over each 128 block of each row; grid (rows, columns
 // / 128), a wave a block. X / Y: 0 F16, 1 F32. `slices` partial inputs are added in order first.
 // One or two transforms a launch (grid z): a linear's, or the two of a gate/up pair.
-// An F16 result is stored a second time, in the order in which the product of many rows reads its operand (see
-// WideProductKernel), where `operand` is given.
+// kOperand: an F16 result is stored a second time, in the order in which the product of many rows reads its operand (see
+// WideProductKernel). A kernel of its own: asked at run time, the question and the grid's size among the arguments cost the
+// other transforms half a microsecond of 4.
 struct HadamardSides {
   const void* x[2];
   void* y[2];
@@ -227,7 +228,7 @@ inline HadamardSides OneSide(const void* x, void* y, const uint16_t* in_scale, c
   return HadamardSides{{x, x}, {y, y}, {in_scale, in_scale}, {out_scale, out_scale}, {nullptr, nullptr}};
 }
 
-template <int X, int Y>
+template <int X, int Y, bool kOperand = false>
 __global__ __launch_bounds__(64) void HadamardKernel(const HadamardSides sides, int columns, int slices,
                                                     int64_t slice_stride) {
   // No fused multiply-adds: the transform inside the product kernel rounds every step the same way, so that a
@@ -270,7 +271,7 @@ __global__ __launch_bounds__(64) void HadamardKernel(const HadamardSides sides, 
   if constexpr (Y == 0) {
     const uint32_t packed = FloatToHalfBits(a) | (FloatToHalfBits(b) << 16);
     *reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(y) + at) = packed;
-    if (sides.operand[blockIdx.z] != nullptr) {
+    if constexpr (kOperand) {
       // Values c and c + 1 of 32 inputs: the K step of sixteen they are of, the lane group and the half of its four.
       const int row = blockIdx.x, pair = c >> 5, step = (c >> 4) & 1, half = (c >> 3) & 1, g = (c & 7) >> 1;
       const int tiles = (gridDim.x + 15) / 16;
@@ -1304,9 +1305,12 @@ int LaunchLinears(const llmp_exl3_weights* const (&w)[2], int count, const void*
   if (!fused) {
     const HadamardSides in{{x, x}, {a_had[0], a_had[1]}, {suh0, suh1}, {nullptr, nullptr},
                            {reinterpret_cast<uint32_t*>(operand[0]), reinterpret_cast<uint32_t*>(operand[1])}};
-    hipLaunchKernelGGL((HadamardKernel<0, 0>),
-                       dim3(static_cast<unsigned>(m), static_cast<unsigned>(w0.k / 128), static_cast<unsigned>(count)),
-                       dim3(64), 0, s, in, w0.k, 1, int64_t{0});
+    const dim3 grid(static_cast<unsigned>(m), static_cast<unsigned>(w0.k / 128), static_cast<unsigned>(count));
+    if (wide) {
+      hipLaunchKernelGGL((HadamardKernel<0, 0, true>), grid, dim3(64), 0, s, in, w0.k, 1, int64_t{0});
+    } else {
+      hipLaunchKernelGGL((HadamardKernel<0, 0>), grid, dim3(64), 0, s, in, w0.k, 1, int64_t{0});
+    }
     if (const int bad = LaunchStatus(what); bad != 0) return bad;
   }
   ProductSides sides;

@@ -2,6 +2,7 @@
 of the build), and the check sees a wait that is one short. Needs hipcc, no GPU; fails, not skips, where hipcc is missing."""
 import importlib.util
 import os
+import re
 
 import pytest
 
@@ -43,6 +44,15 @@ def test_the_reconstructions_words_are_selected_without_branches(module):
     assert len(kernels) >= 45  # three codebooks by five rates: transposed, and the weights themselves both ways
     for name, body in kernels:
         assert "s_cbranch_execz" not in body[body.find("ds_write"):body.rfind("ds_write")], name
+
+
+def test_only_the_wide_products_transform_asks_for_the_grid(module):
+    """The transform that lays its result out for the product of many rows needs the grid's size, which comes with 256 bytes
+    of arguments; the others take their own, fewer than 128 bytes, and no more."""
+    described = module.assembly_of("exl3.hip").split("amdhsa.kernels:")[1].split("- .agpr_count:")[1:]
+    sizes = [int(re.search(r"\.kernarg_segment_size: (\d+)", d).group(1)) for d in described
+             if re.search(r"\.name: +\S*HadamardKernelILi[01]ELi[01]ELb0E", d)]
+    assert len(sizes) >= 3 and max(sizes) < 128, sizes
 
 
 @pytest.mark.parametrize("between,holds", [("v_add_f32_e32 v5, v1, v2", True), ("v_mov_b32_e32 v8, v1", False),
