@@ -148,23 +148,50 @@ __device__ __forceinline__ int RowOf(int g, int j) { return 2 * g + (j & 1) + 8 
 // bits a value the four states lie within 31 bits of the stream, so within the two words from
 // the first state's first bit: one 64-bit shift brings the last state to bit 0 and the others
 // sit at fixed offsets above it.
+// Up to five bits, from the word that holds the first state's first bit and the next.
+template <int CB, int BITS>
+__device__ __forceinline__ Half4 DecodeFour(int first, uint32_t word, uint32_t next) {
+  static_assert(BITS <= 5, "four states of more bits lie within three words");
+  Half4 v;
+  const int end0 = (first + 1) * BITS + 256 * BITS;                      // past the first state's last bit, a period ahead
+  const int shift = 32 * ((end0 - 16) >> 5) + 64 - (end0 + 3 * BITS);  // 2 .. 45
+  const uint64_t merged = (static_cast<uint64_t>(word) << 32) | next;
+  const uint32_t window = static_cast<uint32_t>(merged >> shift);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = Codebook<CB>((window >> ((3 - j) * BITS)) & 0xFFFFu);
+  return v;
+}
 template <int CB, int BITS, typename WordFn>
 __device__ __forceinline__ Half4 DecodeFour(int first, WordFn word) {
   Half4 v;
   if constexpr (BITS <= 5) {
     constexpr int words = BITS * 8;
-    const int end0 = (first + 1) * BITS + 256 * BITS;  // past the first state's last bit, a period ahead
-    const int ia = (end0 - 16) >> 5;
-    const int shift = 32 * ia + 64 - (end0 + 3 * BITS);  // 2 .. 45
-    const uint64_t merged = (static_cast<uint64_t>(word(ia % words)) << 32) | word((ia + 1) % words);
-    const uint32_t window = static_cast<uint32_t>(merged >> shift);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = Codebook<CB>((window >> ((3 - j) * BITS)) & 0xFFFFu);
+    const int ia = ((first + 1) * BITS + 256 * BITS - 16) >> 5;
+    return DecodeFour<CB, BITS>(first, word(ia % words), word((ia + 1) % words));
   } else {
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = Codebook<CB>(State<BITS>(first + j, word));
   }
   return v;
+}
+
+// The same from the words that a lane has loaded: kHeldWords of a tile from FirstWord on (circular).
+template <int BITS>
+constexpr int kHeldWords = BITS <= 5 ? 2 : 3;
+template <int BITS>
+__device__ __forceinline__ int FirstWord(int first) { return (((first + 1) * BITS + 256 * BITS - 16) >> 5) % (BITS * 8); }
+template <int CB, int BITS>
+__device__ __forceinline__ Half4 DecodeHeld(int first, const uint32_t (&held)[kHeldWords<BITS>]) {
+  if constexpr (BITS <= 5) {
+    return DecodeFour<CB, BITS>(first, held[0], held[1]);
+  } else {
+    constexpr int words = BITS * 8;
+    const int word0 = FirstWord<BITS>(first);
+    return DecodeFour<CB, BITS>(first, [&](int i) {
+      const int d = (i - word0 + words) % words;
+      return d == 0 ? held[0] : d == 1 ? held[1] : held[2];
+    });
+  }
 }
 
 // ---------------------------------------------------------------- reconstruct
@@ -302,8 +329,8 @@ __global__ __launch_bounds__(256) void ReconstructTransposedKernel(const uint32_
   // of a tile's stream, the same in every tile: they are asked for from all sixteen tiles before the first is decoded (a
   // tile after the other, each decode would wait for its own loads), and a workgroup goes through its blocks (every
   // gridDim.x-th, columns fastest) with the next block's words asked for ahead of this block's way out.
-  constexpr int kWords = BITS * 8, kHeld = BITS <= 5 ? 2 : 3;
-  const int word0 = (((p.first + 1) * BITS + 256 * BITS - 16) >> 5) % kWords;
+  constexpr int kWords = BITS * 8, kHeld = kHeldWords<BITS>;
+  const int word0 = FirstWord<BITS>(p.first);
   const int blocks_n = columns / 128;
   const int blocks = blocks_n * (k / 128);
   uint32_t words[16][kHeld];
@@ -327,10 +354,7 @@ __global__ __launch_bounds__(256) void ReconstructTransposedKernel(const uint32_
   for (int u = 0; u < 16; ++u) {
     const int t = wave * 16 + u;
     const int kt = t >> 3, nt = t & 7;
-    const Half4 v = DecodeFour<CB, BITS>(p.first, [&](int i) {
-      const int d = (i - word0 + kWords) % kWords;
-      return d == 0 ? words[u][0] : (kHeld == 2 || d == 1) ? words[u][1] : words[u][kHeld - 1];
-    });
+    const Half4 v = DecodeHeld<CB, BITS>(p.first, words[u]);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const _Float16 value = v[j];
@@ -391,8 +415,8 @@ __global__ __launch_bounds__(256, 3) void ReconstructHadKernel(const uint32_t* _
   const int blocks_k = k / 128;
   const int c0 = (static_cast<int>(blockIdx.x) / blocks_k) * 128, k0 = (static_cast<int>(blockIdx.x) % blocks_k) * 128;
   const Place p = PlaceOf(lane);
-  constexpr int kWords = BITS * 8, kHeld = BITS <= 5 ? 2 : 3;  // a lane's states lie within so many words of a tile
-  const int word0 = (((p.first + 1) * BITS + 256 * BITS - 16) >> 5) % kWords;
+  constexpr int kWords = BITS * 8, kHeld = kHeldWords<BITS>;
+  const int word0 = FirstWord<BITS>(p.first);
   const uint32_t* tiles = trellis + (static_cast<int64_t>(k0 / 16) * (n / 16) + (column + c0) / 16) * kWords;
   uint32_t at[kHeld];
 #pragma unroll
@@ -411,11 +435,7 @@ __global__ __launch_bounds__(256, 3) void ReconstructHadKernel(const uint32_t* _
     Half8 two;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const uint32_t(&held)[kHeld] = words[2 * pair + u];
-      const Half4 v = DecodeFour<CB, BITS>(p.first, [&](int i) {
-        const int d = (i - word0 + kWords) % kWords;
-        return d == 0 ? held[0] : (kHeld == 2 || d == 1) ? held[1] : held[kHeld - 1];
-      });
+      const Half4 v = DecodeHeld<CB, BITS>(p.first, words[2 * pair + u]);
 #pragma unroll
       for (int j = 0; j < 4; ++j) two[4 * u + j] = v[j];
     }
