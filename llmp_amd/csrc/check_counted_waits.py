@@ -13,6 +13,7 @@ compiler takes them for written, copies them, and gives those that nothing reads
 
 Needs hipcc, no GPU. Run by the library's build (__graft_entry__.build) and by tests/test_counted_waits.py;
 `python check_counted_waits.py` runs it alone."""
+import concurrent.futures
 import functools
 import os
 import re
@@ -170,13 +171,15 @@ def check_registers(name, body):
 
 def check():
     """The number of kernels followed; raises AssertionError (or the compiler's error) where a count does not hold."""
+    with concurrent.futures.ThreadPoolExecutor() as pool:
+        decode, exl3 = pool.map(assembly_of, ("decode.hip", "exl3.hip"))
     kernels = 0
-    for name, body in kernels_of(assembly_of("decode.hip"), "DecodeMatrixPanelKernel"):
+    for name, body in kernels_of(decode, "DecodeMatrixPanelKernel"):
         check_panel(name, body)
         kernels += 1
     assert kernels >= 5, f"only {kernels} kernels of the matrix product over laid-out inputs were found"
     products = 0
-    for name, body in kernels_of(assembly_of("exl3.hip"), "WideProductKernel|13ProductKernel"):
+    for name, body in kernels_of(exl3, "WideProductKernel|13ProductKernel"):
         check_registers(name, body)
         products += 1
     assert products >= 48, f"only {products} packed products were found"
