@@ -394,8 +394,8 @@ __global__ __launch_bounds__(256) void ReconstructTransposedKernel(const uint32_
 // come out as a lane's four outputs of one index, the next operand's layout: split into three F16, each the remainder of
 // those before it (nothing of an F32 sum is left out), they are the halves of K of two products with H16 along the
 // outputs; H8 along them is three additions a value. The indices are dealt to the rows so that a lane ends with eight
-// consecutive ones, sixteen bytes of a column. Against F64 a result's error is the one rounding to F16: 2.07e-4 over two
-// to six bits and the three codebooks, in every one of them at most the F32 butterflies'.
+// consecutive ones, sixteen bytes of a column. Against F64 a result's error is the one rounding to F16: 2.07e-4 over one
+// to eight bits and the three codebooks, in every one of them at most the F32 butterflies'.
 // Bound by vector issue (decode 1,800 instructions a block and lane, split 2,000, additions 800, scales and rounding 800),
 // 3.5 blocks a SIMD at 4096 x 14336, and 117 MB written (23 us at a copy's rate): 59 us there, where the transforms as
 // butterflies in F32 by data-parallel moves and LDS, 42 operations a value, took 104. A wave a block with all its sums in

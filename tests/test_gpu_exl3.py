@@ -224,6 +224,28 @@ def test_wide_passes_are_the_sixteen_row_passes_bit_for_bit(device, m, k, n, bit
     assert torch.equal(both[1].view(torch.int32), got.view(torch.int32))
 
 
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6])
+@pytest.mark.parametrize("codebook", [ops.EXL3_3INST, ops.EXL3_MCG, ops.EXL3_MUL1])
+def test_fused_reconstruction_is_one_rounding_from_64_bits(device, bits, codebook):
+    """W = diag(suh) H What H diag(svh) / 128 in 64 bits from the rotated weights (exact in F16): the kernel's error is that of
+    one rounding to F16. What else it may add: both transforms' sums in F32, 14 additions deep, and three products, 17
+    roundings of at most 2^-24 of the values' size each (a transform keeps the 2-norm, scaled), twice where one takes a value
+    past the middle between two F16."""
+    k, n = 384, 256
+    trellis, suh, svh = synth.exl3_weights(k, n, bits, 70 + bits)
+    args = (dev(trellis, device), halves(suh, device), halves(svh, device), k, n, bits, codebook)
+    got = ops.exl3_reconstruct(*args, fused=True).cpu().numpy().astype(np.float64)
+    rotated = ops.exl3_reconstruct(*args).cpu().numpy().astype(np.float64)
+    h = np.array([[(-1.0) ** bin(i & j).count("1") for j in range(128)] for i in range(128)])
+    blocks = np.einsum("ai,pibj,jc->pabc", h, rotated.reshape(k // 128, 128, n // 128, 128), h, optimize=True)
+    want = blocks.reshape(k, n) * np.float64(suh.view(np.float16)).reshape(k, 1) * np.float64(svh.view(np.float16)).reshape(1, n) / 128.0
+    size = np.linalg.norm(want)
+    rounding = np.linalg.norm(want.astype(np.float16).astype(np.float64) - want) / size
+    error = np.linalg.norm(got - want) / size
+    assert 1.5e-4 < rounding < 2.5e-4
+    assert error <= rounding + 2 * 17 * 2.0 ** -24, (error, rounding)
+
+
 @pytest.mark.parametrize("m,k,n,bits,codebook", [(200, 1024, 512, 4, ops.EXL3_3INST), (300, 256, 384, 3, ops.EXL3_MCG),
                                                  (1, 128, 128, 5, ops.EXL3_MUL1), (130, 128, 32768 + 256, 2, ops.EXL3_3INST)])
 @pytest.mark.parametrize("fused", [True, False])
