@@ -433,8 +433,9 @@ int llmp_hip_exl3_hadamard(const void* x, void* y, const void* scale, int rows, 
  * into y (m x n, F16 or F32); a_had is the caller's m x k F16 scratch for the transformed input, which the
  * launches write as they compute it. `scratch` (llmp_hip_exl3_linear_scratch bytes, 8-byte aligned: one pass's,
  * shared by the passes in stream order) takes the place of the reference's lock area: the K slices' partial
- * sums, added in slice order (and, of the wide size, the transformed rows in the product's order). Two launches a pass are queued (three above four rows: the input transform is
- * then a launch of its own); a failure after the first is reported as a fault (negative). */
+ * sums, added in slice order (and, of the wide size, the transformed rows in the product's order). An operand within the
+ * least size is refused; one behind it but within the wide size means passes of sixteen. Two launches a pass are queued
+ * (three above four rows: the input transform is then a launch of its own); a failure after the first is reported as a fault (negative). */
 typedef struct llmp_exl3_linear {
   llmp_exl3_weights weights;
   const void* x;

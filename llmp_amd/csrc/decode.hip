@@ -1044,7 +1044,7 @@ __device__ __forceinline__ uint32_t LdsAddress(const void* p) { return static_ca
 // LDS) and 0.07 us a row tile (eight products at 16 cycles); what does not depend on K is 10 us a round of workgroups
 // (the first loads, 17 MB of sums stored at the end). 4096 -> 14336 at 300 rows: 60 us with the launch before, 113 with
 // the tiles of 256 by 128 below it, which convert the inputs 56 times and wait for a chunk's loads in every chunk; 64
-// rows 38 us against 54, 1,024 rows 208 against 235 (NVFP4).
+// rows 38 us against 53, 1,024 rows 193 against 238 (NVFP4).
 template <int D, int MT>
 __global__ __launch_bounds__(256, 2) void DecodeMatrixPanelKernel(const PanelArgs p) {
   constexpr bool kHalf = D == LLMP_DECODER_F16_DENSE || D == LLMP_DECODER_Q8_0_BLOCKS;
@@ -1309,8 +1309,8 @@ PanelShape PanelTiles(uint64_t outputs, uint64_t rows, uint32_t k) {
 // Whether the laid-out form is the faster one: both forms' microseconds by what was measured. The one launch takes a round of
 // its workgroups for every CU's worth of tiles of 256 by 128 or 256, and of its small tiles, several of which share a CU, a
 // time with their number once there is more than one a CU; this form a round of its own tiles. So a product whose last round
-// of large tiles is full stays with the one launch (NVFP4 4096 -> 8192 at 2,048 rows: 197 us against 243), and where most of
-// that round is idle this form is up to 2.6 times faster (4096 -> 14336 at 200 rows: 134 against 52). Three kinds of
+// of large tiles is full stays with the one launch (NVFP4 4096 -> 8192 at 2,048 rows: 193 us against 239), and where most of
+// that round is idle this form is up to 2.6 times faster (4096 -> 14336 at 200 rows: 135 against 51). Three kinds of
 // encoding differ enough to have costs of their own: 16-bit values, whose loads are what the small tiles wait for; the other
 // nine; and affine, whose loads lie under branches, so that this form waits for each where it is asked for. Over 8,097
 // products (twelve encodings, 1,024 to 14,336 outputs, K from 768, 17 to 4,096 rows) the choice by these costs is 0.3 %

@@ -1,5 +1,5 @@
 // The EXL3 trellis-coded linear (QTIP-style) for gfx950: codebook decode, weight
-// reconstruction, the 128-point Hadamard transforms and the packed product for up to 16 rows.
+// reconstruction, the 128-point Hadamard transforms and the packed products: up to 16 rows a pass, and up to 144.
 //
 // Format (src/kernels/reference/decode_exl3.cc of the reference): the weights are
 // [K / 16][N / 16] tiles of 16 x 16 values at K bits a value; a tile's 256 K bits are a
@@ -15,8 +15,8 @@
 // L = g + 4 (n % 2) + 8 ((n % 8) / 2): the values of column n at rows 2 g, 2 g + 1, 2 g + 8,
 // 2 g + 9, which is column n of the operand with its four k slots in that row order; the other
 // operand (the transformed activations, a row a token) is loaded with the same row order. So a
-// wave decodes a tile with four states a lane and multiplies it by one MFMA, whatever the
-// token count up to 16. A wave takes the eight tiles of one 128-column block (1 KB, contiguous)
+// wave decodes a tile with four states a lane, and the tiles of two steps of K are one 16 x 16 x 32
+// MFMA, whatever the token count up to 16. A wave takes the eight tiles of one 128-column block (1 KB, contiguous)
 // per 16 rows of K, fetched with global_load_lds_dwordx4 into a small ring, and a slice of K;
 // the slices' partial sums are added in slice order by the output transform (no atomics).
 //
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(256) void ReconstructTransposedKernel(const uint32_
 // consecutive ones, sixteen bytes of a column. Against F64 a result's error is the one rounding to F16: 2.07e-4 over one
 // to eight bits and the three codebooks, in every one of them at most the F32 butterflies'.
 // Bound by vector issue (decode 1,800 instructions a block and lane, split 2,000, additions 800, scales and rounding 800),
-// 3.5 blocks a SIMD at 4096 x 14336, and 117 MB written (23 us at a copy's rate): 59 us there, where the transforms as
+// 3.5 blocks a SIMD at 4096 x 14336, and 117 MB written (23 us at a copy's rate): 55.6 us there, where the transforms as
 // butterflies in F32 by data-parallel moves and LDS, 42 operations a value, took 104. A wave a block with all its sums in
 // registers (one wave a SIMD) took 74: nothing ran under its waits.
 // kTransposed: w[columns][k], a column's inputs together. Else w[k][columns], the rows turned by way of LDS.
@@ -1341,6 +1341,10 @@ int LaunchLinears(const llmp_exl3_weights* const (&w)[2], int count, const void*
     sides.a_had[i] = fused ? static_cast<uint16_t*>(a_had[i]) : nullptr;
     sides.partial[i] = scratch[i];
   }
+  // Of the counts of row tiles a kernel is built for the fewest that hold the rows; the tiles past the rows are the last
+  // one's products again and cost little beside the decode: 4096 x 14336 at four bits, 17 and 32 rows 25.0 us (two tiles),
+  // 33, 64 and 80 rows 37.0, 39.5 and 42.2 (five), 81, 112 and 144 rows 50.4, 53.8 and 57.7 (nine); in passes of sixteen
+  // the same rows take 44 to 201 us.
   Dispatch(w0.codebook, w0.bits, [&](auto cb, auto bits) {
     constexpr int kCb = decltype(cb)::value, kBits = decltype(bits)::value;
     if (wide) {
