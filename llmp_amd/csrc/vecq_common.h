@@ -234,6 +234,10 @@ void LaunchFlat(int type, const VecQArgs& a, int x_type, int pass, bool deep, hi
 bool MmaTakes(int type, const llmp_vecq_desc& d);
 void LaunchMma(int type, const VecQArgs& a, hipStream_t stream);
 
+// Q4_K rows sorted by expert, rows of up to eight super-blocks, on 32 x 32 matrix instructions (vecq_sorted.hip).
+bool SortedTakes(int type, const llmp_vecq_desc& d);
+void LaunchSorted(const VecQArgs& a, int workgroups, hipStream_t stream);
+
 // The row-a-lane kernel for 2 to 8 tokens of a dense or grouped Q4_K product over Q8_1 activations (vecq_rows.hip).
 constexpr int kRowsTokensMost = 16;  // of the row-a-lane form (the operation's most): eight a launch
 bool RowsTakes(int type, const llmp_vecq_desc& d, int parts = 1);  // parts: the units of a row in a piece (tiles of 64 / parts rows)

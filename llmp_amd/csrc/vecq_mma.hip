@@ -49,6 +49,7 @@
 #include "common.h"
 #include "llmp_hip.h"
 #include "vecq_common.h"
+#include "vecq_sorted_walk.h"
 
 namespace llmp_hip {
 namespace {
@@ -305,7 +306,6 @@ __global__ __launch_bounds__(kMmaGroup, 1) void VecQMma(const VecQArgs a, int ba
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   __shared__ int pairs[kMaxPairs];
   __shared__ int count;
-  __shared__ int scan[kMmaGroup / kWave];
 
   const llmp_vecq_desc& d = a.d;
   const int tid = threadIdx.x;
@@ -511,83 +511,16 @@ __global__ __launch_bounds__(kMmaGroup, 1) void VecQMma(const VecQArgs a, int ba
     for (int p0 = 0; p0 < n; p0 += TG * MT)
       run(Segment{expert, p0, min(TG * MT, n - p0), static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), mine});
   } else {
-    // Sorted rows, shared evenly: expert e brings ceil(rows / (TG MT)) passes, a pass `groups` groups of
-    // tiles, and a group of a pass costs by the pass's live token groups (Cost). The groups of all passes in
-    // expert order lie end to end on a line of cost, and workgroup w takes the groups that start within its
-    // W-th of the line: a few segments of consecutive groups.
-    const int experts = d.used;
-    constexpr int kPass = TG * MT;
-    auto live_of = [](int m) {
-      const int token_groups = (m + MT - 1) / MT;
-      return token_groups <= 1 ? 1 : token_groups <= 2 ? 2 : 4;
-    };
     // A step's instructions: about 12 parts for the weights and 7 a live token group.
-    auto cost_of = [](int live) { return 12 + 7 * min(live, TG); };
-    auto expert_cost = [&](int rows) {
-      if (rows <= 0) return 0;
-      const int passes = (rows + kPass - 1) / kPass;
-      return (passes - 1) * cost_of(TG) + cost_of(live_of(rows - (passes - 1) * kPass));
+    auto cost_of = [](int m) {
+      const int token_groups = (m + MT - 1) / MT;
+      const int live = token_groups <= 1 ? 1 : token_groups <= 2 ? 2 : 4;
+      return 12 + 7 * min(live, TG);
     };
-    int* walk = pairs;  // [0] all experts' cost, [1] the first expert with groups of this workgroup, [2] the cost
-                        // before it, [3] the last such expert
-    if (tid == 0) walk[0] = 0, walk[1] = experts, walk[2] = 0, walk[3] = -1;
-    __syncthreads();
-    for (int base = 0; base < experts; base += kMmaGroup) {
-      const int e = base + tid;
-      int cost = e < experts ? expert_cost(a.offsets[e + 1] - a.offsets[e]) : 0;
-#pragma unroll
-      for (int delta = kWave / 2; delta >= 1; delta /= 2) cost += ShflXor(cost, delta);
-      if (lane == 0 && cost != 0) atomicAdd(&walk[0], cost);
-    }
-    __syncthreads();
-    const int64_t line = static_cast<int64_t>(walk[0]) * groups;
-    const int64_t from = line * blockIdx.x / gridDim.x, to = line * (blockIdx.x + 1) / gridDim.x;
-    int carried = 0;  // cost of the experts before this round of kMmaGroup
-    for (int base = 0; base < experts; base += kMmaGroup) {
-      const int e = base + tid;
-      const int cost = e < experts ? expert_cost(a.offsets[e + 1] - a.offsets[e]) : 0;
-      int inclusive = cost;  // over the wave, then over the workgroup
-#pragma unroll
-      for (int delta = 1; delta < kWave; delta *= 2) {
-        const int other = __shfl_up(inclusive, delta, kWave);
-        if (lane >= delta) inclusive += other;
-      }
-      __syncthreads();  // the last round's readers of scan
-      if (lane == kWave - 1) scan[wave] = inclusive;
-      __syncthreads();
-      int before = carried;
-      for (int w = 0; w < kMmaGroup / kWave; ++w) {
-        if (w < wave) before += scan[w];
-        carried += scan[w];
-      }
-      const int exclusive = before + inclusive - cost;
-      const bool mine = cost != 0 && max(from, static_cast<int64_t>(exclusive) * groups) <
-                                         min(to, static_cast<int64_t>(exclusive + cost) * groups);
-      if (mine) {
-        atomicMin(&walk[1], e);
-        atomicMax(&walk[3], e);
-      }
-      __syncthreads();
-      if (mine && walk[1] == e) walk[2] = exclusive;
-    }
-    __syncthreads();
-    const int e_first = walk[1], e_last = walk[3];
-    int before = walk[2];
-    __syncthreads();  // pairs is free again
-    for (int e = e_first; e <= e_last; ++e) {
-      sorted_first = a.offsets[e];
-      const int rows = a.offsets[e + 1] - sorted_first;
-      for (int p0 = 0; p0 < rows; p0 += kPass) {
-        const int m = min(kPass, rows - p0);
-        const int cost = cost_of(live_of(m));
-        // The pass's groups start at start, start + cost, ...: those within [from, to).
-        const int64_t start = static_cast<int64_t>(before) * groups;
-        const int g_first = from <= start ? 0 : static_cast<int>((from - start + cost - 1) / cost);
-        const int g_end = to <= start ? 0 : static_cast<int>(min<int64_t>((to - start + cost - 1) / cost, groups));
-        if (g_first < g_end) run(Segment{e, p0, m, g_first, 1, g_end - g_first});
-        before += cost;
-      }
-    }
+    WalkSortedRows(a.offsets, d.used, groups, TG * MT, [](int) { return 0; }, cost_of, [&](const SortedSegment& seg) {
+      sorted_first = seg.rows_first;
+      run(Segment{seg.expert, seg.first, seg.m, seg.group_first, 1, seg.group_count});
+    });
   }
 }
 
@@ -996,6 +929,9 @@ void LaunchMma(int type, const VecQArgs& a, hipStream_t stream) {
     const int cus = llmp_hip_compute_units();
     g_mma_compute_units = cus > 0 ? cus : 256;
   }
+  // Sorted Q4_K rows of up to eight super-blocks: the 32 x 32 form, which was the faster at every count of rows an expert
+  // from 2 to 128 (2048 -> 2 x 768, 128 experts: 66 -> 59, 91 -> 68, 125 -> 95 us at 2, 16 and 32 rows).
+  if (a.offsets != nullptr && SortedTakes(type, d)) return LaunchSorted(a, g_mma_compute_units, stream);
   const int slots = a.offsets != nullptr ? d.used : d.ids != nullptr ? d.used * d.tokens : d.used;
   const int tiles = (d.nrows + 15) / 16;
   const int tiles_group = q8 ? kQ8Tiles : nsb <= kWholeRow ? kMmaWaves : kTilesGroup;

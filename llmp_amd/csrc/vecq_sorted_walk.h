@@ -1,0 +1,80 @@
+// How the workgroups of a product over rows sorted by expert share its work (vecq_mma.hip, vecq_sorted.hip).
+#ifndef LLMP_AMD_CSRC_VECQ_SORTED_WALK_H_
+#define LLMP_AMD_CSRC_VECQ_SORTED_WALK_H_
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "common.h"
+
+namespace llmp_hip {
+
+// A value that every lane of the wave holds, as one the compiler knows to be such.
+__device__ __forceinline__ int64_t Uniform(int64_t v) {
+  const uint32_t low = __builtin_amdgcn_readfirstlane(static_cast<int>(v));
+  const uint32_t high = __builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32));
+  return static_cast<int64_t>((static_cast<uint64_t>(high) << 32) | low);
+}
+
+// Consecutive groups of row tiles of one expert against up to a pass's rows of its tokens: the sorted rows
+// rows_first + first .. rows_first + first + m - 1, the groups group_first .. group_first + group_count - 1.
+struct SortedSegment {
+  int expert, rows_first, first, m, group_first, group_count;
+};
+
+// Expert e brings ceil(rows / pass) passes; a pass costs `fixed_of(its rows)` (its tokens' staging) and then, each of its
+// `groups` groups of tiles, `cost_of(its rows)`. The passes in expert order lie end to end on a line of cost, and workgroup
+// w takes the groups that start within its w-th of the line: a few segments of consecutive groups, `run` called on each
+// by every thread. Every wave works its workgroup's part out for itself, a lane a run of consecutive experts: no
+// barriers, and no trip to memory but the offsets'.
+template <typename FixedOf, typename CostOf, typename Run>
+__device__ __forceinline__ void WalkSortedRows(const int32_t* __restrict__ offsets, int experts, int groups, int pass,
+                                               FixedOf fixed_of, CostOf cost_of, Run run) {
+  const int lane = threadIdx.x & (kWave - 1);
+  auto pass_cost = [&](int rows) { return static_cast<int64_t>(fixed_of(rows)) + static_cast<int64_t>(groups) * cost_of(rows); };
+  auto expert_cost = [&](int rows) -> int64_t {
+    if (rows <= 0) return 0;
+    const int passes = (rows + pass - 1) / pass;
+    return (passes - 1) * pass_cost(pass) + pass_cost(rows - (passes - 1) * pass);
+  };
+  const int per = (experts + kWave - 1) / kWave;
+  const int mine = min(lane * per, experts), after = min(mine + per, experts);
+  int64_t cost = 0;
+  for (int e = mine; e < after; ++e) cost += expert_cost(offsets[e + 1] - offsets[e]);
+  int64_t inclusive = cost;
+#pragma unroll
+  for (int delta = 1; delta < kWave; delta <<= 1) {
+    const int64_t other = __shfl_up(inclusive, delta, kWave);
+    if (lane >= delta) inclusive += other;
+  }
+  const int64_t line = Uniform(__shfl(inclusive, kWave - 1, kWave));
+  const int64_t from = line * blockIdx.x / gridDim.x, to = line * (blockIdx.x + 1) / gridDim.x;
+  // The lane whose experts hold `from`, and of them the expert: the first whose cost ends past it.
+  const unsigned long long past = __ballot(inclusive > from);
+  if (past == 0) return;  // an empty line
+  const int first_lane = __ffsll(past) - 1;
+  int64_t before = Uniform(__shfl(inclusive - cost, first_lane, kWave));
+  for (int e = first_lane * per; e < experts && before < to; ++e) {
+    const int rows_first = __builtin_amdgcn_readfirstlane(offsets[e]);
+    const int rows = __builtin_amdgcn_readfirstlane(offsets[e + 1]) - rows_first;
+    const int64_t all = expert_cost(rows);
+    if (before + all <= from) {
+      before += all;
+      continue;
+    }
+    for (int p0 = 0; p0 < rows; p0 += pass) {
+      const int m = min(pass, rows - p0);
+      const int each = cost_of(m);
+      // The pass's groups start at start, start + each, ...: those within [from, to).
+      const int64_t start = before + fixed_of(m);
+      const int g_first = from <= start ? 0 : static_cast<int>(min<int64_t>((from - start + each - 1) / each, groups));
+      const int g_end = to <= start ? 0 : static_cast<int>(min<int64_t>((to - start + each - 1) / each, groups));
+      if (g_first < g_end) run(SortedSegment{e, rows_first, p0, m, g_first, g_end - g_first});
+      before += pass_cost(m);
+    }
+  }
+}
+
+}  // namespace llmp_hip
+
+#endif  // LLMP_AMD_CSRC_VECQ_SORTED_WALK_H_

@@ -253,6 +253,37 @@ def test_routed_and_sorted_long_rows_match_oracle(device, t, k):
     assert np.array_equal(sorted_out.view(np.uint32), got.reshape(tokens * used, n)[order].view(np.uint32))
 
 
+@pytest.mark.parametrize("k,n,glu", [(256, 40, False), (512, 24, True), (768, 513, False), (1024, 88, True), (1280, 34, True),
+                                     (2048, 264, True), (2048, 31, False), (2304, 40, False)])
+def test_sorted_q4k_rows_at_the_edges_of_passes_and_tiles(device, k, n, glu):
+    """Experts of no rows, of one, and of one below, at and above a pass of 32 and of 64, tiles that end past the matrix, rows
+    of one to nine super-blocks (from nine on the 16 x 16 form): against the oracle, within 1e-5 of the RMS (sums of up to 72
+    F32 terms that cancel), and a row's values bit for bit whatever rows stand beside it."""
+    counts = np.array([0, 1, 31, 32, 33, 64, 65, 100, 0, 7], dtype=np.int32)
+    experts, rows = len(counts), int(counts.sum())
+    blocks = k // 256
+    w = make_weights(Q4_K, experts * 2 * n, k, 91).reshape(experts, -1)
+    up = w.reshape(-1)[n * blocks * 144:]
+    q8 = oracle.q8_1_quantize(synth.activations(rows, k, 92)).reshape(rows, -1)
+    ids = np.repeat(np.arange(experts, dtype=np.int32), counts).reshape(-1, 1)
+    kind = ops.GLU_SWIGLU if glu else ops.GLU_NONE
+    # (The oracle's pairs name experts of one table: w, whose expert is its n gate rows and then its n up rows.)
+    want = oracle.vecq(Q4_K, up, q8, k, n, gate=w if glu else None, ids=ids, tokens=rows, used=1, stride_expert=2 * n * blocks,
+                       glu=kind, experts=experts, threads=oracle.max_threads()).reshape(rows, n)
+    wd = dev(w, device)
+
+    def product(picked, sizes):
+        offsets = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+        return ops.vecq_sorted(Q4_K, wd.view(-1)[n * blocks * 144:], dev(q8[picked], device), dev(offsets, device), k, n, experts,
+                               gate=wd if glu else None, stride_expert=2 * n * blocks, glu=kind).cpu().numpy()
+
+    got = product(np.arange(rows), counts)
+    ok, worst = rel_close(got, want, 1e-5, floor=1.0)
+    assert ok, worst
+    last = np.cumsum(counts)[counts > 0] - 1
+    assert np.array_equal(product(last, (counts > 0).astype(np.int32)).view(np.uint32), got[last].view(np.uint32))
+
+
 def same_sums(t, a, b):
     """Q8_0: the matrix-core kernel repeats the flat kernel's float operations and its summation tree, bit for bit.
     Q4_K: its sub-block sums are the same exact integers, scaled and added in another order (one fma a sub-block
