@@ -151,60 +151,75 @@ __global__ void RouteAssign(const int32_t* __restrict__ ids, int ids_stride, Rou
   }
 }
 
-// The whole grouping by one workgroup, for problems whose ids and per-run counters fit LDS
-// (up to 8192 slots and runs x experts up to 8192): the slots are cut into runs of 64 in slot
-// order; a run's ids are counted per expert with LDS integer atomics (a count does not depend
-// on their order), a thread an expert turns the runs' counts into bases, one thread the
-// experts' totals into offsets, and a thread a slot then takes its expert's first row, plus
-// its run's base, plus the equal ids before it in its run (at most 63 compares).
-// LDS: the ids, padded to fours; runs x experts counters; experts + 1 offsets.
-constexpr int kRouteOneSlots = 8192;
-constexpr int kRouteOneCounters = 8192;
-constexpr int kRouteOneThreads = 1024;
+// The whole grouping in one launch, for problems of up to 8192 slots whose counters fit LDS. A workgroup places 512
+// consecutive slots, a thread a slot, and counts all slots' ids itself, 16 KB of them at 4096 slots: in LDS, with integer
+// atomics (a count does not depend on their order), those of its own slots, those before them and those after apart. Its
+// own are counted a wave at a time: the lanes that hold the same id are found by a ballot a bit of the id, which gives
+// each its rank, and the first of them notes how many. A slot's row is then its expert's first row, plus the expert's
+// slots before the workgroup's, plus those of the workgroup's earlier waves, plus its rank. What bounds it is latency:
+// the launch, one trip for the ids, three barriers. One workgroup doing it all (a prefix over 64 runs of 128 counters and
+// up to 63 compares a slot end to end on one compute unit) took 13.4 us at 4096 slots of 128 experts.
+// LDS, ints: the waves' counts [wave][expert], zeros before the slots' [expert], counts before and after [2][expert],
+// offsets [expert + 1].
+constexpr int kRouteSpread = 512;  // slots, and threads, a workgroup
+constexpr int kRouteSpreadSlots = 8192;
+constexpr int kRouteSpreadLds = 152 * 1024;
 
-__global__ __launch_bounds__(kRouteOneThreads) void RouteOne(const int32_t* __restrict__ ids, int ids_stride, Route r) {
-  extern __shared__ __attribute__((aligned(16))) int32_t staged[];
+__host__ __device__ inline int64_t RouteSpreadInts(int64_t slots, int experts) {
+  const int64_t waves = ((slots < kRouteSpread ? slots : kRouteSpread) + kWave - 1) / kWave;
+  return (waves + 3) * experts + 1;
+}
+
+__global__ __launch_bounds__(kRouteSpread) void RouteSpread(const int32_t* __restrict__ ids, int ids_stride, Route r) {
+  extern __shared__ int32_t counts[];
   const int slots = r.tokens * r.used;
-  const int runs = (slots + 63) / 64;
-  int32_t* counters = staged + ((slots + 3) & ~3);  // [run][expert]
-  int32_t* offsets = counters + runs * r.experts;    // [expert + 1]
-  const int tid = threadIdx.x;
-  for (int i = tid; i < slots; i += kRouteOneThreads) staged[i] = ids[static_cast<int64_t>(i / r.used) * ids_stride + i % r.used];
-  if (tid < 4 && slots + tid < ((slots + 3) & ~3)) staged[slots + tid] = INT32_MIN;
-  for (int i = tid; i < runs * r.experts; i += kRouteOneThreads) counters[i] = 0;
+  const int waves = (min(slots, kRouteSpread) + kWave - 1) / kWave;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+  int32_t* before = counts + waves * r.experts;
+  int32_t* after = before + r.experts;
+  int32_t* offsets = after + r.experts;  // [expert + 1]
+  const int first = blockIdx.x * kRouteSpread;
+  const int mine = first + tid;
+  auto id_at = [&](int i) { return ids[ids_stride == r.used ? i : static_cast<int64_t>(i / r.used) * ids_stride + i % r.used]; };
+  const int e = mine < slots ? id_at(mine) : -1;
+  const bool placed = e >= 0 && e < r.experts;
+  for (int i = tid; i < (waves + 2) * r.experts; i += kRouteSpread) counts[i] = 0;
   __syncthreads();
-  for (int i = tid; i < slots; i += kRouteOneThreads) {
-    const int e = staged[i];
-    if (e >= 0 && e < r.experts) atomicAdd(&counters[(i / 64) * r.experts + e], 1);
-  }
-  __syncthreads();
-  for (int e = tid; e < r.experts; e += kRouteOneThreads) {
-    int running = 0;
-    // Sixteen runs' counts read together (a read after a write to the same array would
-    // otherwise wait for it), then their bases written.
-    for (int run0 = 0; run0 < runs; run0 += 16) {
-      int v[16];
+  // The other workgroups' slots, eight ids in flight a thread.
+  for (int i0 = tid; i0 < slots; i0 += 8 * kRouteSpread) {
+    int id[8];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) v[u] = counters[min(run0 + u, runs - 1) * r.experts + e];
+    for (int u = 0; u < 8; ++u) id[u] = id_at(min(i0 + u * kRouteSpread, slots - 1));
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        if (run0 + u < runs) {
-          counters[(run0 + u) * r.experts + e] = running;
-          running += v[u];
-        }
-      }
+    for (int u = 0; u < 8; ++u) {
+      const int i = i0 + u * kRouteSpread;
+      if (i < slots && (i < first || i >= first + kRouteSpread) && id[u] >= 0 && id[u] < r.experts)
+        atomicAdd(i < first ? &before[id[u]] : &after[id[u]], 1);
     }
-    offsets[e + 1] = running;  // the expert's total, for now
   }
+  unsigned long long same = __ballot(placed);
+  for (int bit = 0; (r.experts - 1) >> bit != 0; ++bit) {
+    const bool set = (e >> bit) & 1;
+    const unsigned long long with = __ballot(set);
+    same &= set ? with : ~with;
+  }
+  const int rank = __popcll(same & ((1ull << lane) - 1ull));
+  if (placed && rank == 0) counts[wave * r.experts + e] = __popcll(same);
   __syncthreads();
-  // The experts' totals into offsets: each lane of the first wave a block of consecutive
-  // experts, the blocks' sums scanned across the wave.
-  if (tid < kWave) {
+  // The experts' totals into offsets: each lane of the first wave a run of consecutive experts, the runs' sums scanned
+  // across the wave.
+  if (wave == 0) {
     const int per = (r.experts + kWave - 1) / kWave;
-    const int e0 = min(tid * per, r.experts), e1 = min(e0 + per, r.experts);
+    const int e0 = min(lane * per, r.experts), e1 = min(e0 + per, r.experts);
+    auto total_of = [&](int at) {
+      int total = before[at] + after[at];
+      for (int w = 0; w < waves; ++w) total += counts[w * r.experts + at];
+      return total;
+    };
     int rows = 0, scale_rows = 0;
-    for (int e = e0; e < e1; ++e) {
-      const int total = offsets[e + 1];
+    for (int at = e0; at < e1; ++at) {
+      const int total = total_of(at);
+      offsets[at + 1] = total;  // for now
       rows += total;
       scale_rows += (total + kScaleRows - 1) / kScaleRows * kScaleRows;
     }
@@ -213,38 +228,33 @@ __global__ __launch_bounds__(kRouteOneThreads) void RouteOne(const int32_t* __re
     for (int step = 1; step < kWave; step <<= 1) {
       const int a = __shfl_up(rows_before, step, kWave);
       const int b = __shfl_up(scale_before, step, kWave);
-      if (tid >= step) rows_before += a, scale_before += b;
+      if (lane >= step) rows_before += a, scale_before += b;
     }
     int offset = rows_before - rows, scale_row = scale_before - scale_rows;
-    if (tid == 0) {
+    const bool writes = blockIdx.x == 0;
+    if (lane == 0) {
       offsets[0] = 0;
-      r.offsets[0] = 0;
-      r.scale_rows[0] = 0;
+      if (writes) r.offsets[0] = 0, r.scale_rows[0] = 0;
     }
-    for (int e = e0; e < e1; ++e) {
-      const int total = offsets[e + 1];
+    for (int at = e0; at < e1; ++at) {
+      const int total = offsets[at + 1];
       offset += total;
       scale_row += (total + kScaleRows - 1) / kScaleRows * kScaleRows;
-      offsets[e + 1] = offset;
-      r.offsets[e + 1] = offset;
-      r.scale_rows[e + 1] = scale_row;
+      offsets[at + 1] = offset;
+      if (writes) r.offsets[at + 1] = offset, r.scale_rows[at + 1] = scale_row;
     }
   }
   __syncthreads();
-  for (int i = tid; i < slots; i += kRouteOneThreads) {
-    const int e = staged[i];
-    if (e < 0 || e >= r.experts) {  // ids outside the experts have no row
-      r.position[i] = -1;
-      continue;
-    }
-    const int run0 = i & ~63;
-    int before = CountEqual(staged + run0, (i - run0) & ~3, e);
-    for (int j = i & ~3; j < i; ++j) before += staged[j] == e;
-    const int row = offsets[e] + counters[(i / 64) * r.experts + e] + before;
-    r.position[i] = row;
-    r.token[row] = i / r.used;
-    r.expert[row] = e;
+  if (mine >= slots) return;
+  if (!placed) {  // ids outside the experts have no row
+    r.position[mine] = -1;
+    return;
   }
+  int row = offsets[e] + before[e] + rank;
+  for (int w = 0; w < wave; ++w) row += counts[w * r.experts + e];
+  r.position[mine] = row;
+  r.token[row] = mine / r.used;
+  r.expert[row] = e;
 }
 
 // ------------------------------------------------------- gathering quantizer
@@ -370,13 +380,14 @@ extern "C" int llmp_hip_moe_route(const int32_t* ids, int ids_stride, int expert
   const Route r = RouteOf(route, experts, used, tokens);
   const auto s = static_cast<hipStream_t>(stream);
   const int64_t slots = static_cast<int64_t>(used) * tokens;
-  const int64_t runs = (slots + 63) / 64;
-  if (slots <= kRouteOneSlots && runs * experts <= kRouteOneCounters) {
-    const size_t bytes = static_cast<size_t>(((slots + 3) & ~int64_t{3}) + runs * experts + experts + 1) * sizeof(int32_t);
+  // One launch where a workgroup's counters fit LDS, three where they don't or where every workgroup counting all slots
+  // would no longer be little beside the launches.
+  const int64_t bytes = RouteSpreadInts(slots, experts) * static_cast<int64_t>(sizeof(int32_t));
+  if (slots <= kRouteSpreadSlots && bytes <= kRouteSpreadLds) {
     static bool sized = false;  // more than 64 KB of dynamic LDS must be asked for once
-    if (!AllowLds(reinterpret_cast<const void*>(&RouteOne), (kRouteOneSlots + kRouteOneCounters + kRouteOneCounters + 4) * 4, &sized))
-      return LaunchStatus("moe.route");
-    hipLaunchKernelGGL(RouteOne, dim3(1), dim3(kRouteOneThreads), bytes, s, ids, ids_stride, r);
+    if (!AllowLds(reinterpret_cast<const void*>(&RouteSpread), kRouteSpreadLds, &sized)) return LaunchStatus("moe.route");
+    hipLaunchKernelGGL(RouteSpread, dim3(static_cast<unsigned>((slots + kRouteSpread - 1) / kRouteSpread)), dim3(kRouteSpread),
+                       static_cast<size_t>(bytes), s, ids, ids_stride, r);
     return LaunchStatus("moe.route");
   }
   const int threads = experts < 256 ? (experts + 63) / 64 * 64 : 256;

@@ -74,6 +74,27 @@ def test_route_groups_pairs_by_expert_in_token_order(device, tokens, experts, us
     assert np.array_equal(route.scale_rows.cpu().numpy(), padded)
 
 
+@pytest.mark.parametrize("tokens,experts,used", [(1, 1, 1), (513, 1, 1), (64, 8192, 1), (512, 2, 1), (8, 1000, 64), (171, 129, 6),
+                                                 (1025, 128, 8), (1024, 3500, 8), (1024, 4000, 8)])
+def test_route_at_the_edges_of_the_one_launch(device, tokens, experts, used):
+    """Slots at, one past and below a workgroup's 512, ids of one bit and of 13, counters that fit LDS and not, ids outside the
+    experts among them, rows of ids further apart than they are long: against a stable sort."""
+    g = synth.rng(17 + tokens)
+    table = g.integers(-1, experts + 1, size=(tokens, used + 3), dtype=np.int32)
+    ids = table[:, :used].reshape(-1)
+    route = ops.moe_route(dev(table, device)[:, :used], experts)
+    slots = np.flatnonzero((ids >= 0) & (ids < experts))
+    order = slots[np.argsort(ids[slots], kind="stable")]
+    position = np.full(tokens * used, -1)
+    position[order] = np.arange(len(order))
+    counts = np.bincount(ids[slots], minlength=experts)
+    assert np.array_equal(route.offsets.cpu().numpy(), np.concatenate([[0], np.cumsum(counts)]))
+    assert np.array_equal(route.scale_rows.cpu().numpy(), np.concatenate([[0], np.cumsum((counts + 127) // 128 * 128)]))
+    assert np.array_equal(route.position.cpu().numpy(), position)
+    assert np.array_equal(route.token.cpu().numpy()[:len(order)], order // used)
+    assert np.array_equal(route.expert.cpu().numpy()[:len(order)], ids[order])
+
+
 def test_route_marks_ids_outside_the_experts(device):
     ids = np.array([[0, 5], [9, 1], [-1, 0]], dtype=np.int32)
     route = ops.moe_route(dev(ids, device), 4)
