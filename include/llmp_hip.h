@@ -148,6 +148,12 @@ int llmp_hip_vecq_block_sums(int type, const llmp_vecq_desc* d, int variant, int
  * form takes (the rows form has no sorted variant). */
 int llmp_hip_vecq_sorted(int type, const llmp_vecq_desc* d, const int32_t* offsets, int experts,
                          int variant, void* stream);
+/* The same where the activations lie once a token, not gathered into sorted order: sorted row r's are
+ * row rows[r] of d->y (the route buffer's token), its output row r of dst. The matrix-core forms, where
+ * llmp_hip_vecq_sorted_takes_rows says 1 for the product; the results are the gathered rows' bit for bit. */
+int llmp_hip_vecq_sorted_takes_rows(int type, const llmp_vecq_desc* d);
+int llmp_hip_vecq_sorted_rows(int type, const llmp_vecq_desc* d, const int32_t* offsets, const int32_t* rows,
+                              int experts, int variant, void* stream);
 
 /* ------------------------------------------------------------------ routed experts
  * llmp.moe.router (src/kernels/ggml/llmp_fused.cu:1307-1407; the definition is kRoute with

@@ -656,7 +656,7 @@ int CheckDesc(int type, const llmp_vecq_desc* d, bool sorted = false) {
 }
 
 int Launch(int type, const llmp_vecq_desc* d, const llmp_vecq_source* x, int variant, int32_t* dump, void* stream,
-           const int32_t* offsets = nullptr) {
+           const int32_t* offsets = nullptr, const int32_t* rows = nullptr) {
   if (const int bad = CheckDesc(type, d, offsets != nullptr); bad != 0) return bad;
   int x_type = -1;
   VecQArgs a{};
@@ -674,6 +674,7 @@ int Launch(int type, const llmp_vecq_desc* d, const llmp_vecq_source* x, int var
   a.kp = PaddedK(d->ncols_x);
   a.dump = dump;
   a.offsets = offsets;
+  a.rows = rows;
   if (variant < 0) variant = DefaultVariant(type, *d, a.kp, x != nullptr);
   if (variant >= kVariantCount) return Refuse(1, "vecq: no variant %d", variant);
   const Variant& v = kVariants[variant];
@@ -785,8 +786,10 @@ extern "C" int llmp_hip_vecq_block_sums(int type, const llmp_vecq_desc* d, int v
   return Launch(type, d, nullptr, variant, sums, stream);
 }
 
-extern "C" int llmp_hip_vecq_sorted(int type, const llmp_vecq_desc* d, const int32_t* offsets, int experts, int variant,
-                                    void* stream) {
+namespace {
+
+int LaunchSortedRows(int type, const llmp_vecq_desc* d, const int32_t* offsets, const int32_t* rows, int experts, int variant,
+                     void* stream) {
   BeginLaunches();
   if (offsets == nullptr || d == nullptr) return Refuse(1, "vecq: null offsets");
   if (experts < 1 || experts > 65535) return Refuse(1, "vecq: 1 to 65535 experts");
@@ -801,7 +804,25 @@ extern "C" int llmp_hip_vecq_sorted(int type, const llmp_vecq_desc* d, const int
     return Refuse(1, "vecq: sorted rows take weights the flat or the matrix-core form takes");
   // An expert's rows are many tokens of one matrix: the matrix cores where they apply.
   if (variant < 0) variant = MmaTakes(type, *d) ? kMmaVariant : kFlatFirst + 1;
-  return Launch(type, &sorted, nullptr, variant, nullptr, stream, offsets);
+  if (rows != nullptr && variant != kMmaVariant) return Refuse(1, "vecq: sorted rows by index take the matrix-core form");
+  return Launch(type, &sorted, nullptr, variant, nullptr, stream, offsets, rows);
+}
+
+}  // namespace
+
+extern "C" int llmp_hip_vecq_sorted(int type, const llmp_vecq_desc* d, const int32_t* offsets, int experts, int variant,
+                                    void* stream) {
+  return LaunchSortedRows(type, d, offsets, nullptr, experts, variant, stream);
+}
+
+extern "C" int llmp_hip_vecq_sorted_takes_rows(int type, const llmp_vecq_desc* d) {
+  return d != nullptr && d->ncols_x > 0 && MmaTakes(type, *d) ? 1 : 0;
+}
+
+extern "C" int llmp_hip_vecq_sorted_rows(int type, const llmp_vecq_desc* d, const int32_t* offsets, const int32_t* rows,
+                                         int experts, int variant, void* stream) {
+  if (rows == nullptr) return Refuse(1, "vecq: null rows");
+  return LaunchSortedRows(type, d, offsets, rows, experts, variant, stream);
 }
 
 extern "C" int llmp_hip_vecq_variants(void) { return kVariantCount; }

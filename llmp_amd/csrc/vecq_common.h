@@ -111,6 +111,9 @@ struct VecQArgs {
   // Sorted rows: expert e computes rows offsets[e] .. offsets[e + 1] of the activations into
   // the same rows of the output (d.ids unused), or null.
   const int32_t* offsets;
+  // Sorted rows whose activations lie once a token: sorted row r's are row rows[r] of d.y. Null: row r. (The matrix-core
+  // forms.)
+  const int32_t* rows;
   // The row-a-lane form over weights the importer relaid out (llmp_hip_relayout_q4_k_tiles64): within every 64
   // rows the blocks lie super-block after super-block, a super-block's 64 rows together.
   int tiled = 0;

@@ -355,7 +355,9 @@ __global__ __launch_bounds__(kMmaGroup, 1) void VecQMma(const VecQArgs a, int ba
     auto row_of = [&](int j) {
       const int pr = pair_at(p0 + min(j, m - 1));  // tokens past m repeat the last: computed and dropped
       return static_cast<const uint8_t*>(d.y) +
-             (static_cast<int64_t>(pr >> 8) * d.y_token + static_cast<int64_t>(pr & 0xFF) * d.y_slot) * kQ8Block;
+             (static_cast<int64_t>(a.rows != nullptr ? a.rows[pr >> 8] : pr >> 8) * d.y_token +
+              static_cast<int64_t>(pr & 0xFF) * d.y_slot) *
+                 kQ8Block;
     };
     uint32_t held[kStageAhead][9];
 #pragma unroll
@@ -737,7 +739,9 @@ __global__ __launch_bounds__(kMmaGroup, 1) void VecQMmaQ8(const VecQArgs a) {
     auto row_of = [&](int j) {
       const int pr = pair_at(p0 + j);
       return static_cast<const uint8_t*>(d.y) +
-             (static_cast<int64_t>(pr >> 8) * d.y_token + static_cast<int64_t>(pr & 0xFF) * d.y_slot) * kQ8Block;
+             (static_cast<int64_t>(a.rows != nullptr ? a.rows[pr >> 8] : pr >> 8) * d.y_token +
+              static_cast<int64_t>(pr & 0xFF) * d.y_slot) *
+                 kQ8Block;
     };
     StageTokensQ8(row_of, m, blocks, codes, scales);
     __syncthreads();

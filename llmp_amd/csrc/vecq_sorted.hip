@@ -292,8 +292,9 @@ __global__ __launch_bounds__(Staged<TG>::kGroup, 1) void VecQSorted(const VecQAr
     };
     auto fetch_block = [&](int t, int b, uint32_t(&w)[9]) {
       // Tokens past m repeat the last: computed and dropped.
-      const uint32_t* src = reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(d.y) +
-                                                              (static_cast<int64_t>(first_row + min(t, seg.m - 1)) * d.y_token + b) * kQ8Block);
+      const int r = first_row + min(t, seg.m - 1);
+      const int64_t y_row = a.rows != nullptr ? a.rows[r] : r;
+      const uint32_t* src = reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(d.y) + (y_row * d.y_token + b) * kQ8Block);
 #pragma unroll
       for (int i = 0; i < 9; ++i) w[i] = src[i];
     };

@@ -128,17 +128,28 @@ def vecq_variants():
 
 
 def vecq_sorted(t, w, q8, offsets, k, nrows, experts, *, gate=None, stride_row=None, stride_expert=0,
-                glu=GLU_NONE, limit=0.0, variant=-1, out=None):
-    """llmp.vecq over rows sorted by expert: q8 [rows, blocks*36] -> float32 [rows, nrows]."""
+                glu=GLU_NONE, limit=0.0, variant=-1, out=None, rows=None):
+    """llmp.vecq over rows sorted by expert: q8 [rows, blocks*36] -> float32 [rows, nrows]. `rows` (int32): sorted row r's
+    activations are q8's row rows[r] (where sorted_takes_rows says so)."""
     lib = _lib.load()
-    rows = q8.shape[0]
+    count = q8.shape[0] if rows is None else rows.numel()
     if out is None:
-        out = torch.empty((rows, nrows), dtype=torch.float32, device=w.device)
+        out = torch.empty((count, nrows), dtype=torch.float32, device=w.device)
     d = _desc(t, w, k, nrows, gate=gate, q8=q8, ids=None, tokens=1, used=1, stride_row=stride_row,
               stride_expert=stride_expert, y_token=None, y_slot=0, glu=glu, limit=limit, out=out)
     d.dst_token = nrows
-    _lib.check(lib.llmp_hip_vecq_sorted(t, C.byref(d), _ptr(offsets), experts, variant, _stream()))
+    if rows is None:
+        _lib.check(lib.llmp_hip_vecq_sorted(t, C.byref(d), _ptr(offsets), experts, variant, _stream()))
+    else:
+        _lib.check(lib.llmp_hip_vecq_sorted_rows(t, C.byref(d), _ptr(offsets), _ptr(rows), experts, variant, _stream()))
     return out
+
+
+def sorted_takes_rows(t, w, k, nrows, *, gate=None, stride_expert=0):
+    """Whether vecq_sorted over these weights takes its activations by index."""
+    d = _desc(t, w, k, nrows, gate=gate, q8=None, ids=None, tokens=1, used=1, stride_row=None, stride_expert=stride_expert,
+              y_token=0, y_slot=0, glu=GLU_NONE, limit=0.0, out=w)
+    return _lib.load().llmp_hip_vecq_sorted_takes_rows(t, C.byref(d)) == 1
 
 
 def set_rows_quant(t, x, ids, destination, row_bytes=None):
@@ -271,8 +282,10 @@ def moe_ffn(t, logits, x, gate_up, down, hidden, ffn, experts, used, glu=GLU_SWI
             keep.update(h=h, hq=hq, y=y)
         return moe_combine(y.view(tokens * used, hidden), weights), ids, weights
     route = moe_route(ids, experts)
-    q8 = quantize_q8_1_rows(x, route.token)
-    h = vecq_sorted(t, up, q8, route.offsets, hidden, ffn, experts, gate=gate, stride_expert=gu_stride, glu=glu)
+    # A token's row is quantized once, not once for each of its experts (512 tokens of top 8, 2048 values: 12.3 us gathered).
+    rows = route.token if sorted_takes_rows(t, up, hidden, ffn, gate=gate, stride_expert=gu_stride) else None
+    q8 = quantize_q8_1_rows(x, route.token if rows is None else None)
+    h = vecq_sorted(t, up, q8, route.offsets, hidden, ffn, experts, gate=gate, stride_expert=gu_stride, glu=glu, rows=rows)
     hq = quantize_q8_1_rows(h)
     y = vecq_sorted(t, down, hq, route.offsets, ffn, hidden, experts, stride_expert=down_stride)
     if keep is not None:

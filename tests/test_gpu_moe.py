@@ -95,6 +95,24 @@ def test_route_at_the_edges_of_the_one_launch(device, tokens, experts, used):
     assert np.array_equal(route.expert.cpu().numpy()[:len(order)], ids[order])
 
 
+@pytest.mark.parametrize("t,k", [(Q4_K, 768), (Q4_K, 2048), (Q4_K, 2304), (ops.TYPE_Q8_0, 640)])
+def test_sorted_rows_by_index_equal_the_gathered_rows(device, t, k):
+    experts, n, tokens, used = 6, 40, 45, 3
+    g = synth.rng(23)
+    ids = np.stack([g.permutation(experts)[:used] for _ in range(tokens)]).astype(np.int32)
+    weights = synth.q4_k_weights if t == Q4_K else synth.q8_0_weights
+    w = dev(weights(experts * n, k, 24).reshape(experts, -1), device)
+    x = dev(synth.activations(tokens, k, 25), device)
+    stride = n * k // ops.BLOCK_ELEMENTS[t]
+    assert ops.sorted_takes_rows(t, w, k, n, stride_expert=stride)
+    route = ops.moe_route(dev(ids, device), experts)
+    gathered = ops.vecq_sorted(t, w, ops.quantize_q8_1_rows(x, route.token), route.offsets, k, n, experts, stride_expert=stride)
+    indexed = ops.vecq_sorted(t, w, ops.quantize_q8_1_rows(x), route.offsets, k, n, experts, stride_expert=stride, rows=route.token)
+    assert np.array_equal(indexed.cpu().numpy().view(np.uint32), gathered.cpu().numpy().view(np.uint32))
+    with pytest.raises(ops.KernelFailure):  # the flat form takes gathered rows alone
+        ops.vecq_sorted(t, w, ops.quantize_q8_1_rows(x), route.offsets, k, n, experts, stride_expert=stride, rows=route.token, variant=7)
+
+
 def test_route_marks_ids_outside_the_experts(device):
     ids = np.array([[0, 5], [9, 1], [-1, 0]], dtype=np.int32)
     route = ops.moe_route(dev(ids, device), 4)
