@@ -613,6 +613,15 @@ int DefaultVariant(int type, const llmp_vecq_desc& d, int kp, bool fused) {
   }
 }
 
+// Whether a super-block of 16 rows a wave (vecq_tile16.hip) is the default: nine to sixteen tokens, the faster everywhere it
+// was measured (fourteen shapes from 1024 -> 512 to 15360 -> 8192: 1.1 to 2.1 times the 16 x 16 form and the two launches of
+// the row-a-lane form). Up to eight the row-a-lane form, whose bits a token keeps from two to eight: at eight this one is
+// the faster for rows of more than 8192 values (9216 -> 2048 10.6 against 17.6 us), at four mostly not (15360 -> 3840 13.4
+// against 11.4).
+bool Tile16Pays(int type, const llmp_vecq_desc& d) {
+  return type == LLMP_TYPE_Q4_K && d.ids == nullptr && d.tokens > 8 && d.tokens <= 16;
+}
+
 int CheckDesc(int type, const llmp_vecq_desc* d, bool sorted = false) {
   if (d == nullptr) return Refuse(1, "vecq: null descriptor");
   const bool legacy = type == LLMP_TYPE_Q4_0 || type == LLMP_TYPE_Q4_1 || type == LLMP_TYPE_Q5_0 || type == LLMP_TYPE_Q5_1 ||
@@ -675,6 +684,8 @@ int Launch(int type, const llmp_vecq_desc* d, const llmp_vecq_source* x, int var
   a.dump = dump;
   a.offsets = offsets;
   a.rows = rows;
+  if (variant < 0 && x == nullptr && dump == nullptr && Tile16Pays(type, *d) && LaunchTile16(a, static_cast<hipStream_t>(stream)))
+    return LaunchStatus("vecq");
   if (variant < 0) variant = DefaultVariant(type, *d, a.kp, x != nullptr);
   if (variant >= kVariantCount) return Refuse(1, "vecq: no variant %d", variant);
   const Variant& v = kVariants[variant];

@@ -241,6 +241,10 @@ void LaunchMma(int type, const VecQArgs& a, hipStream_t stream);
 bool SortedTakes(int type, const llmp_vecq_desc& d);
 void LaunchSorted(const VecQArgs& a, int workgroups, hipStream_t stream);
 
+// Q4_K, 9 to 16 tokens of a dense or grouped product over Q8_1 activations, a super-block of 16 rows a wave
+// (vecq_tile16.hip). False: nothing was queued, the shape is not this form's.
+bool LaunchTile16(const VecQArgs& a, hipStream_t stream);
+
 // The row-a-lane kernel for 2 to 8 tokens of a dense or grouped Q4_K product over Q8_1 activations (vecq_rows.hip).
 constexpr int kRowsTokensMost = 16;  // of the row-a-lane form (the operation's most): eight a launch
 bool RowsTakes(int type, const llmp_vecq_desc& d, int parts = 1);  // parts: the units of a row in a piece (tiles of 64 / parts rows)

@@ -39,6 +39,7 @@
 #include "common.h"
 #include "llmp_hip.h"
 #include "vecq_common.h"
+#include "vecq_q4k_part.h"
 #include "vecq_sorted_walk.h"
 
 namespace llmp_hip {
@@ -51,7 +52,6 @@ constexpr float kLift = 524288.0f;  // 2^19
 typedef float V16f __attribute__((ext_vector_type(16)));
 typedef _Float16 H2 __attribute__((ext_vector_type(2)));
 typedef _Float16 H8 __attribute__((ext_vector_type(8)));
-typedef __bf16 B8 __attribute__((ext_vector_type(8)));
 
 // The staged tokens: TG groups of 32, in operand layout, a super-block after the other.
 //   codes   [sub-block][half of its K steps][K half][token] 16 bytes: eight codes as F16, a dword's in the order 0, 2, 1, 3;
@@ -72,7 +72,7 @@ struct Staged {
 };
 
 // A lane's part of one super-block of its row: the header and its 16 bytes of each pair of sub-blocks.
-struct RowPart {
+struct HalfPart {
   U32x4 header;
   U32x4 q[4];
 };
@@ -107,18 +107,6 @@ __device__ __forceinline__ H2 Scale(const Q4KHeader& h, int g) {
                     : __builtin_elementwise_fma(biased, Both(2.0f), Both(-2048.0f));
 }
 
-// The eight minimums as bf16.
-__device__ __forceinline__ B8 Minimums(const Q4KHeader& h) {
-  U32x4 m;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t word = h.mn[i >> 1] >> (16 * (i & 1));
-    const float m0 = static_cast<float>(word & 0xFFu), m1 = static_cast<float>((word >> 8) & 0xFFu);
-    m[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, m1), __builtin_bit_cast(uint32_t, m0), 0x07060302u);
-  }
-  return __builtin_bit_cast(B8, m);
-}
-
 // Eight codes (two dwords) as F16, a dword's in the order 0, 2, 1, 3: a code plus 128 is a byte, 1024 + 128 + code less 1152.
 __device__ __forceinline__ U32x4 TokenCodes(uint32_t w0, uint32_t w1) {
   const uint32_t a = w0 ^ 0x80808080u, c = w1 ^ 0x80808080u;
@@ -129,21 +117,6 @@ __device__ __forceinline__ U32x4 TokenCodes(uint32_t w0, uint32_t w1) {
   packed.z = __builtin_bit_cast(uint32_t, Biased(c, k02) - Both(1152.0f));
   packed.w = __builtin_bit_cast(uint32_t, Biased(c, k13) - Both(1152.0f));
   return packed;
-}
-
-// d8 * sum in three groups of eight bits, each in the high half of its word: 11 bits times 12, nothing of a finite product
-// is left over (one that is not finite is its leading group alone).
-struct SumParts {
-  uint32_t lead, middle, last;
-};
-__device__ __forceinline__ SumParts SplitSum(float d8, int sum) {
-  const float product = d8 * static_cast<float>(sum);
-  SumParts parts;
-  parts.lead = __builtin_bit_cast(uint32_t, product) & 0xFFFF0000u;
-  const float rest = __builtin_isfinite(product) ? product - __builtin_bit_cast(float, parts.lead) : 0.0f;
-  parts.middle = __builtin_bit_cast(uint32_t, rest) & 0xFFFF0000u;
-  parts.last = __builtin_bit_cast(uint32_t, rest - __builtin_bit_cast(float, parts.middle));
-  return parts;
 }
 
 // One Q8_1 block (sub-block g of super-block sb) of token t into the staged layout.
@@ -173,7 +146,7 @@ __device__ __forceinline__ void StageBlock(const uint32_t (&w)[9], int t, int sb
 // One super-block of a tile times the staged tokens of LIVE groups. `staged`: the super-block's; `lane_at`: 16 (lane % 32),
 // this lane's token, `rows`: 64 floats of LDS, the wave's own.
 template <int TG, int LIVE>
-__device__ __forceinline__ void DotStep(const RowPart& part, int kg, const uint8_t* staged, int lane_at, float* rows, int lane,
+__device__ __forceinline__ void DotStep(const HalfPart& part, int kg, const uint8_t* staged, int lane_at, float* rows, int lane,
                                         V16f (&out)[TG]) {
   using L = Staged<TG>;
   const Q4KHeader h = DecodeQ4KHeader(part.header);
@@ -320,7 +293,7 @@ __global__ __launch_bounds__(Staged<TG>::kGroup, 1) void VecQSorted(const VecQAr
     // Queued here and no later. A wave's next tile is the next that no wave has begun: of a SIMD's waves the older get
     // more of it. Past the segment's end its last tile again: a load under a branch would make every wait for loads a
     // wait for all of them.
-    auto fetch = [&](RowPart& part) {
+    auto fetch = [&](HalfPart& part) {
       if (fetch_sb == nsb) {
         fetch_sb = 0;
         int taken = 0;
@@ -335,7 +308,7 @@ __global__ __launch_bounds__(Staged<TG>::kGroup, 1) void VecQSorted(const VecQAr
       __builtin_amdgcn_sched_barrier(0);
       ++fetch_sb;
     };
-    RowPart even, odd;
+    HalfPart even, odd;
     aim();
     fetch(even);
 
@@ -387,7 +360,7 @@ __global__ __launch_bounds__(Staged<TG>::kGroup, 1) void VecQSorted(const VecQAr
         out[tg] = V16f{};
       }
     };
-    auto step = [&](const RowPart& part) {
+    auto step = [&](const HalfPart& part) {
       const uint8_t* at = lds + sb * L::kAll;
       if (TG == 1 || live == TG) {
         DotStep<TG, TG>(part, kg, at, lane_at, rows, lane, out);

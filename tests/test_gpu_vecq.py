@@ -284,6 +284,32 @@ def test_sorted_q4k_rows_at_the_edges_of_passes_and_tiles(device, k, n, glu):
     assert np.array_equal(product(last, (counts > 0).astype(np.int32)).view(np.uint32), got[last].view(np.uint32))
 
 
+@pytest.mark.parametrize("k,n,tokens,glu,used", [(256, 17, 9, False, 1), (256, 1, 16, True, 1), (1280, 33, 11, False, 3),
+                                                 (2304, 100, 13, True, 2), (4096, 520, 16, False, 1), (4352, 24, 10, True, 1),
+                                                 (8448, 40, 10, False, 1), (15360, 48, 12, False, 1), (15360, 31, 16, False, 2),
+                                                 (512, 8200, 9, True, 1), (1024, 40000, 12, False, 1)])
+def test_q4k_tiles_of_sixteen_rows(device, k, n, tokens, glu, used):
+    """The default of nine and more tokens: tiles that end past the matrix, rows of fewer
+    super-blocks than a workgroup has waves and of several spans, workgroups that take tiles more than once, grouped matrices.
+    Against the oracle within 1e-5 of the RMS (sums of up to 480 F32 terms that cancel); a token's values bit for bit whatever
+    the tokens beside it."""
+    blocks = k // 256
+    up = make_weights(Q4_K, used * n, k, 95)
+    gate = make_weights(Q4_K, used * n, k, 96) if glu else None
+    kind = ops.GLU_GEGLU if glu else ops.GLU_NONE
+    y_row = ops.padded_k(k) // 32
+    q8 = oracle.q8_1_quantize(synth.activations(tokens * used, k, 97))
+    common = dict(used=used, stride_expert=n * blocks, y_token=y_row * used, y_slot=y_row, glu=kind)
+    want = oracle.vecq(Q4_K, up, q8, k, n, gate=gate, tokens=tokens, threads=oracle.max_threads(), **common)
+    gd = None if gate is None else dev(gate, device)
+    got = ops.vecq(Q4_K, dev(up, device), dev(q8, device), k, n, gate=gd, tokens=tokens, **common).cpu().numpy()
+    ok, worst = rel_close(got, want, 1e-5, floor=1.0)
+    assert ok, worst
+    fewest = 9
+    fewer = ops.vecq(Q4_K, dev(up, device), dev(q8, device), k, n, gate=gd, tokens=fewest, **common).cpu().numpy()
+    assert np.array_equal(fewer.view(np.uint32), got[:fewest].view(np.uint32))
+
+
 def same_sums(t, a, b):
     """Q8_0: the matrix-core kernel repeats the flat kernel's float operations and its summation tree, bit for bit.
     Q4_K: its sub-block sums are the same exact integers, scaled and added in another order (one fma a sub-block
