@@ -897,6 +897,19 @@ struct WideSides {
 };
 constexpr int kWideTiles = 4;  // 16-column tiles a wave
 
+// LDS: the waves' rings, and behind them, where both fit 64 KB, the meeting's sums of sixteen rows (else over the rings, 32
+// rows at a time). Apart, a workgroup takes several column blocks one after the other, the next one's first stages, words
+// and rows on their way under the last one's meeting: a wave has often no more than four steps of a column block, and a
+// workgroup's start (its first stage's trip from memory) and its meeting cost as much as they do. 4096 x 14336 at four bits,
+// 77 rows, where a compute unit's registers hold one workgroup and 3.5 are its share: 38.4 -> 36.0 us.
+// (Two row tiles take 23.4 us so against 23.1; nine tiles' sums leave no registers for the next column block's.)
+template <int BITS, int TILES>
+struct WideLds {
+  static constexpr int kRings = kProductWaves * kRingDepth * ((2 * kWideTiles * BITS * 32 + 1023) / 1024) * 1024;
+  static constexpr bool kApart = TILES == 5 && kRings + kReduceBytes / 2 <= 64 * 1024;
+  static constexpr int kBytes = kApart ? kRings + kReduceBytes / 2 : kRings > kReduceBytes ? kRings : kReduceBytes;
+};
+
 template <int CB, int BITS, int TILES>
 __global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const WideSides sides, int m, int n, int k,
                                                                        int blocks_per_wave) {
@@ -921,19 +934,32 @@ __global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const Wi
   const Place p = PlaceOf(lane);
   const Windows<BITS> windows = WindowsOf<BITS>(p.first);
   const int64_t row_bytes = static_cast<int64_t>(n / 16) * kTileBytes;
-  const uint8_t* source = trellis + static_cast<int64_t>(blockIdx.x) * kStepBytes;
+  constexpr bool kApart = WideLds<BITS, TILES>::kApart;
+  const int column_blocks = n / 64;
+  const int mine = kApart ? (column_blocks - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x) : 1;
   const uint32_t ring_at = LdsAddress(ring);
   const int chunks = (m + 15) / 16;  // TILES or, of the last pass, fewer
 
-  auto fetch = [&](int step) {
-    const uint8_t* from = source + static_cast<int64_t>(2 * min(step, last - 1)) * row_bytes;
-    uint8_t* to = ring + (step % kRingDepth) * kStageBytes;
+  int next_step = first, next_block = 0, next_slot = 0;  // (a wave's steps are whole 128 blocks: a column block's begin at slot 0)
+  auto fetch = [&](int step) {  // apart: the next in order, whatever `step`
+    const int block = kApart ? blockIdx.x + next_block * gridDim.x : blockIdx.x;
+    const int64_t at_step = kApart ? next_step : min(step, last - 1);
+    const uint8_t* from = trellis + static_cast<int64_t>(block) * kStepBytes + 2 * at_step * row_bytes;
+    uint8_t* to = ring + (kApart ? next_slot : step % kRingDepth) * kStageBytes;
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int unit = i * 64 + lane;
       const int64_t at = unit < kUnits ? unit * 16 : row_bytes + (unit - kUnits) * 16;
       if (unit < 2 * kUnits) {
         __builtin_amdgcn_global_load_lds((GlobalPointer)(from + at), (LdsPointer)(to + i * 1024), 16, 0, 0);
+      }
+    }
+    if constexpr (kApart) {
+      next_slot = (next_slot + 1) % kRingDepth;
+      if (next_step + 1 < last) {
+        ++next_step;
+      } else if (next_block + 1 < mine) {  // (past the last one's end its last stage again)
+        next_step = first, ++next_block;
       }
     }
   };
@@ -961,16 +987,50 @@ __global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const Wi
   };
 
   V4f acc[TILES][kWideTiles];
+  auto clear = [&]() {
 #pragma unroll
-  for (int r = 0; r < TILES; ++r)
+    for (int r = 0; r < TILES; ++r)
 #pragma unroll
-    for (int t = 0; t < kWideTiles; ++t) acc[r][t] = V4f{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int t = 0; t < kWideTiles; ++t) acc[r][t] = V4f{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  clear();
+
+  // The waves' sums in wave order through LDS, 16 or 32 rows at a time: [wave][row tile][4 t + q][lane].
+  constexpr int kAtOnce = kApart ? 1 : 2;  // row tiles
+  float* sums = reinterpret_cast<float*>(lds + (kApart ? WideLds<BITS, TILES>::kRings : 0));
+  auto meet = [&](int block) {
+    float* out = partial + static_cast<int64_t>(blockIdx.y) * m * n + block * 64;
+#pragma unroll
+    for (int r0 = 0; r0 < TILES; r0 += kAtOnce) {
+      __syncthreads();
+#pragma unroll
+      for (int r = r0; r < r0 + kAtOnce && r < TILES; ++r)
+#pragma unroll
+        for (int t = 0; t < kWideTiles; ++t)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sums[((wave * kAtOnce + r - r0) * 16 + t * 4 + q) * 64 + lane] = acc[r][t][q];
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < 2 * kAtOnce; ++j) {
+        const int e = tid + j * (kProductWaves * 64);  // of kAtOnce x 16 x 64
+        const int r = r0 + (e >> 10);
+        if (r < TILES) {
+          float total = sums[e];
+#pragma unroll
+          for (int w = 1; w < kProductWaves; ++w) total += sums[w * (kAtOnce * 1024) + e];
+          const int tq = (e >> 6) & 15, l = e & 63;
+          const int row = 16 * r + 4 * (l >> 4) + (tq & 3);
+          if (row < m) out[static_cast<int64_t>(row) * n + (tq >> 2) * 16 + (l & 15)] = total;
+        }
+      }
+    }
+  };
 
   if (first < last) {
     uint32_t words[2][2 * kWideTiles][kWords];
     U32x4 x[TILES];
     auto ask_rows = [&](int step) {  // (a chunk past the pass's last is its last again: no load is skipped)
-      const uint8_t* at = rows + (static_cast<int64_t>(min(step, last - 1)) * chunks * 64 + lane) * 16;
+      const uint8_t* at = rows + (static_cast<int64_t>(kApart ? step : min(step, last - 1)) * chunks * 64 + lane) * 16;
 #pragma unroll
       for (int r = 0; r < TILES; ++r) {
         const uint8_t* from = at + min(r, chunks - 1) * 1024;
@@ -1006,11 +1066,17 @@ __global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const Wi
 #pragma unroll
         for (int t = 0; t < kWideTiles; ++t)
           acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(Half8, x[r]), wv[t], acc[r][t], 0, 0, 0);
-      ask_rows(step + 1);
+      ask_rows(!kApart || step + 1 < last ? step + 1 : first);
     };
-    for (int step = first; step < last; step += 2) {
-      one(step, 0);
-      one(step + 1, 1);
+    for (int u = 0; u < mine; ++u) {
+      for (int step = first; step < last; step += 2) {
+        one(step, 0);
+        one(step + 1, 1);
+      }
+      if constexpr (kApart) {
+        meet(blockIdx.x + u * gridDim.x);
+        clear();
+      }
     }
     // (As in the product of sixteen rows: nothing asked for past the end is left on its way to a register.)
     LdsWaited();
@@ -1018,35 +1084,10 @@ __global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const Wi
     LoadsWaited<0>();
 #pragma unroll
     for (int r = 0; r < TILES; ++r) LLMP_TIE(x[r]);
+  } else if constexpr (kApart) {  // no K of its own: the others' meetings, with sums of zero
+    for (int u = 0; u < mine; ++u) meet(blockIdx.x + u * gridDim.x);
   }
-
-  // The waves' sums in wave order through LDS, 32 rows at a time: [wave][row tile][4 t + q][lane].
-  float* sums = reinterpret_cast<float*>(lds);
-  float* out = partial + static_cast<int64_t>(blockIdx.y) * m * n + blockIdx.x * 64;
-#pragma unroll
-  for (int r0 = 0; r0 < TILES; r0 += 2) {
-    __syncthreads();
-#pragma unroll
-    for (int r = r0; r < r0 + 2 && r < TILES; ++r)
-#pragma unroll
-      for (int t = 0; t < kWideTiles; ++t)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sums[((wave * 2 + r - r0) * 16 + t * 4 + q) * 64 + lane] = acc[r][t][q];
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = tid + j * (kProductWaves * 64);  // of 2 x 16 x 64
-      const int r = r0 + (e >> 10);
-      if (r < TILES) {
-        float total = sums[e];
-#pragma unroll
-        for (int w = 1; w < kProductWaves; ++w) total += sums[w * 2048 + e];
-        const int tq = (e >> 6) & 15, l = e & 63;
-        const int row = 16 * r + 4 * (l >> 4) + (tq & 3);
-        if (row < m) out[static_cast<int64_t>(row) * n + (tq >> 2) * 16 + (l & 15)] = total;
-      }
-    }
-  }
+  if constexpr (!kApart) meet(blockIdx.x);
 }
 
 // Outer slices of K: enough workgroups for about 4096 waves, each wave at least one 128 block.
@@ -1176,14 +1217,28 @@ size_t PassBytes(const llmp_exl3_weights& w, int rows) {
   return PartialBytes(w, rows) + (rows > kPassRows ? static_cast<size_t>((rows + 15) / 16) * 16 * w.k * 2 : 0);
 }
 
+int ComputeUnits() {
+  static const int units = [] {
+    const int cus = llmp_hip_compute_units();
+    return cus > 0 ? cus : 256;
+  }();
+  return units;
+}
+
 template <int CB, int BITS, int TILES>
 void LaunchWide(const llmp_exl3_weights& w, const WideSides& sides, int count, int m, int slices, hipStream_t stream) {
-  constexpr int kRing = kProductWaves * kRingDepth * ((2 * kWideTiles * BITS * 32 + 1023) / 1024) * 1024;
-  constexpr int kLds = kRing > kReduceBytes ? kRing : kReduceBytes;
+  constexpr int kLds = WideLds<BITS, TILES>::kBytes;
   static_assert(kLds <= 64 * 1024, "more must be asked for, ahead of a capture too (llmp_hip_exl3_linear_static_prepare)");
   const int blocks = w.k / 128;
   const int per = (blocks + slices * kProductWaves - 1) / (slices * kProductWaves);
-  const dim3 grid(static_cast<unsigned>(w.n / 64), static_cast<unsigned>(slices), static_cast<unsigned>(count));
+  // As many workgroups as the registers hold at a time, each the same number of column blocks or one fewer.
+  int columns = w.n / 64;
+  if constexpr (WideLds<BITS, TILES>::kApart) {
+    const int resident = ComputeUnits();
+    const int share = (columns * slices * count + resident - 1) / resident;
+    columns = (columns + share - 1) / share;
+  }
+  const dim3 grid(static_cast<unsigned>(columns), static_cast<unsigned>(slices), static_cast<unsigned>(count));
   hipLaunchKernelGGL((WideProductKernel<CB, BITS, TILES>), grid, dim3(kProductWaves * 64), kLds, stream, sides, m, w.n, w.k, per);
 }
 
