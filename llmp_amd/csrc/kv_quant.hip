@@ -141,7 +141,27 @@ __global__ __launch_bounds__(kStoreThreads) void RopeSetRowsQuantKernel(const ll
   extern __shared__ float2 rotation[];  // of pair p: magnitude * (cos, sin)
   const int64_t token = blockIdx.x;
   const int half = s.n_dims / 2;
+  const int blocks_head = s.head_dim / 32, blocks_row = s.heads * blocks_head;
+  const bool wide = half % 32 == 0 && s.x_head_stride % 4 == 0 && s.x_token_stride % 4 == 0 &&
+                    reinterpret_cast<uintptr_t>(s.x) % 16 == 0;
+  // The first block's values and their partners are asked for ahead of the angles: behind the barrier they were a second
+  // trip to memory (a token of 8 heads of 256 values 4.14 -> 3.80 us, 64 tokens 4.30 -> 4.02).
+  float4 own[8], other[8];
+  auto load = [&](int block) {
+    const int head = block / blocks_head, first = (block - head * blocks_head) * 32;
+    const float* x = s.x + head * s.x_head_stride + token * s.x_token_stride;
+    const float4* at = reinterpret_cast<const float4*>(x + first);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) own[i] = at[i];
+    if (first < s.n_dims) {
+      const float4* partners = reinterpret_cast<const float4*>(x + (first < half ? first + half : first - half));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) other[i] = partners[i];
+    }
+  };
   const float position = static_cast<float>(s.pos[token]);
+  const int64_t row = s.ids[token];
+  if (wide && static_cast<int>(threadIdx.x) < blocks_row) load(threadIdx.x);
   float magnitude = s.attn_factor;
   if (s.ext_factor != 0.0f) magnitude *= 1.0f + 0.1f * logf(1.0f / s.freq_scale);
   for (int pair = threadIdx.x; pair < half; pair += kStoreThreads) {
@@ -157,10 +177,7 @@ __global__ __launch_bounds__(kStoreThreads) void RopeSetRowsQuantKernel(const ll
     rotation[pair] = make_float2(cosf(theta) * magnitude, sinf(theta) * magnitude);
   }
   __syncthreads();  // every thread: the loop below has no barrier
-  const int blocks_head = s.head_dim / 32, blocks_row = s.heads * blocks_head;
-  const bool wide = half % 32 == 0 && s.x_head_stride % 4 == 0 && s.x_token_stride % 4 == 0 &&
-                    reinterpret_cast<uintptr_t>(s.x) % 16 == 0;
-  uint8_t* to = static_cast<uint8_t*>(s.destination) + s.ids[token] * s.row_bytes;
+  uint8_t* to = static_cast<uint8_t*>(s.destination) + row * s.row_bytes;
   for (int block = threadIdx.x; block < blocks_row; block += kStoreThreads) {
     const int head = block / blocks_head;
     const int first = (block - head * blocks_head) * 32;  // channel within the head
@@ -169,16 +186,12 @@ __global__ __launch_bounds__(kStoreThreads) void RopeSetRowsQuantKernel(const ll
     if (wide) {
       // The block lies within one half of the rotated channels (or past them): its 32 values and their partners'
       // as 16-byte loads.
-      const float4* own = reinterpret_cast<const float4*>(x + first);
+      if (block != static_cast<int>(threadIdx.x)) load(block);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float4 f = own[i];
-        v[4 * i] = f.x, v[4 * i + 1] = f.y, v[4 * i + 2] = f.z, v[4 * i + 3] = f.w;
-      }
+      for (int i = 0; i < 8; ++i) v[4 * i] = own[i].x, v[4 * i + 1] = own[i].y, v[4 * i + 2] = own[i].z, v[4 * i + 3] = own[i].w;
       if (first < s.n_dims) {
         const bool lower = first < half;
         const int pair0 = lower ? first : first - half;
-        const float4* other = reinterpret_cast<const float4*>(x + (lower ? first + half : pair0));
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const float4 f = other[i];
