@@ -415,7 +415,7 @@ def other_configs(device, args, only=None):
                 q8 = ops.quantize_q8_1_rows(xs, route.token)
                 product = lambda i: ops.vecq_sorted(ops.TYPE_Q4_K, up_of(gus[i % sets]), q8, route.offsets, hidden, ffn, experts,
                                                     gate=gus[i % sets], stride_expert=gu_stride, glu=ops.GLU_SWIGLU, out=h)
-                kernel = "VecQMma<glu> over rows sorted by expert (gate/up)"
+                kernel = "VecQSorted<glu> over rows sorted by expert (gate/up)"
             product_us = timed(product, 2 * sets)
             product_bytes = distinct * gu_bytes + tokens * hidden * 4 + pairs * ffn * 4
             layer_bytes = distinct * (gu_bytes + dn_bytes) + tokens * hidden * 4 * 2

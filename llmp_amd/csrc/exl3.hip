@@ -1552,6 +1552,7 @@ extern "C" int llmp_hip_exl3_linear_static_prepare(const llmp_exl3_linear* op) {
     (void)llmp_hip::SizeProduct<decltype(cb)::value, decltype(bits)::value, true>();
     (void)llmp_hip::SizeProduct<decltype(cb)::value, decltype(bits)::value, false>();
   });
+  (void)llmp_hip::ComputeUnits();  // asked here, so that a captured linear asks the runtime for nothing but launches
   return LaunchStatus("exl3.linear_static_prepare");
 }
 

@@ -37,12 +37,12 @@
 // matrices with a GLU) and all of K (rows of up to eight super-blocks) or one half of it (two
 // waves a tile, meeting in LDS).
 //
-// On this chip the vector unit and the matrix cores of a SIMD do not run at the same time (448
-// fma and 32 of these products a wave take the sum of their separate times at one, two and four
-// waves a SIMD): a step costs its vector instructions at 4 cycles plus its matrix instructions at
-// 16 (F16) and 32 (F32) cycles, and most of it is preparing the weight operand, which is why a
-// pass takes as many tokens as LDS holds. Sorted rows (an expert's rows, any number) are shared
-// among the workgroups by cost, not by expert: see the kernel.
+// What bounds it is vector issue: a step costs its vector instructions at 4 cycles, half of its F16 matrix instructions'
+// 16 cycles (16 fma and four of these products a wave and round, four waves a SIMD: 101 cycles where each alone takes 68)
+// and all of its F32 ones' 32, and most of it is preparing the weight operand, which is why a pass takes as many tokens as
+// LDS holds. Sorted rows (an expert's rows, any number) are shared among the workgroups by cost, not by expert
+// (vecq_sorted_walk.h); those of up to eight super-blocks go to vecq_sorted.hip, and dense products of nine to sixteen
+// tokens to vecq_tile16.hip by default.
 
 #include <hip/hip_runtime.h>
 
@@ -187,9 +187,8 @@ __device__ __forceinline__ void End(const Prepared& prepared, int kg, const floa
 // 4 (lane / 16) + q. `codes`, `d8`, `ds8`: this lane's places in the super-block's staged tokens; LIVE: the token
 // groups the pass holds (a constant: a branch a group would cut the step into pieces). A pair of sub-blocks at a
 // time, both matrices against the same token operands (read from LDS once), one matrix after the other, the
-// compiler kept from moving work between them: the matrix cores and the vector unit do not run at the same
-// time on this chip, so there is nothing to gain from interleaving further, and holding more operands and
-// results at once costs registers the kernel does not have.
+// compiler kept from moving work between them: the SIMD's other waves run under a wave's matrix instructions, and
+// holding more operands and results at once costs registers the kernel does not have.
 template <bool kGlu, int TG, int MT, int LIVE>
 __device__ __forceinline__ void DotStep(const RowPart& up, const RowPart& gate, int kg, const uint8_t* codes, const uint8_t* d8,
                                         const uint8_t* ds8, V4f (&up_out)[TG], V4f (&gate_out)[TG]) {
