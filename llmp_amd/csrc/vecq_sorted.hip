@@ -382,10 +382,12 @@ __global__ __launch_bounds__(Staged<TG>::kGroup, 1) void VecQSorted(const VecQAr
     }
   };
 
-  // A step of one and of two live token groups takes 1.0 and 1.6 us of a SIMD, a staging 4 to 5 us of the workgroup: in
-  // units of a fifth of a step, four SIMDs' of which pass at a time.
+  // A step of one and of two live token groups takes 1.0 and 1.6 us of a SIMD, a staging 4 to 5 us of the workgroup and the
+  // wait for the last segment's tiles before it as much again: in units of a fifth of a step, four SIMDs' of which pass at a
+  // time. (With the staging alone, half of it: 1024 -> 2 x 768 of 64 experts 46 -> 42.5 us, 1536 -> 2 x 768 60 -> 57.4, 768 ->
+  // 2048 of 128 experts 49.6 -> 48.3; half as much again is no better.)
   auto cost_of = [nsb](int m) { return nsb * (m <= kTokens ? 5 : 8); };
-  auto fixed_of = [nsb](int m) { return 50 + 6 * nsb * (m <= kTokens ? 1 : TG); };
+  auto fixed_of = [nsb](int m) { return 110 + 10 * nsb * (m <= kTokens ? 1 : TG); };
   WalkSortedRows(a.offsets, d.used, tiles, TG * kTokens, fixed_of, cost_of, run);
 }
 
