@@ -9,7 +9,9 @@ only those asked for since the barrier before may be on their way (at the first,
 
 exl3.hip, the packed products: words and activations are loaded into registers by instructions, from LDS and from memory.
 From such a load to the wait that covers it, past the loop too, no instruction may name a register that it writes: the
-compiler takes them for written, copies them, and gives those that nothing reads to other values.
+compiler takes them for written, copies them, and gives those that nothing reads to other values. The weights go by a ring
+of four stages in LDS: a stage's words may be asked for when its loads have landed, and its place filled again when they
+have come.
 
 Needs hipcc, no GPU. Run by the library's build (__graft_entry__.build) and by tests/test_counted_waits.py;
 `python check_counted_waits.py` runs it alone."""
@@ -169,6 +171,57 @@ def check_registers(name, body):
     follow(body, ((), ()), step)
 
 
+RING_STAGES = 4  # exl3.hip's kRingDepth
+ASK_LEAST = 16   # words of a stage that a lane asks for at a time, at least
+
+
+def check_ring(name, body, loads):
+    """Raises AssertionError where a stage of the ring (`loads` loads to LDS, in order) may not have landed when its words are
+    asked for, or is asked for again while the words of the stage in its place may still be on their way. An ask is a run
+    of reads of LDS written by hand with no wait among them (shorter runs read the activations, which lie apart). Of two parts
+    that lanes go through by a condition, a load in the second is one in the first for the other lanes, as far as those go."""
+
+    def step(code, own, state):
+        # Loads to LDS issued since the first load of the oldest stage whose words have not come; of the stages since, those
+        # asked for; the reads of LDS since the last wait; the memory operations on their way, oldest first, True: to LDS.
+        # And the loads to LDS of a part under a condition (-1: in none), and of the first part's those the second has yet to repeat.
+        held, asked, reads, queue, part, again = state
+        if code.startswith("global_load_lds"):
+            held, again, part = held + (again == 0), max(again - 1, 0), part + (part >= 0)
+            queue += (True,)
+            assert held <= RING_STAGES * loads, f"{name}: a stage is filled again before its words have come"
+        elif MEMORY.match(code):
+            queue += (False,)
+        elif own and code.startswith("ds_read"):
+            reads += 1
+            if reads == ASK_LEAST:
+                asked += 1
+                late = sum(queue) - (held - asked * loads)
+                assert late <= 0, f"{name}: {late} loads of a stage may be on their way when its words are asked for"
+        elif code.startswith("s_waitcnt"):
+            left = re.search(r"vmcnt\((\d+)\)", code)
+            if left:
+                queue = after_wait(queue, int(left.group(1)))
+            if "lgkmcnt(0)" in code:
+                held -= asked * loads
+                asked, reads = 0, 0
+        elif "_saveexec_b64" in code:
+            part, again = 0, max(part, 0) if code.startswith("s_andn2") else 0
+        elif code.startswith("s_or_b64 exec"):
+            part, again = -1, 0
+        while queue and not queue[0]:
+            queue = queue[1:]
+        return held, asked, reads, queue, part, again
+
+    follow(body, (0, 0, 0, (), -1, 0), step)
+
+
+def ring_loads(name):
+    """Of a packed product: its loads to LDS a stage, 256 bytes a bit of a weight, a KB a load."""
+    bits = int(re.search(r"ProductKernelILi\d+ELi(\d+)E", name).group(1))
+    return (bits * 256 + 1023) // 1024
+
+
 def check():
     """The number of kernels followed; raises AssertionError (or the compiler's error) where a count does not hold."""
     with concurrent.futures.ThreadPoolExecutor() as pool:
@@ -181,6 +234,7 @@ def check():
     products = 0
     for name, body in kernels_of(exl3, "WideProductKernel|13ProductKernel"):
         check_registers(name, body)
+        check_ring(name, body, ring_loads(name))
         products += 1
     assert products >= 48, f"only {products} packed products were found"
     return kernels + products

@@ -580,7 +580,9 @@ struct ProductSides {  // one or two linears a launch (grid z)
 // LDS accesses written as instructions, for the product's loop: while a global_load_lds is in flight the
 // compiler makes every access of LDS it knows of wait until all of them have landed (it cannot tell which the
 // access could alias), the ring's newest fetch included, and the ring would never overlap a fetch with a decode.
-// The loop orders its reads and the loads itself: LdsWaited, then Tie on every register read.
+// The loop orders its reads and the loads itself: LdsWaited, then Tie on every register read. Its waits count the ring's loads,
+// which the compiler may move, together with those written here: a load of these and a wait touch memory, as far as the
+// compiler knows, so that nothing of either kind moves across the other (check_counted_waits.py reads what came of it).
 #define LLMP_TIE(x) asm volatile("" : "+v"(x))
 template <int OFFSET>
 __device__ __forceinline__ uint32_t LdsRead4(uint32_t at) {
@@ -589,12 +591,12 @@ __device__ __forceinline__ uint32_t LdsRead4(uint32_t at) {
   return v;
 }
 __device__ __forceinline__ void LdsWrite4(uint32_t at, uint32_t value) { asm volatile("ds_write_b32 %0, %1" : : "v"(at), "v"(value)); }
-__device__ __forceinline__ void LdsWaited() { asm volatile("s_waitcnt lgkmcnt(0)"); }
+__device__ __forceinline__ void LdsWaited() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 // The same for the few loads from global memory into registers inside that loop: the compiler's own wait for one
 // is a wait for every load in flight, the ring's included.
 __device__ __forceinline__ uint32_t GlobalLoad4(const void* from) {
   uint32_t v;
-  asm volatile("global_load_dword %0, %1, off" : "=v"(v) : "v"(from));
+  asm volatile("global_load_dword %0, %1, off" : "=v"(v) : "v"(from) : "memory");
   return v;
 }
 template <int LEFT>
@@ -1034,7 +1036,7 @@ __global__ __launch_bounds__(kProductWaves * 64) void WideProductKernel(const Wi
 #pragma unroll
       for (int r = 0; r < TILES; ++r) {
         const uint8_t* from = at + min(r, chunks - 1) * 1024;
-        asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(x[r]) : "v"(from));
+        asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(x[r]) : "v"(from) : "memory");
       }
     };
 #pragma unroll

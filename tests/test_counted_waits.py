@@ -69,3 +69,31 @@ def test_a_register_named_while_a_load_to_it_is_on_its_way_is_found(module, betw
     else:
         with pytest.raises(AssertionError, match="on its way"):
             module.check_registers("kernel", body)
+
+
+@pytest.mark.parametrize("ahead,loop,holds", [
+    (3, "load vm2 lgkm ask", True),
+    (3, "load vm3 lgkm ask", False),  # a wait one short
+    (3, "vm2 lgkm ask load", False),  # the next stage asked for behind the words: the wait counts a load that is not there
+    (4, "load vm3 lgkm ask", False),  # a stage filled while it is read
+])
+def test_a_stage_asked_for_before_it_landed_is_found(module, ahead, loop, holds):
+    """A ring of one load a stage whose words are asked for a step ahead of their use, in the loop's order and in others."""
+    ask = "\n".join(["\t;;#ASMSTART\n\tds_read_b32 v1, v2\n\t;;#ASMEND"] * module.ASK_LEAST)
+    text = {"load": "\tglobal_load_lds_dwordx4 v[2:3], off", "vm2": "\ts_waitcnt vmcnt(2)", "vm3": "\ts_waitcnt vmcnt(3)",
+            "lgkm": "\ts_waitcnt lgkmcnt(0)", "ask": ask}
+    body = "\n".join([text["load"]] * ahead + [f"\ts_waitcnt vmcnt({ahead - 1})", ask, ".LBB0_1:"] + [text[w] for w in loop.split()] +
+                     ["\ts_cbranch_scc1 .LBB0_1", "\ts_waitcnt vmcnt(0) lgkmcnt(0)", "\ts_endpgm"])
+    if holds:
+        module.check_ring("kernel", body, 1)
+    else:
+        with pytest.raises(AssertionError, match="words"):
+            module.check_ring("kernel", body, 1)
+
+
+def test_the_packed_products_loads_keep_their_places_among_the_compilers():
+    """Their waits count the ring's loads, which the compiler may move, with those written as instructions: each of these, and
+    the wait for LDS, says that it touches memory, so that nothing moves across it."""
+    with open(os.path.join(ROOT, "llmp_amd", "csrc", "exl3.hip")) as f:
+        written = re.findall(r'asm volatile\("(?:global_load|s_waitcnt)[^;]*;', f.read())
+    assert len(written) >= 3 and all('"memory"' in w for w in written), written
