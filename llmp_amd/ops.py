@@ -131,6 +131,7 @@ def vecq_sorted(t, w, q8, offsets, k, nrows, experts, *, gate=None, stride_row=N
                 glu=GLU_NONE, limit=0.0, variant=-1, out=None, rows=None):
     """llmp.vecq over rows sorted by expert: q8 [rows, blocks*36] -> float32 [rows, nrows]. `rows` (int32): sorted row r's
     activations are q8's row rows[r] (where sorted_takes_rows says so)."""
+    assert rows is None or (rows.dtype == torch.int32 and rows.is_contiguous())
     lib = _lib.load()
     count = q8.shape[0] if rows is None else rows.numel()
     if out is None:
@@ -145,9 +146,9 @@ def vecq_sorted(t, w, q8, offsets, k, nrows, experts, *, gate=None, stride_row=N
     return out
 
 
-def sorted_takes_rows(t, w, k, nrows, *, gate=None, stride_expert=0):
+def sorted_takes_rows(t, w, k, nrows, *, gate=None, stride_row=None, stride_expert=0):
     """Whether vecq_sorted over these weights takes its activations by index."""
-    d = _desc(t, w, k, nrows, gate=gate, q8=None, ids=None, tokens=1, used=1, stride_row=None, stride_expert=stride_expert,
+    d = _desc(t, w, k, nrows, gate=gate, q8=None, ids=None, tokens=1, used=1, stride_row=stride_row, stride_expert=stride_expert,
               y_token=0, y_slot=0, glu=GLU_NONE, limit=0.0, out=w)
     return _lib.load().llmp_hip_vecq_sorted_takes_rows(t, C.byref(d)) == 1
 

@@ -339,3 +339,20 @@ def test_rope_store_refusals_queue_nothing():
         assert lib.llmp_hip_rope_set_rows_quant(C.byref(s), None) > 0 and why in lib.llmp_hip_last_error(), field
         setattr(s, field, old)
     assert lib.llmp_hip_rope_set_rows_quant(None, None) > 0
+
+
+def test_sorted_rows_by_index_are_asked_about_as_they_run():
+    """sorted_takes_rows sees the row stride that the product will have (the Q8_0 matrix-core form takes even ones alone), and
+    an index that is not int32 in one piece is refused ahead of the launch, which would read it as such."""
+    import torch
+
+    from llmp_amd import ops
+
+    w = torch.zeros(4 * 9 * 34, dtype=torch.uint8)
+    assert ops.sorted_takes_rows(ops.TYPE_Q8_0, w, 256, 4) and ops.sorted_takes_rows(ops.TYPE_Q8_0, w, 256, 4, stride_row=10)
+    assert not ops.sorted_takes_rows(ops.TYPE_Q8_0, w, 256, 4, stride_row=9)
+    q8 = torch.zeros((2, 16 * 36), dtype=torch.uint8)
+    offsets = torch.tensor([0, 2], dtype=torch.int32)
+    for rows in (torch.arange(2), torch.arange(4, dtype=torch.int32)[::2]):
+        with pytest.raises(AssertionError):
+            ops.vecq_sorted(ops.TYPE_Q8_0, w, q8, offsets, 256, 4, 1, rows=rows)
