@@ -284,6 +284,36 @@ def test_sorted_q4k_rows_at_the_edges_of_passes_and_tiles(device, k, n, glu):
     assert np.array_equal(product(last, (counts > 0).astype(np.int32)).view(np.uint32), got[last].view(np.uint32))
 
 
+@pytest.mark.parametrize("experts,k,n", [(1, 256, 33), (64, 256, 64), (65, 2304, 96), (129, 512, 40), (130, 256, 1041), (130, 2048, 700),
+                                         (513, 512, 40), (4100, 256, 8), (4100, 2304, 8)])
+def test_sorted_q4k_rows_of_few_and_of_thousands_of_experts(device, experts, k, n):
+    """The workgroups' shares where a lane of the walk has one expert, two, and runs of more than it reads at a time, most
+    experts without rows, the first and the last among them; tiles enough for a wave to have several of a segment, whose
+    tokens are then all staged, and too few for that. Against the oracle, within 1e-5 of the RMS (sums of up to 72 F32 terms
+    that cancel), and a row's values bit for bit whatever rows stand beside it."""
+    g = synth.rng(93 + experts)
+    counts = g.choice(np.array([0, 0, 0, 1, 3, 9, 17], dtype=np.int32), size=experts)
+    counts[[0, -1]] = 0
+    counts[experts // 2] = 70
+    rows, blocks = int(counts.sum()), k // 256
+    w = make_weights(Q4_K, experts * n, k, 94).reshape(experts, -1)
+    q8 = oracle.q8_1_quantize(synth.activations(rows, k, 95)).reshape(rows, -1)
+    ids = np.repeat(np.arange(experts, dtype=np.int32), counts).reshape(-1, 1)
+    want = oracle.vecq(Q4_K, w, q8, k, n, ids=ids, tokens=rows, used=1, stride_expert=n * blocks, experts=experts,
+                       threads=oracle.max_threads()).reshape(rows, n)
+    wd = dev(w, device)
+
+    def product(picked, sizes):
+        offsets = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+        return ops.vecq_sorted(Q4_K, wd, dev(q8[picked], device), dev(offsets, device), k, n, experts, stride_expert=n * blocks).cpu().numpy()
+
+    got = product(np.arange(rows), counts)
+    ok, worst = rel_close(got, want, 1e-5, floor=1.0)
+    assert ok, worst
+    last = np.cumsum(counts)[counts > 0] - 1
+    assert np.array_equal(product(last, (counts > 0).astype(np.int32)).view(np.uint32), got[last].view(np.uint32))
+
+
 @pytest.mark.parametrize("k,n,tokens,glu,used", [(256, 17, 9, False, 1), (256, 1, 16, True, 1), (1280, 33, 11, False, 3),
                                                  (2304, 100, 13, True, 2), (4096, 520, 16, False, 1), (4352, 24, 10, True, 1),
                                                  (8448, 40, 10, False, 1), (15360, 48, 12, False, 1), (15360, 31, 16, False, 2),
