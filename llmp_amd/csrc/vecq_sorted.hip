@@ -255,12 +255,17 @@ __global__ __launch_bounds__(Staged<TG>::kGroup, 1) void VecQSorted(const VecQAr
 
     // The tokens' blocks are asked for before the weights (loads return in order, and the tokens are needed whole before
     // the first step), staged after the first weights are. Eight consecutive threads hold the same block of eight
-    // consecutive tokens, whose 16-byte pieces lie side by side in LDS.
-    const int staged = live * kTokens * nsb * 8;
+    // consecutive tokens, whose 16-byte pieces lie side by side in LDS. Where a wave has no second tile the staging is much
+    // of the segment, and only eights of tokens that hold rows are staged (1536 -> 512, four rows of each of 64 experts 17.6
+    // -> 16.6 us; with more tiles nothing gained: 1536 -> 2 x 4096, two rows of 128, 190 us, 195 so); the columns past those
+    // are what LDS held: a result's column is its own operand column's, and theirs are dropped.
+    const bool few = seg.group_count <= kWaves;
+    const int eights_log = few && seg.m <= 8 ? 0 : few && seg.m <= 16 ? 1 : live == 1 ? 2 : 3;
+    const int staged = nsb << (6 + eights_log);
     auto place = [&](int index, int* t, int* b) {
       const int rest = index >> 6;
-      const int sb = rest / (live * (kTokens / 8));
-      *t = (rest - sb * live * (kTokens / 8)) * 8 + (index & 7);
+      const int sb = rest >> eights_log;
+      *t = (rest - (sb << eights_log)) * 8 + (index & 7);
       *b = sb * 8 + ((index >> 3) & 7);
     };
     auto fetch_block = [&](int t, int b, uint32_t(&w)[9]) {
