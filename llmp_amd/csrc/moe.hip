@@ -157,7 +157,7 @@ __global__ void RouteAssign(const int32_t* __restrict__ ids, int ids_stride, Rou
 // own are counted a wave at a time: the lanes that hold the same id are found by a ballot a bit of the id, which gives
 // each its rank, and the first of them notes how many. A slot's row is then its expert's first row, plus the expert's
 // slots before the workgroup's, plus those of the workgroup's earlier waves, plus its rank. What bounds it is latency:
-// the launch, one trip for the ids, three barriers. One workgroup doing it all (a prefix over 64 runs of 128 counters and
+// the launch, one trip for the ids, three or four barriers. One workgroup doing it all (a prefix over 64 runs of 128 counters and
 // up to 63 compares a slot end to end on one compute unit) took 13.4 us at 4096 slots of 128 experts.
 // LDS, ints: the waves' counts [wave][expert], zeros before the slots' [expert], counts before and after [2][expert],
 // offsets [expert + 1].
@@ -170,8 +170,13 @@ __host__ __device__ inline int64_t RouteSpreadInts(int64_t slots, int experts) {
   return (waves + 3) * experts + 1;
 }
 
+// kOneWave: up to 128 experts, whose totals the first wave scans by itself. More are scanned by all waves, whose sums meet at
+// a further barrier, and a workgroup alone neither clears nor reads the counts of others (0.2 us the more at 128 experts; by
+// the first wave alone 8 slots of 2048 experts took 15.1 us, 5.6 so).
+template <bool kOneWave>
 __global__ __launch_bounds__(kRouteSpread) void RouteSpread(const int32_t* __restrict__ ids, int ids_stride, Route r) {
   extern __shared__ int32_t counts[];
+  __shared__ int2 wave_sums[kOneWave ? 1 : kRouteSpread / kWave];
   const int slots = r.tokens * r.used;
   const int waves = (min(slots, kRouteSpread) + kWave - 1) / kWave;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
@@ -183,10 +188,11 @@ __global__ __launch_bounds__(kRouteSpread) void RouteSpread(const int32_t* __res
   auto id_at = [&](int i) { return ids[ids_stride == r.used ? i : static_cast<int64_t>(i / r.used) * ids_stride + i % r.used]; };
   const int e = mine < slots ? id_at(mine) : -1;
   const bool placed = e >= 0 && e < r.experts;
-  for (int i = tid; i < (waves + 2) * r.experts; i += kRouteSpread) counts[i] = 0;
+  const bool alone = !kOneWave && gridDim.x == 1;
+  for (int i = tid; i < (alone ? waves : waves + 2) * r.experts; i += kRouteSpread) counts[i] = 0;
   __syncthreads();
   // The other workgroups' slots, eight ids in flight a thread.
-  for (int i0 = tid; i0 < slots; i0 += 8 * kRouteSpread) {
+  for (int i0 = alone ? slots : tid; i0 < slots; i0 += 8 * kRouteSpread) {
     int id[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) id[u] = id_at(min(i0 + u * kRouteSpread, slots - 1));
@@ -206,19 +212,15 @@ __global__ __launch_bounds__(kRouteSpread) void RouteSpread(const int32_t* __res
   const int rank = __popcll(same & ((1ull << lane) - 1ull));
   if (placed && rank == 0) counts[wave * r.experts + e] = __popcll(same);
   __syncthreads();
-  // The experts' totals into offsets: each lane of the first wave a run of consecutive experts, the runs' sums scanned
-  // across the wave.
-  if (wave == 0) {
-    const int per = (r.experts + kWave - 1) / kWave;
-    const int e0 = min(lane * per, r.experts), e1 = min(e0 + per, r.experts);
-    auto total_of = [&](int at) {
-      int total = before[at] + after[at];
-      for (int w = 0; w < waves; ++w) total += counts[w * r.experts + at];
-      return total;
-    };
+  // The experts' totals into offsets: a thread a run of consecutive experts, the runs' sums scanned across the wave.
+  if (!kOneWave || wave == 0) {
+    constexpr int kScanners = kOneWave ? kWave : kRouteSpread;
+    const int per = (r.experts + kScanners - 1) / kScanners;
+    const int e0 = min(tid * per, r.experts), e1 = min(e0 + per, r.experts);
     int rows = 0, scale_rows = 0;
     for (int at = e0; at < e1; ++at) {
-      const int total = total_of(at);
+      int total = alone ? 0 : before[at] + after[at];
+      for (int w = 0; w < waves; ++w) total += counts[w * r.experts + at];
       offsets[at + 1] = total;  // for now
       rows += total;
       scale_rows += (total + kScaleRows - 1) / kScaleRows * kScaleRows;
@@ -231,8 +233,17 @@ __global__ __launch_bounds__(kRouteSpread) void RouteSpread(const int32_t* __res
       if (lane >= step) rows_before += a, scale_before += b;
     }
     int offset = rows_before - rows, scale_row = scale_before - scale_rows;
+    if constexpr (!kOneWave) {
+      if (lane == kWave - 1) wave_sums[wave] = make_int2(rows_before, scale_before);
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kRouteSpread / kWave - 1; ++w) {
+        const int2 sum = wave_sums[w];
+        if (w < wave) offset += sum.x, scale_row += sum.y;
+      }
+    }
     const bool writes = blockIdx.x == 0;
-    if (lane == 0) {
+    if (tid == 0) {
       offsets[0] = 0;
       if (writes) r.offsets[0] = 0, r.scale_rows[0] = 0;
     }
@@ -250,7 +261,7 @@ __global__ __launch_bounds__(kRouteSpread) void RouteSpread(const int32_t* __res
     r.position[mine] = -1;
     return;
   }
-  int row = offsets[e] + before[e] + rank;
+  int row = offsets[e] + (alone ? 0 : before[e]) + rank;
   for (int w = 0; w < wave; ++w) row += counts[w * r.experts + e];
   r.position[mine] = row;
   r.token[row] = mine / r.used;
@@ -384,10 +395,13 @@ extern "C" int llmp_hip_moe_route(const int32_t* ids, int ids_stride, int expert
   // would no longer be little beside the launches.
   const int64_t bytes = RouteSpreadInts(slots, experts) * static_cast<int64_t>(sizeof(int32_t));
   if (slots <= kRouteSpreadSlots && bytes <= kRouteSpreadLds) {
-    static bool sized = false;  // more than 64 KB of dynamic LDS must be asked for once
-    if (!AllowLds(reinterpret_cast<const void*>(&RouteSpread), kRouteSpreadLds, &sized)) return LaunchStatus("moe.route");
-    hipLaunchKernelGGL(RouteSpread, dim3(static_cast<unsigned>((slots + kRouteSpread - 1) / kRouteSpread)), dim3(kRouteSpread),
-                       static_cast<size_t>(bytes), s, ids, ids_stride, r);
+    const auto launch = [&](auto kernel, bool* sized) {  // (more than 64 KB of dynamic LDS must be asked for once a kernel)
+      if (!AllowLds(reinterpret_cast<const void*>(kernel), kRouteSpreadLds, sized)) return;
+      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((slots + kRouteSpread - 1) / kRouteSpread)), dim3(kRouteSpread),
+                         static_cast<size_t>(bytes), s, ids, ids_stride, r);
+    };
+    static bool sized[2] = {false, false};
+    experts <= 2 * kWave ? launch(&RouteSpread<true>, &sized[0]) : launch(&RouteSpread<false>, &sized[1]);
     return LaunchStatus("moe.route");
   }
   const int threads = experts < 256 ? (experts + 63) / 64 * 64 : 256;
