@@ -137,6 +137,16 @@ __global__ __launch_bounds__(kStoreThreads) void SetRowsQuantGroupKernel(const S
 // the frequency factor, YaRN's ramp mixes the interpolated (freq_scale) and the extrapolated angle between the
 // correction dims and raises the magnitude; channels from n_dims on pass through.
 // A workgroup a token: the token's n_dims / 2 cosines and sines once, in LDS, for every head's blocks.
+//
+// When a block's values and their partners are asked for is a matter of registers (119 ahead of the angles, 103 together, 71
+// in turn) against trips to memory, us in turn / together / ahead:
+//   a token of 8 heads of 128 values    5.53 / 5.75 / 5.30    behind the barrier they are a second trip;
+//   2048 of 2 heads of 256              7.51 / 8.77 / 8.31    what counts is how many workgroups a compute unit holds;
+//   4096 of 32 heads of 128             26.8 / 24.3 / 24.2    bytes: the longer the trip, the more must be on their way;
+//   4096 of 64 heads of 256             113 / 90 / -          (ahead is a thread's only block).
+// So ahead below four workgroups a compute unit and up to half a block a thread, and then together from more than a quarter.
+enum RopeLoads { kInTurn, kTogether, kAhead };
+template <RopeLoads LOADS>
 __global__ __launch_bounds__(kStoreThreads) void RopeSetRowsQuantKernel(const llmp_rope_store s) {
   extern __shared__ float2 rotation[];  // of pair p: magnitude * (cos, sin)
   const int64_t token = blockIdx.x;
@@ -144,24 +154,28 @@ __global__ __launch_bounds__(kStoreThreads) void RopeSetRowsQuantKernel(const ll
   const int blocks_head = s.head_dim / 32, blocks_row = s.heads * blocks_head;
   const bool wide = half % 32 == 0 && s.x_head_stride % 4 == 0 && s.x_token_stride % 4 == 0 &&
                     reinterpret_cast<uintptr_t>(s.x) % 16 == 0;
-  // The first block's values and their partners are asked for ahead of the angles: behind the barrier they were a second
-  // trip to memory (a token of 8 heads of 256 values 4.14 -> 3.80 us, 64 tokens 4.30 -> 4.02).
   float4 own[8], other[8];
-  auto load = [&](int block) {
+  auto values_of = [&](int head) { return s.x + head * s.x_head_stride + token * s.x_token_stride; };
+  auto load_own = [&](int block) {
     const int head = block / blocks_head, first = (block - head * blocks_head) * 32;
-    const float* x = s.x + head * s.x_head_stride + token * s.x_token_stride;
-    const float4* at = reinterpret_cast<const float4*>(x + first);
+    const float4* at = reinterpret_cast<const float4*>(values_of(head) + first);
 #pragma unroll
     for (int i = 0; i < 8; ++i) own[i] = at[i];
+  };
+  auto load_partners = [&](int block) {
+    const int head = block / blocks_head, first = (block - head * blocks_head) * 32;
     if (first < s.n_dims) {
-      const float4* partners = reinterpret_cast<const float4*>(x + (first < half ? first + half : first - half));
+      const float4* partners = reinterpret_cast<const float4*>(values_of(head) + (first < half ? first + half : first - half));
 #pragma unroll
       for (int i = 0; i < 8; ++i) other[i] = partners[i];
     }
   };
   const float position = static_cast<float>(s.pos[token]);
   const int64_t row = s.ids[token];
-  if (wide && static_cast<int>(threadIdx.x) < blocks_row) load(threadIdx.x);
+  if (LOADS == kAhead && wide && static_cast<int>(threadIdx.x) < blocks_row) {
+    load_own(threadIdx.x);
+    load_partners(threadIdx.x);
+  }
   float magnitude = s.attn_factor;
   if (s.ext_factor != 0.0f) magnitude *= 1.0f + 0.1f * logf(1.0f / s.freq_scale);
   for (int pair = threadIdx.x; pair < half; pair += kStoreThreads) {
@@ -176,22 +190,23 @@ __global__ __launch_bounds__(kStoreThreads) void RopeSetRowsQuantKernel(const ll
     }
     rotation[pair] = make_float2(cosf(theta) * magnitude, sinf(theta) * magnitude);
   }
-  __syncthreads();  // every thread: the loop below has no barrier
+  __syncthreads();  // every thread: what follows has no barrier
   uint8_t* to = static_cast<uint8_t*>(s.destination) + row * s.row_bytes;
-  for (int block = threadIdx.x; block < blocks_row; block += kStoreThreads) {
+  auto store = [&](int block) {
     const int head = block / blocks_head;
     const int first = (block - head * blocks_head) * 32;  // channel within the head
-    const float* x = s.x + head * s.x_head_stride + token * s.x_token_stride;
     float v[32];
     if (wide) {
       // The block lies within one half of the rotated channels (or past them): its 32 values and their partners'
       // as 16-byte loads.
-      if (block != static_cast<int>(threadIdx.x)) load(block);
+      if (LOADS != kAhead) load_own(block);
+      if (LOADS == kTogether) load_partners(block);
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[4 * i] = own[i].x, v[4 * i + 1] = own[i].y, v[4 * i + 2] = own[i].z, v[4 * i + 3] = own[i].w;
       if (first < s.n_dims) {
         const bool lower = first < half;
         const int pair0 = lower ? first : first - half;
+        if (LOADS == kInTurn) load_partners(block);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const float4 f = other[i];
@@ -205,6 +220,7 @@ __global__ __launch_bounds__(kStoreThreads) void RopeSetRowsQuantKernel(const ll
         }
       }
     } else {
+      const float* x = values_of(head);
 #pragma unroll 8
       for (int j = 0; j < 32; ++j) {
         const int channel = first + j;
@@ -223,6 +239,11 @@ __global__ __launch_bounds__(kStoreThreads) void RopeSetRowsQuantKernel(const ll
     } else {
       StoreQ4_0(v, to + block * 18);
     }
+  };
+  if constexpr (LOADS == kAhead) {
+    if (static_cast<int>(threadIdx.x) < blocks_row) store(threadIdx.x);
+  } else {
+    for (int block = threadIdx.x; block < blocks_row; block += kStoreThreads) store(block);
   }
 }
 
@@ -338,7 +359,10 @@ extern "C" int llmp_hip_rope_set_rows_quant(const llmp_rope_store* store, void* 
   const int64_t total = s.tokens * blocks_row;
   if (total > 0xFFFFFFFFll / 32) return Refuse(1, "%s: more than 2^32 - 1 values", op);
   if (s.tokens > 0x7FFFFFFFll || s.n_dims > 8192) return Refuse(1, "%s: more than 2^31 - 1 tokens or 8192 rotated dims", op);
-  hipLaunchKernelGGL(RopeSetRowsQuantKernel, dim3(static_cast<unsigned>(s.tokens)), dim3(kStoreThreads),
+  auto* kernel = s.tokens < 1024 && blocks_row <= kStoreThreads / 2 ? &RopeSetRowsQuantKernel<kAhead>
+                 : blocks_row > kStoreThreads / 4                     ? &RopeSetRowsQuantKernel<kTogether>
+                                                                      : &RopeSetRowsQuantKernel<kInTurn>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(s.tokens)), dim3(kStoreThreads),
                      static_cast<size_t>(s.n_dims / 2) * sizeof(float2), static_cast<hipStream_t>(stream), s);
   return LaunchStatus(op);
 }

@@ -158,6 +158,25 @@ def test_rope_then_store_matches_the_oracles_rotation_and_quantizer(device, t, y
         assert np.array_equal(stored[0], plain[0])
 
 
+@pytest.mark.parametrize("t", [ops.TYPE_Q8_0, ops.TYPE_Q4_0])
+@pytest.mark.parametrize("tokens,heads,head_dim", [(1030, 2, 256), (1030, 9, 256), (1030, 20, 128), (5, 34, 128), (3, 33, 256)])
+def test_a_tokens_stored_bytes_are_the_same_whatever_the_launch(device, t, tokens, heads, head_dim):
+    """A token's values are asked for ahead of the angles, together behind them, or in turn, by the launch's tokens and the
+    blocks of a row: the same bytes as from a launch of one token and one head (ahead)."""
+    n_dims, theta_scale = head_dim - 64, 0.93
+    x = dev(synth.activations(tokens, heads * head_dim, 97).reshape(tokens, heads, head_dim), device)
+    pos = torch.arange(7, 7 + tokens, dtype=torch.int32, device=device)
+    ids = torch.arange(tokens, dtype=torch.int64, device=device)
+    head_bytes = head_dim // 32 * ops.BLOCK_BYTES[t]
+    cache = torch.zeros((tokens, heads * head_bytes), dtype=torch.uint8, device=device)
+    ops.rope_set_rows_quant(t, x, pos, ids, cache, n_dims, theta_scale)
+    alone = torch.zeros((1, head_bytes), dtype=torch.uint8, device=device)
+    for token in sorted({0, 1, tokens // 2, tokens - 1}):
+        for head in sorted({0, heads // 2, heads - 1}):
+            ops.rope_set_rows_quant(t, x[token:token + 1, head:head + 1].contiguous(), pos[token:token + 1], ids[:1], alone, n_dims, theta_scale)
+            assert torch.equal(alone[0], cache[token, head * head_bytes:(head + 1) * head_bytes]), (token, head)
+
+
 def test_rope_store_refusals(device):
     x = torch.zeros((2, 2, 64), dtype=torch.float32, device=device)
     pos = torch.zeros(2, dtype=torch.int32, device=device)
