@@ -195,6 +195,10 @@ def test_linear_of_more_than_sixteen_rows_runs_in_passes(device, m):
     (81, 1024, 256, 4, ops.EXL3_MUL1), (144, 1152, 128, 5, ops.EXL3_MCG),
     (81, 1024, 256, 6, ops.EXL3_3INST),    # two passes above five bits
     (145, 512, 256, 4, ops.EXL3_3INST),    # two passes, the second short of its tiles
+    # 33 to 80 rows, more workgroups' worth of column blocks than compute units: several a workgroup, in even shares and
+    # (226 blocks of four slices, 260 and 258 of one) in ragged ones; one and nine 128 blocks of K, waves without any.
+    (77, 4096, 14336, 4, ops.EXL3_3INST), (48, 4096, 14464, 2, ops.EXL3_MCG), (80, 1152, 16640, 3, ops.EXL3_MUL1),
+    (33, 128, 16512, 1, ops.EXL3_3INST), (65, 128, 33024, 4, ops.EXL3_MCG),
     (290, 256, 128, 8, ops.EXL3_MUL1)])
 def test_wide_passes_are_the_sixteen_row_passes_bit_for_bit(device, m, k, n, bits, codebook):
     """Passes of up to 144 rows (the scratch's wide size) against the linear's passes of sixteen (its least size)."""
