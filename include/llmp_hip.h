@@ -94,6 +94,9 @@ typedef struct llmp_vecq_desc {
 int llmp_hip_vecq(int type, const llmp_vecq_desc* d, int variant, void* stream);
 int llmp_hip_vecq_variants(void);
 const char* llmp_hip_vecq_variant_name(int variant);
+/* The form that llmp_hip_vecq takes for a product by default: a variant's name, or "tiles of sixteen rows" (Q4_K at 9 to 16
+ * tokens), which has no number. Null where the product is refused. */
+const char* llmp_hip_vecq_default_name(int type, const llmp_vecq_desc* d);
 
 /* An import-time relayout for this device, lossless and undone by inverse != 0 (the reference does its
  * platform-specific relayouts at import, src/import/expert_relayout.h:4-17: a table rewritten into the tile order

@@ -576,7 +576,8 @@ int DefaultVariant(int type, const llmp_vecq_desc& d, int kp, bool fused) {
   // mostly name different experts, one or two tokens each: the flat form.
   // Q4_K, 2 to 8 tokens: a weight row a lane on the 4 x 4 x 4 instruction (at 3840 x 2 x 15360 with a GLU 17.8 us
   // at two and at four tokens, 21.3 at eight, against the 16 x 16 form's 25 at any count and the flat form's
-  // four-token passes' 18 / 25 / 43). More tokens, and rows that form does not take: the 16 x 16 form, whose time
+  // four-token passes' 18 / 25 / 43). Nine to sixteen have a form of their own (Tile16Pays); what comes here beyond eight are
+  // the shapes it refuses. Rows that the row-a-lane form does not take: the 16 x 16 form, whose time
   // hardly depends on the tokens; the flat form's four-token pass stays under it up to five tokens for Q8_0
   // (15 / 17 / 20 / 27 us against 29 at 4096 x 14336).
   // The row-a-lane form's time hardly depends on the tokens. Its tiles are 64 rows a workgroup of four waves, or 32 or
@@ -584,13 +585,14 @@ int DefaultVariant(int type, const llmp_vecq_desc& d, int kp, bool fused) {
   // 12.8 / 12.6 / 19 us at two, four and eight tokens in tiles of 16 against 24.8 / 24.5 / 34 in tiles of 64 and the
   // flat form's four-token passes' 13.7 / 25 / 44; 4096 x 4096: 7.0 / 7.1 / 8.0 against 10.5 / 10.5 / 12.4 and
   // 7.0 / 9.0 / 14.5). At two tokens the four-token pass is as fast, here a tenth faster (5120 x 5120: 8.0 against
-  // 9.2 us) and there a tenth slower; the row-a-lane form from two tokens keeps a token's bits the same at every count.
+  // 9.2 us) and there a tenth slower; the row-a-lane form from two tokens keeps a token's bits the same from two to eight
+  // (of Q8_0 rows too long for the 16 x 16 form, to sixteen).
   // Q8_0: the same (4096 x 14336: 16.2-17.4 us at 2 to 8 tokens against 19 / 22 / 31 for the four-token passes and
   // the 16 x 16 form; 14336 x 4096 in tiles of 16 rows: 17 us at 2 to 4 tokens and 22 at 5 to 8 against 26 / 35 / 44
   // / 54-82).
   if (tokens > 1 && !fused && (type == LLMP_TYPE_Q4_K || type == LLMP_TYPE_Q8_0) && RowsTakes(type, d)) {
-    // (More than eight tokens are launches of eight: for rows too long for the 16 x 16 form. Q4_K 15360 x 3840 at
-    // sixteen tokens: 2 x 19 us against the four-token passes' 82.)
+    // (More than eight tokens are launches of eight: for rows too long for the 16 x 16 form, Q8_0's and the Q4_K shapes
+    // that Tile16Pays' form refuses. Q4_K 15360 x 3840 at sixteen tokens: 2 x 19 us against the four-token passes' 82.)
     if (tokens <= 8 || !MmaTakes(type, d)) return kRowsVariant;
   }
   // (A plain Q4_K product of few rows: the four-token pass up to four tokens, 9.0 us against the 16 x 16 form's 13.1
@@ -613,13 +615,14 @@ int DefaultVariant(int type, const llmp_vecq_desc& d, int kp, bool fused) {
   }
 }
 
-// Whether a super-block of 16 rows a wave (vecq_tile16.hip) is the default: nine to sixteen tokens, the faster everywhere it
-// was measured (fourteen shapes from 1024 -> 512 to 15360 -> 8192: 1.1 to 2.1 times the 16 x 16 form and the two launches of
-// the row-a-lane form). Up to eight the row-a-lane form, whose bits a token keeps from two to eight: at eight this one is
-// the faster for rows of more than 8192 values (9216 -> 2048 10.6 against 17.6 us), at four mostly not (15360 -> 3840 13.4
-// against 11.4).
+// Whether a super-block of 16 rows a wave (vecq_tile16.hip) is the default: nine to sixteen tokens, never the slower of it and
+// what was the default, the 16 x 16 form and the two launches of the row-a-lane form (31 shapes from 256 -> 512 to 28672 ->
+// 8192 at 9, 12 and 16 tokens: 0.21 to 1.00 of their time). Up to eight the row-a-lane form, whose bits a token keeps from two
+// to eight (beyond, it has this form's, where rows too long for the 16 x 16 form had one form's from two to sixteen): at eight
+// this one is the faster for rows of more than 8192 values (9216 -> 2048 10.6 against 17.6 us), at four mostly not (15360 ->
+// 3840 13.4 against 11.4).
 bool Tile16Pays(int type, const llmp_vecq_desc& d) {
-  return type == LLMP_TYPE_Q4_K && d.ids == nullptr && d.tokens > 8 && d.tokens <= 16;
+  return type == LLMP_TYPE_Q4_K && d.ids == nullptr && d.tokens > 8 && d.tokens <= 16 && Tile16Takes(d);
 }
 
 int CheckDesc(int type, const llmp_vecq_desc* d, bool sorted = false) {
@@ -684,8 +687,10 @@ int Launch(int type, const llmp_vecq_desc* d, const llmp_vecq_source* x, int var
   a.dump = dump;
   a.offsets = offsets;
   a.rows = rows;
-  if (variant < 0 && x == nullptr && dump == nullptr && Tile16Pays(type, *d) && LaunchTile16(a, static_cast<hipStream_t>(stream)))
+  if (variant < 0 && x == nullptr && dump == nullptr && Tile16Pays(type, *d)) {  // (sorted rows have one token)
+    LaunchTile16(a, static_cast<hipStream_t>(stream));
     return LaunchStatus("vecq");
+  }
   if (variant < 0) variant = DefaultVariant(type, *d, a.kp, x != nullptr);
   if (variant >= kVariantCount) return Refuse(1, "vecq: no variant %d", variant);
   const Variant& v = kVariants[variant];
@@ -840,4 +845,10 @@ extern "C" int llmp_hip_vecq_variants(void) { return kVariantCount; }
 
 extern "C" const char* llmp_hip_vecq_variant_name(int variant) {
   return variant >= 0 && variant < kVariantCount ? kVariants[variant].name : "default";
+}
+
+extern "C" const char* llmp_hip_vecq_default_name(int type, const llmp_vecq_desc* d) {
+  if (CheckDesc(type, d) != 0) return nullptr;
+  if (Tile16Pays(type, *d)) return "tiles of sixteen rows";
+  return kVariants[DefaultVariant(type, *d, PaddedK(d->ncols_x), false)].name;
 }

@@ -242,8 +242,9 @@ bool SortedTakes(int type, const llmp_vecq_desc& d);
 void LaunchSorted(const VecQArgs& a, int workgroups, hipStream_t stream);
 
 // Q4_K, 9 to 16 tokens of a dense or grouped product over Q8_1 activations, a super-block of 16 rows a wave
-// (vecq_tile16.hip). False: nothing was queued, the shape is not this form's.
-bool LaunchTile16(const VecQArgs& a, hipStream_t stream);
+// (vecq_tile16.hip).
+bool Tile16Takes(const llmp_vecq_desc& d);  // by the shape alone
+void LaunchTile16(const VecQArgs& a, hipStream_t stream);
 
 // The row-a-lane kernel for 2 to 8 tokens of a dense or grouped Q4_K product over Q8_1 activations (vecq_rows.hip).
 constexpr int kRowsTokensMost = 16;  // of the row-a-lane form (the operation's most): eight a launch

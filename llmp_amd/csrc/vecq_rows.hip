@@ -857,8 +857,8 @@ void LaunchRows(const VecQArgs& whole, hipStream_t stream) {
   }
   if (a.parts == 0) a.parts = RowsParts(a, g_rows_compute_units);
   if (d.tokens > 8) {
-    // Equal shares of eight tokens or fewer, a launch each (the weights read once a launch): for rows too long for the
-    // 16 x 16 form, whose other choice is a pass for every four tokens.
+    // Equal shares of eight tokens or fewer, a launch each (the weights read once a launch): for Q8_0 rows too long for the
+    // 16 x 16 form, whose other choice is a pass for every four tokens, and the Q4_K shapes that vecq_tile16.hip refuses too.
     const int launches = (d.tokens + 7) / 8, share = (d.tokens + launches - 1) / launches;
     for (int first = 0; first < d.tokens; first += share) {
       VecQArgs some = a;

@@ -16,8 +16,8 @@
 //
 // What bounds it is the vector unit and the loads' issue: with the weights in the Infinity Cache the gate/up pair below
 // takes two microseconds less. HBM traffic is 1.01 of the weights. Measured, 9 and 16 tokens, against what was the default:
-// 3840 -> 2 x 15360 with GeGLU 26.0 / 26.5 -> 21.5 / 22.9 us, 15360 -> 3840 28.4 / 35.2 -> 17.0 / 22.6, 4096 -> 4096
-// 15.4 / 15.7 -> 8.0 / 9.4, 2048 -> 2 x 8192 22.2 / 22.0 -> 9.5 / 10.6, 1024 -> 4096 8.8 / 9.0 -> 5.3 / 5.5. Error against
+// 3840 -> 2 x 15360 with GeGLU 27.2 / 28.1 -> 22.3 / 23.2 us, 15360 -> 3840 28.5 / 35.2 -> 16.8 / 22.1, 4096 -> 4096
+// 15.4 / 15.9 -> 8.2 / 9.6, 2048 -> 2 x 8192 22.8 / 22.7 -> 10.1 / 10.4, 1024 -> 4096 8.4 / 8.6 -> 5.4 / 5.5. Error against
 // F64 1.2e-7 (1.4e-7 in the row-a-lane form, 2.4e-7 in the 16 x 16 form).
 // Measured and not kept: up to eight tokens with a pair of sub-blocks in one v_mfma_i32_16x16x64_i8, a token's first and
 // second sub-blocks in rows 0 to 7 and 8 to 15 (134 vector instructions; 15360 -> 3840 at 6 tokens 18.3 -> 14.3 us, but at 4
@@ -256,7 +256,13 @@ __global__ __launch_bounds__(kGroup, 1) void VecQTile16(const VecQArgs a, const 
   }
 }
 
-int g_tile16_compute_units = 0;
+int ComputeUnits() {
+  static const int units = [] {
+    const int cus = llmp_hip_compute_units();
+    return cus > 0 ? cus : 256;
+  }();
+  return units;
+}
 
 // The super-blocks whose tokens fit LDS beside the sums.
 int64_t Room(int tokens, int parts) { return (kLdsMost - parts * kPartBytes) / StagedBytes(tokens); }
@@ -299,18 +305,19 @@ void LaunchOne(const VecQArgs& a, const Tile16Plan& plan, dim3 grid, hipStream_t
 
 }  // namespace
 
-bool LaunchTile16(const VecQArgs& a, hipStream_t stream) {
-  const llmp_vecq_desc& d = a.d;
-  if (g_tile16_compute_units == 0) {
-    const int cus = llmp_hip_compute_units();
-    g_tile16_compute_units = cus > 0 ? cus : 256;
-  }
+bool Tile16Takes(const llmp_vecq_desc& d) {
   Tile16Plan plan;
   int workgroups;
-  if (!PlanTile16(d, g_tile16_compute_units, &plan, &workgroups)) return false;
+  return PlanTile16(d, ComputeUnits(), &plan, &workgroups);
+}
+
+void LaunchTile16(const VecQArgs& a, hipStream_t stream) {
+  const llmp_vecq_desc& d = a.d;
+  Tile16Plan plan;
+  int workgroups;
+  if (!PlanTile16(d, ComputeUnits(), &plan, &workgroups)) return;
   const dim3 grid(static_cast<unsigned>(workgroups), static_cast<unsigned>(d.used));
   d.g != nullptr ? LaunchOne<true>(a, plan, grid, stream) : LaunchOne<false>(a, plan, grid, stream);
-  return true;
 }
 
 }  // namespace llmp_hip

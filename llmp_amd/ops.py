@@ -127,6 +127,14 @@ def vecq_variants():
     return [lib.llmp_hip_vecq_variant_name(i).decode() for i in range(lib.llmp_hip_vecq_variants())]
 
 
+def vecq_default_name(t, w, k, nrows, *, gate=None, ids=None, tokens=1, used=1, stride_row=None, stride_expert=0, glu=GLU_NONE):
+    """The form that vecq takes for a product by default: a variant's name or "tiles of sixteen rows"."""
+    d = _desc(t, w, k, nrows, gate=gate, q8=None, ids=ids, tokens=tokens, used=used, stride_row=stride_row,
+              stride_expert=stride_expert, y_token=None, y_slot=0, glu=glu, limit=0.0, out=w)
+    name = _lib.load().llmp_hip_vecq_default_name(t, C.byref(d))
+    return None if name is None else name.decode()
+
+
 def vecq_sorted(t, w, q8, offsets, k, nrows, experts, *, gate=None, stride_row=None, stride_expert=0,
                 glu=GLU_NONE, limit=0.0, variant=-1, out=None, rows=None):
     """llmp.vecq over rows sorted by expert: q8 [rows, blocks*36] -> float32 [rows, nrows]. `rows` (int32): sorted row r's

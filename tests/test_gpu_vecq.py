@@ -1,6 +1,8 @@
 """Parity of llmp.q8_1 and llmp.vecq (HIP, through the C ABI) against the CPU oracle on
 the same seeded inputs. Integer work is compared bit for bit; float outputs to a maximum
 relative error of 1e-3 (the accumulation order is the only difference)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -338,6 +340,198 @@ def test_q4k_tiles_of_sixteen_rows(device, k, n, tokens, glu, used):
     fewest = 9
     fewer = ops.vecq(Q4_K, dev(up, device), dev(q8, device), k, n, gate=gd, tokens=fewest, **common).cpu().numpy()
     assert np.array_equal(fewer.view(np.uint32), got[:fewest].view(np.uint32))
+
+
+def same_bits(a, b):
+    return bool((a.contiguous().view(torch.int32) == b.contiguous().view(torch.int32)).all())
+
+
+@pytest.mark.parametrize("k,n,tokens,glu,used,kind", [(512, 40, 9, False, 1, "sixteen"), (4352, 33, 16, True, 2, "sixteen"),
+                                                      (9216, 48, 12, False, 1, "sixteen"), (5888, 32768, 9, False, 1, "sixteen"),
+                                                      (5888, 32784, 9, False, 1, "mma pass16"), (8704, 32784, 10, False, 1, "rows pass8")])
+def test_q4k_form_of_nine_to_sixteen_tokens(device, k, n, tokens, glu, used, kind):
+    """Which form runs by default, at both sides of the shapes that the form of sixteen rows refuses (rows of more than 22
+    super-blocks and more rows than the device takes in one go), where the product is the other form's bit for bit; and that
+    rows apart, fewer rows than the matrix holds, an output that no vector store fits with room between its rows, and permuted
+    tokens change no bit of a value nor anything beside the output."""
+    blocks = k // 256
+    g = torch.Generator(device=device).manual_seed(k + n)
+    rows = used * n * (2 if glu else 1)
+    w = torch.randint(0, 256, (rows, blocks, 144), dtype=torch.uint8, device=device, generator=g)
+    w[:, :, 0:4] = torch.tensor([0, 0x14, 0, 0x1A], dtype=torch.uint8, device=device)  # d, dmin
+    up, gate = (w[:rows // 2], w[rows // 2:]) if glu else (w, None)
+    x = synth.activations(tokens * used, k, 98)
+    q8 = ops.quantize_q8_1(dev(x, device))
+    y_row = ops.padded_k(k) // 32
+    common = dict(used=used, glu=ops.GLU_GEGLU if glu else ops.GLU_NONE)
+    name = ops.vecq_default_name(Q4_K, up, k, n, gate=gate, tokens=tokens, stride_expert=n * blocks, **common)
+    assert name == ("tiles of sixteen rows" if kind == "sixteen" else kind)
+    common.update(tokens=tokens, y_token=y_row * used, y_slot=y_row)
+    want = ops.vecq(Q4_K, up, q8, k, n, gate=gate, stride_expert=n * blocks, **common)
+    if kind != "sixteen":
+        other = ops.vecq(Q4_K, up, q8, k, n, variant=ops.vecq_variants().index(kind), **common)
+        assert same_bits(other, want)
+        return
+    order = torch.from_numpy(synth.rng(99).permutation(tokens)).to(device)
+    mixed = q8.view(tokens, used, -1)[order].contiguous()
+    got = ops.vecq(Q4_K, up, mixed, k, n, gate=gate, stride_expert=n * blocks, **common)
+    assert same_bits(got, want[order])
+    if n > 1000:
+        return
+    apart = torch.full((rows, blocks + 3, 144), 0xFF, dtype=torch.uint8, device=device)  # NaNs between the rows
+    apart[:, :blocks] = w
+    fewer, pitch = n - 5, n + 3
+    buffer = torch.full((1 + tokens * used * pitch,), 7.0, dtype=torch.float32, device=device)
+    up2, gate2 = (apart[:rows // 2], apart[rows // 2:]) if glu else (apart, None)
+    d = ops._desc(Q4_K, up2, k, fewer, gate=gate2, q8=q8, ids=None, stride_row=blocks + 3, stride_expert=n * (blocks + 3), limit=0.0,
+                  out=buffer[1:], **common)
+    d.dst_token, d.dst_slot = used * pitch, pitch
+    ops._lib.check(ops._lib.load().llmp_hip_vecq(Q4_K, C.byref(d), -1, ops._stream()))
+    got = buffer[1:].view(tokens, used, pitch)
+    assert same_bits(got[:, :, :fewer], want[:, :, :fewer])
+    assert buffer[0] == 7.0 and bool((got[:, :, fewer:] == 7.0).all())
+
+
+def integer_blocks(n, k, tokens, seed, minimums):
+    """Q4_K rows and Q8_1 tokens whose products are integers: d = 1, every code, scale and (with `minimums`, dmin = 1, else 0)
+    minimum in use, unit block scales. -> blocks, Q8_1 rows, the products and the sums of their terms' magnitudes."""
+    g = synth.rng(seed)
+    nsb = k // 256
+    sc, mn = g.integers(0, 64, size=(2, n, nsb, 8), dtype=np.int64)
+    q = g.integers(0, 16, size=(n, nsb, 8, 32), dtype=np.int64)
+    codes = g.integers(-127, 128, size=(tokens, nsb, 8, 32), dtype=np.int64)
+    mn *= int(minimums)
+    sums, totals = np.einsum("rbgk,tbgk->trbg", q, codes), codes.sum(axis=3)
+    main, low = sums * sc[None], totals[:, None] * mn[None]
+    return (q4k_bytes(q, sc, mn, 1.0, float(minimums)), q8_1_bytes(codes, np.ones((tokens, nsb, 8), dtype=np.float16)),
+            (main - low).sum(axis=(2, 3)), (np.abs(main) + np.abs(low)).sum(axis=(2, 3)))
+
+
+def q4k_bytes(q, sc, mn, d, dmin):
+    n, nsb = q.shape[:2]
+    w = np.zeros((n, nsb, 144), dtype=np.uint8)
+    w[:, :, 0:4] = np.frombuffer(np.array([d, dmin], dtype=np.float16).tobytes(), dtype=np.uint8)
+    w[:, :, 4:8] = sc[..., :4] | (sc[..., 4:] >> 4 << 6)
+    w[:, :, 8:12] = mn[..., :4] | (mn[..., 4:] >> 4 << 6)
+    w[:, :, 12:16] = (sc[..., 4:] & 15) | ((mn[..., 4:] & 15) << 4)
+    w[:, :, 16:] = (q[:, :, 0::2] | (q[:, :, 1::2] << 4)).reshape(n, nsb, 128)
+    return w
+
+
+def q8_1_bytes(codes, scales):
+    tokens, nsb = codes.shape[:2]
+    q8 = np.zeros((tokens, ops.padded_k(256 * nsb) // 32, 36), dtype=np.uint8)
+    q8[:, :8 * nsb, 0:2] = scales.reshape(tokens, 8 * nsb, 1).view(np.uint8).reshape(tokens, 8 * nsb, 2)
+    q8[:, :8 * nsb, 4:] = codes.astype(np.int8).view(np.uint8).reshape(tokens, 8 * nsb, 32)
+    return q8
+
+
+def default_forms(device, w, q8, k, n):
+    """The product by the two forms without a number, [tokens, n] each: dense, and as rows sorted by expert (every expert's
+    matrix the same; passes of one and of two token groups)."""
+    tokens = q8.shape[0]
+    wd, qd = dev(w.reshape(-1), device), dev(q8, device)
+    if tokens <= 16:
+        assert ops.vecq_default_name(Q4_K, wd, k, n, tokens=tokens) == "tiles of sixteen rows"
+        yield ops.vecq(Q4_K, wd, qd, k, n, tokens=tokens).cpu().numpy().reshape(tokens, n)
+    first = tokens // 3
+    offsets = dev(np.array([0, first, tokens], dtype=np.int32), device)
+    yield ops.vecq_sorted(Q4_K, wd, qd.view(tokens, -1), offsets, k, n, 2, stride_expert=0).cpu().numpy()
+
+
+@pytest.mark.parametrize("k,tokens,minimums", [(256, 9, True), (256, 60, True), (1024, 16, False), (1024, 99, True), (2048, 16, True), (2048, 60, False)])
+def test_default_forms_sums_are_exact_integers(device, k, tokens, minimums):
+    """Every scale, minimum, nibble and place: while the terms' magnitudes add to less than 2^24, F32 holds every partial sum
+    and the forms (one of them with F16 subnormals for operands and its result scaled back) must return the integer."""
+    n = 48
+    w, q8, want, magnitude = integer_blocks(n, k, tokens, 325 + k + tokens, minimums)
+    assert magnitude.max() < 2 ** 24
+    for got in default_forms(device, w, q8, k, n):
+        assert np.array_equal(got, want.astype(np.float32))
+
+
+@pytest.mark.parametrize("k,tokens", [(256, 16), (1024, 60), (2048, 16), (2048, 40)])
+def test_default_forms_minimums_are_exact_in_three_parts(device, k, tokens):
+    """One minimum of 1 a row, all scales 0: the value is -(d8 * sum of the codes) of that sub-block, 11 bits times 12, which
+    F32 holds, so the three bf16 parts it goes through must add to it without an error."""
+    n, nsb = 80, k // 256
+    g = synth.rng(326 + k)
+    codes = g.integers(-127, 128, size=(tokens, nsb, 8, 32), dtype=np.int64)
+    codes[::3] = np.abs(codes[::3])  # sums of twelve bits
+    scales = (g.integers(1024, 2048, size=(tokens, nsb, 8)) | 1).astype(np.float16) / np.float16(1024)
+    q = g.integers(0, 16, size=(n, nsb, 8, 32), dtype=np.int64)
+    mn = np.zeros((n, nsb * 8), dtype=np.int64)
+    at = np.arange(n) % (nsb * 8)
+    mn[np.arange(n), at] = 1
+    w = q4k_bytes(q, np.zeros((n, nsb, 8), dtype=np.int64), mn.reshape(n, nsb, 8), 1.0, 1.0)
+    want = -(scales.astype(np.float64) * codes.sum(axis=3)).reshape(tokens, nsb * 8)[:, at]
+    assert np.array_equal(want, want.astype(np.float32))
+    for got in default_forms(device, w, q8_1_bytes(codes, scales), k, n):
+        assert np.array_equal(got, want.astype(np.float32))
+
+
+@pytest.mark.parametrize("k,tokens", [(512, 13), (1024, 70), (2048, 16), (2048, 45)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_default_forms_keep_what_is_not_finite_to_its_values(device, k, tokens, bad):
+    """A token's block scale, a row's d and a row's dmin that are infinite or NaN: that token's and those rows' values are not
+    finite, every other value is the bits it is without them."""
+    n = 70
+    g = synth.rng(327 + k)
+    w = synth.q4_k_weights(n, k, 328).reshape(n, k // 256, 144).copy()
+    w[:, :, 4:16] |= 1  # no scale or minimum of 0 in the sub-blocks below
+    q8 = oracle.q8_1_quantize(synth.activations(tokens, k, 329)).reshape(tokens, -1, 36).copy()
+    clean = list(default_forms(device, w, q8, k, n))
+    half = np.frombuffer(np.float16(bad).tobytes(), dtype=np.uint8)
+    token, row_d, row_dmin = tokens - 2, 17, 64
+    q8[token, g.integers(0, k // 32), 0:2] = half
+    w[row_d, -1, 0:2] = half
+    w[row_dmin, 0, 2:4] = half
+    for got, before in zip(default_forms(device, w, q8, k, n), clean):
+        rest = np.ones_like(before, dtype=bool)
+        rest[token] = False
+        rest[:, [row_d, row_dmin]] = False
+        assert not np.isfinite(got[~rest]).any()
+        assert np.isfinite(before).all() and np.array_equal(got[rest].view(np.uint32), before[rest].view(np.uint32))
+
+
+@pytest.mark.parametrize("k", [512, 1024, 2048, 2304])
+@pytest.mark.parametrize("glu", [ops.GLU_NONE, ops.GLU_SWIGLU_CLAMP, ops.GLU_GEGLU])
+def test_sorted_q4k_rows_glus_and_pitches(device, k, glu):
+    """GeGLU and the clamped SwiGLU of sorted rows, weight rows and matrices apart, fewer rows than a matrix holds, and an output
+    that no vector store fits, with room between its rows that stays as it was: against the oracle within 1e-5 of the RMS, of the
+    clamped SwiGLU within what 1e-5 of the sums' RMS makes of it: silu(g) u, its slope at most 1.1, |u| and silu at most the limit
+    (silu of what is not clamped, the negative g, at most 0.28), so 1.1 limit + max(limit, 0.28) times the sums' error."""
+    counts = np.array([3, 0, 70, 1, 33], dtype=np.int32)
+    experts, rows, n, blocks = len(counts), int(counts.sum()), 90, k // 256
+    limit = 0.05 if glu == ops.GLU_SWIGLU_CLAMP else 0.0
+    up, gate = (make_weights(Q4_K, experts * n, k, seed).reshape(experts, n, blocks, 144) for seed in (101, 102))
+    q8 = oracle.q8_1_quantize(synth.activations(rows, k, 103)).reshape(rows, -1)
+    ids = np.repeat(np.arange(experts, dtype=np.int32), counts).reshape(-1, 1)
+    want = oracle.vecq(Q4_K, up.reshape(experts, -1), q8, k, n, gate=gate.reshape(experts, -1) if glu else None, ids=ids, tokens=rows, used=1,
+                       stride_expert=n * blocks, glu=glu, limit=limit, experts=experts, threads=oracle.max_threads()).reshape(rows, n)
+    bound = 1e-5 * np.sqrt(np.mean(want.astype(np.float64) ** 2))
+    if limit:
+        sums = [oracle.vecq(Q4_K, w.reshape(experts, -1), q8, k, n, ids=ids, tokens=rows, used=1, stride_expert=n * blocks, experts=experts,
+                            threads=oracle.max_threads()) for w in (up, gate)]
+        bound = 1e-5 * np.sqrt(np.mean(np.square(sums, dtype=np.float64))) * (1.1 * limit + max(limit, 0.28))
+
+    def apart(w):
+        out = torch.full((experts, n + 2, blocks + 1, 144), 0xFF, dtype=torch.uint8, device=device)  # NaNs between rows and matrices
+        out[:, :n, :blocks] = dev(w, device)
+        return out
+
+    upd, gated = apart(up), apart(gate) if glu else None
+    offsets = dev(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32), device)
+    fewer, pitch = n - 7, n + 6
+    for shift in (0, 1):  # at a boundary for vector stores, whose rows end within one, and not
+        buffer = torch.full((shift + rows * pitch,), 7.0, dtype=torch.float32, device=device)
+        d = ops._desc(Q4_K, upd, k, fewer, gate=gated, q8=dev(q8, device), ids=None, tokens=1, used=1, stride_row=blocks + 1,
+                      stride_expert=(n + 2) * (blocks + 1), y_token=None, y_slot=0, glu=glu, limit=limit, out=buffer[shift:])
+        d.dst_token = pitch
+        ops._lib.check(ops._lib.load().llmp_hip_vecq_sorted(Q4_K, C.byref(d), offsets.data_ptr(), experts, -1, ops._stream()))
+        got = buffer[shift:].view(rows, pitch).cpu().numpy()
+        assert (np.abs(got[:, :fewer] - want[:, :fewer]) <= np.maximum(bound, 1e-5 * np.abs(want[:, :fewer]))).all()
+        assert (got[:, fewer:] == 7.0).all() and (shift == 0 or float(buffer[0]) == 7.0)
 
 
 def same_sums(t, a, b):
