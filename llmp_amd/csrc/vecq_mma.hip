@@ -254,11 +254,12 @@ struct Segment {
   int expert, first, m, group_first, group_step, group_count;
 };
 
-// grid (workgroups, slots), or (workgroups) with `balanced` (sorted rows: the workgroups share the
-// passes of all experts evenly, whatever the experts' row counts); LDS: codes, d8, ds8, the waves'
-// partial sums.
-template <bool kGlu, int TG, int MT>
-__global__ __launch_bounds__(kMmaGroup, 1) void VecQMma(const VecQArgs a, int balanced) {
+// grid (workgroups, slots), or (workgroups) with kSorted (sorted rows of more than eight super-blocks, of which LDS holds
+// one token group: the workgroups share the passes of all experts evenly, whatever the experts' row counts); LDS: codes,
+// d8, ds8, the waves' partial sums.
+template <bool kGlu, int TG, int MT, bool kSorted>
+__global__ __launch_bounds__(kMmaGroup, 1) void VecQMma(const VecQArgs a) {
+  static_assert(!kSorted || TG == 1);
   using L = Staged<TG, MT>;
   constexpr int kDepth = TG == 1 ? 3 : TG == 2 ? 3 : 2;  // weight buffers: the fetches run kDepth - 1 steps ahead
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -294,7 +295,7 @@ __global__ __launch_bounds__(kMmaGroup, 1) void VecQMma(const VecQArgs a, int ba
   const uint8_t* my_ds8 = ds8 + token_in_group * 32 + kg * 8;
 
   int sorted_first = 0;
-  auto pair_at = [&](int i) { return a.offsets != nullptr ? (sorted_first + i) << 8 : pairs[i]; };
+  auto pair_at = [&](int i) { return kSorted ? (sorted_first + i) << 8 : pairs[i]; };
 
   bool staged_before = false;
   auto run = [&](const Segment& seg) {
@@ -457,30 +458,18 @@ __global__ __launch_bounds__(kMmaGroup, 1) void VecQMma(const VecQArgs a, int ba
     }
   };
 
-  if (balanced == 0) {
-    int expert = blockIdx.y;
-    if (a.offsets != nullptr) {
-      sorted_first = a.offsets[expert];
-      if (tid == 0) count = a.offsets[expert + 1] - sorted_first;
-      __syncthreads();
-    } else {
-      expert = ResolvePairs(d, blockIdx.y, pairs, &count);
-    }
+  if constexpr (kSorted) {
+    // Every pass has one token group, and its start costs little beside its tiles' long rows.
+    WalkSortedRows(a.offsets, d.used, groups, MT, [](int) { return 0; }, [](int) { return 1; }, [&](const SortedSegment& seg) {
+      sorted_first = seg.rows_first;
+      run(Segment{seg.expert, seg.first, seg.m, seg.group_first, 1, seg.group_count});
+    });
+  } else {
+    const int expert = ResolvePairs(d, blockIdx.y, pairs, &count);
     const int n = count;
     const int mine = (groups - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
     for (int p0 = 0; p0 < n; p0 += TG * MT)
       run(Segment{expert, p0, min(TG * MT, n - p0), static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), mine});
-  } else {
-    // A step's instructions: about 12 parts for the weights and 7 a live token group.
-    auto cost_of = [](int m) {
-      const int token_groups = (m + MT - 1) / MT;
-      const int live = token_groups <= 1 ? 1 : token_groups <= 2 ? 2 : 4;
-      return 12 + 7 * min(live, TG);
-    };
-    WalkSortedRows(a.offsets, d.used, groups, TG * MT, [](int) { return 0; }, cost_of, [&](const SortedSegment& seg) {
-      sorted_first = seg.rows_first;
-      run(Segment{seg.expert, seg.first, seg.m, seg.group_first, 1, seg.group_count});
-    });
   }
 }
 
@@ -863,22 +852,24 @@ void LaunchMmaQ8(const VecQArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
   hipLaunchKernelGGL((VecQMmaQ8<kGlu>), grid, dim3(kMmaGroup), lds, stream, a);
 }
 
-template <bool kGlu, int TG, int MT>
-void LaunchMmaQ4K(const VecQArgs& a, dim3 grid, size_t lds, int balanced, hipStream_t stream) {
+template <bool kGlu, int TG, int MT, bool kSorted>
+void LaunchMmaQ4K(const VecQArgs& a, dim3 grid, size_t lds, hipStream_t stream) {
   static bool sized = false;
-  if (!AllowLds(reinterpret_cast<const void*>(&VecQMma<kGlu, TG, MT>), static_cast<int>(kMmaLdsLimit), &sized)) return;
-  hipLaunchKernelGGL((VecQMma<kGlu, TG, MT>), grid, dim3(kMmaGroup), lds, stream, a, balanced);
+  if (!AllowLds(reinterpret_cast<const void*>(&VecQMma<kGlu, TG, MT, kSorted>), static_cast<int>(kMmaLdsLimit), &sized)) return;
+  hipLaunchKernelGGL((VecQMma<kGlu, TG, MT, kSorted>), grid, dim3(kMmaGroup), lds, stream, a);
 }
 
-template <bool kGlu>
-void LaunchMmaQ4KShape(const MmaShape& shape, const VecQArgs& a, dim3 grid, int balanced, hipStream_t stream) {
-  if constexpr (!kGlu) {
-    if (shape.groups == 4) return LaunchMmaQ4K<kGlu, 4, 16>(a, grid, shape.lds, balanced, stream);
+template <bool kGlu, bool kSorted>
+void LaunchMmaQ4KShape(const MmaShape& shape, const VecQArgs& a, dim3 grid, hipStream_t stream) {
+  if constexpr (!kSorted) {
+    if constexpr (!kGlu) {
+      if (shape.groups == 4) return LaunchMmaQ4K<kGlu, 4, 16, false>(a, grid, shape.lds, stream);
+    }
+    if (shape.groups == 2) return LaunchMmaQ4K<kGlu, 2, 16, false>(a, grid, shape.lds, stream);
+    if (shape.tokens == 4) return LaunchMmaQ4K<kGlu, 1, 4, false>(a, grid, shape.lds, stream);
   }
-  if (shape.groups == 2) return LaunchMmaQ4K<kGlu, 2, 16>(a, grid, shape.lds, balanced, stream);
-  if (shape.tokens == 16) return LaunchMmaQ4K<kGlu, 1, 16>(a, grid, shape.lds, balanced, stream);
-  if (shape.tokens == 8) return LaunchMmaQ4K<kGlu, 1, 8>(a, grid, shape.lds, balanced, stream);
-  return LaunchMmaQ4K<kGlu, 1, 4>(a, grid, shape.lds, balanced, stream);
+  if (shape.tokens == 16) return LaunchMmaQ4K<kGlu, 1, 16, kSorted>(a, grid, shape.lds, stream);
+  return LaunchMmaQ4K<kGlu, 1, 8, kSorted>(a, grid, shape.lds, stream);
 }
 
 }  // namespace
@@ -891,8 +882,11 @@ void LaunchMma(int type, const VecQArgs& a, hipStream_t stream) {
     const int cus = llmp_hip_compute_units();
     g_mma_compute_units = cus > 0 ? cus : 256;
   }
-  // Sorted Q4_K rows of up to eight super-blocks: the 32 x 32 form, which was the faster at every count of rows an expert
-  // from 2 to 128 (2048 -> 2 x 768, 128 experts: 66 -> 59, 91 -> 68, 125 -> 95 us at 2, 16 and 32 rows).
+  // Sorted Q4_K rows of up to eight super-blocks: the 32 x 32 form (2048 -> 2 x 768, 128 experts: 66 -> 59, 91 -> 68, 125 -> 95
+  // us at 2, 16 and 32 rows an expert; 0.78 of this form's time over 44 shapes of 256 to 2048 values, 1 to 256 experts and 0.2
+  // to 128 rows an expert). Slower where 128 experts and more have up to 512 rows each (with a GLU 256) and about four tokens:
+  // a workgroup's share is then a piece of two experts, each with its start (2048 -> 256 of 128 experts 17.5 -> 19.5 us at one
+  // token an expert, 18.9 -> 27.9 at four, 33.9 -> 22.7 at sixteen). The tokens an expert has are not known here.
   if (a.offsets != nullptr && SortedTakes(type, d)) return LaunchSorted(a, g_mma_compute_units, stream);
   const int slots = a.offsets != nullptr ? d.used : d.ids != nullptr ? d.used * d.tokens : d.used;
   const int tiles = (d.nrows + 15) / 16;
@@ -909,15 +903,15 @@ void LaunchMma(int type, const VecQArgs& a, hipStream_t stream) {
     glu ? LaunchMmaQ8<true>(a, grid, lds, stream) : LaunchMmaQ8<false>(a, grid, lds, stream);
     return;
   }
-  // A slot's tokens: a dense or grouped product's own; sorted rows bring any number an expert, a
-  // routed product up to all its pairs.
-  const int tokens = a.offsets != nullptr ? 64 : d.ids != nullptr ? d.used * d.tokens : d.tokens;
-  const MmaShape shape = ShapeFor(nsb, tokens, glu);
-  // Sorted rows: one workgroup a compute unit, the passes of all experts shared among them evenly.
-  const int balanced = a.offsets != nullptr ? 1 : 0;
-  const dim3 shared_grid(static_cast<unsigned>(g_mma_compute_units), 1);
-  glu ? LaunchMmaQ4KShape<true>(shape, a, balanced ? shared_grid : grid, balanced, stream)
-      : LaunchMmaQ4KShape<false>(shape, a, balanced ? shared_grid : grid, balanced, stream);
+  if (a.offsets != nullptr) {  // one workgroup a compute unit, the passes of all experts shared among them evenly
+    const MmaShape shape = ShapeFor(nsb, 16, glu);
+    const dim3 shared_grid(static_cast<unsigned>(g_mma_compute_units), 1);
+    glu ? LaunchMmaQ4KShape<true, true>(shape, a, shared_grid, stream) : LaunchMmaQ4KShape<false, true>(shape, a, shared_grid, stream);
+    return;
+  }
+  // A slot's tokens: a dense or grouped product's own; a routed product up to all its pairs.
+  const MmaShape shape = ShapeFor(nsb, d.ids != nullptr ? d.used * d.tokens : d.tokens, glu);
+  glu ? LaunchMmaQ4KShape<true, false>(shape, a, grid, stream) : LaunchMmaQ4KShape<false, false>(shape, a, grid, stream);
 }
 
 }  // namespace llmp_hip
