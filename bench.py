@@ -130,7 +130,7 @@ PROFILED_TRAFFIC = {
     "mxfp8_gemm_2048x12288x4096": _traffic(93182.8, 49173.6),
     "moe_q4_k_ffn_t1": _traffic(7028.8, 24.0),        # the gate/up launch
     "moe_q4_k_ffn_t16": _traffic(76769.0, 469.8),     # the gate/up launch
-    "moe_q4_k_ffn_t512": _traffic(182457.3, 12338.4),  # the gate/up launch: the experts' tokens once a segment of rows
+    "moe_q4_k_ffn_t512": _traffic(190284.4, 13840.6),  # the gate/up launch: an expert's weights again for rows past 32, its tokens once a segment
     "attn_vec_q8_0_d256_h16_kv8_cells8192_rows1": _traffic(17562.0 + 279.5, 528.0 + 16.0),  # the splits + their combination
     "attn_vec_q4_0_d256_h16_kv8_cells8192_rows1": _traffic(9369.5 + 279.5, 528.0 + 16.0),
     "attn_vec_q8_0_d256_h16_kv8_cells32768_rows1": _traffic(73938.5 + 537.5, 1056.0 + 16.0),

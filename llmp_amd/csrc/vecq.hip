@@ -616,8 +616,8 @@ int DefaultVariant(int type, const llmp_vecq_desc& d, int kp, bool fused) {
 }
 
 // Whether a super-block of 16 rows a wave (vecq_tile16.hip) is the default: nine to sixteen tokens, never the slower of it and
-// what was the default, the 16 x 16 form and the two launches of the row-a-lane form (31 shapes from 256 -> 512 to 28672 ->
-// 8192 at 9, 12 and 16 tokens: 0.21 to 1.00 of their time). Up to eight the row-a-lane form, whose bits a token keeps from two
+// what was the default, the 16 x 16 form and the two launches of the row-a-lane form (30 shapes from 256 -> 512 to 28672 ->
+// 8192 at 9, 12 and 16 tokens: 0.21 to 0.99 of their time). Up to eight the row-a-lane form, whose bits a token keeps from two
 // to eight (beyond, it has this form's, where rows too long for the 16 x 16 form had one form's from two to sixteen): at eight
 // this one is the faster for rows of more than 8192 values (9216 -> 2048 10.6 against 17.6 us), at four mostly not (15360 ->
 // 3840 13.4 against 11.4).
