@@ -460,7 +460,7 @@ __global__ __launch_bounds__(kMmaGroup, 1) void VecQMma(const VecQArgs a) {
 
   if constexpr (kSorted) {
     // Every pass has one token group, and its start costs little beside its tiles' long rows.
-    WalkSortedRows(a.offsets, d.used, groups, MT, [](int) { return 0; }, [](int) { return 1; }, [&](const SortedSegment& seg) {
+    WalkSortedRows<false>(a.offsets, d.used, groups, MT, [](int) { return 0; }, [](int) { return 1; }, [&](const SortedSegment& seg) {
       sorted_first = seg.rows_first;
       run(Segment{seg.expert, seg.first, seg.m, seg.group_first, 1, seg.group_count});
     });
@@ -884,9 +884,7 @@ void LaunchMma(int type, const VecQArgs& a, hipStream_t stream) {
   }
   // Sorted Q4_K rows of up to eight super-blocks: the 32 x 32 form (2048 -> 2 x 768, 128 experts: 66 -> 59, 91 -> 68, 125 -> 95
   // us at 2, 16 and 32 rows an expert; 0.78 of this form's time over 44 shapes of 256 to 2048 values, 1 to 256 experts and 0.2
-  // to 128 rows an expert). Slower where 128 experts and more have up to 512 rows each (with a GLU 256) and about four tokens:
-  // a workgroup's share is then a piece of two experts, each with its start (2048 -> 256 of 128 experts 17.5 -> 19.5 us at one
-  // token an expert, 18.9 -> 27.9 at four, 33.9 -> 22.7 at sixteen). The tokens an expert has are not known here.
+  // to 128 rows an expert).
   if (a.offsets != nullptr && SortedTakes(type, d)) return LaunchSorted(a, g_mma_compute_units, stream);
   const int slots = a.offsets != nullptr ? d.used : d.ids != nullptr ? d.used * d.tokens : d.used;
   const int tiles = (d.nrows + 15) / 16;

@@ -221,9 +221,9 @@ __device__ __forceinline__ void DotStep(const HalfPart& part, int kg, const uint
   }
 }
 
-// grid: a workgroup a compute unit, sharing the passes of all experts (WalkSortedRows); a wave a tile of 32 rows (with a
+// grid: a workgroup a compute unit, sharing the passes of all experts (WalkSortedRows, kWhole too); a wave a tile of 32 rows (with a
 // GLU 16 of each matrix) and all of K, the workgroup's waves consecutive tiles. LDS: the staged tokens, the waves' row scales.
-template <bool kGlu, int TG>
+template <bool kGlu, int TG, bool kWhole>
 __global__ __launch_bounds__(Staged<TG>::kGroup, 1) void VecQSorted(const VecQArgs a) {
   using L = Staged<TG>;
   constexpr int kWaves = L::kWaves, kGroup = L::kGroup;
@@ -393,14 +393,14 @@ __global__ __launch_bounds__(Staged<TG>::kGroup, 1) void VecQSorted(const VecQAr
   // 2048 of 128 experts 49.6 -> 48.3; half as much again is no better.)
   auto cost_of = [nsb](int m) { return nsb * (m <= kTokens ? 5 : 8); };
   auto fixed_of = [nsb](int m) { return 110 + 10 * nsb * (m <= kTokens ? 1 : TG); };
-  WalkSortedRows(a.offsets, d.used, tiles, TG * kTokens, fixed_of, cost_of, run);
+  WalkSortedRows<kWhole>(a.offsets, d.used, tiles, TG * kTokens, fixed_of, cost_of, run);
 }
 
-template <bool kGlu, int TG>
+template <bool kGlu, int TG, bool kWhole>
 void LaunchOne(const VecQArgs& a, int workgroups, hipStream_t stream) {
   static bool sized = false;
-  if (!AllowLds(reinterpret_cast<const void*>(&VecQSorted<kGlu, TG>), static_cast<int>(kLdsMost), &sized)) return;
-  hipLaunchKernelGGL((VecQSorted<kGlu, TG>), dim3(static_cast<unsigned>(workgroups)), dim3(Staged<TG>::kGroup),
+  if (!AllowLds(reinterpret_cast<const void*>(&VecQSorted<kGlu, TG, kWhole>), static_cast<int>(kLdsMost), &sized)) return;
+  hipLaunchKernelGGL((VecQSorted<kGlu, TG, kWhole>), dim3(static_cast<unsigned>(workgroups)), dim3(Staged<TG>::kGroup),
                      Staged<TG>::Bytes(a.d.ncols_x / 256), stream, a);
 }
 
@@ -410,13 +410,21 @@ bool SortedTakes(int type, const llmp_vecq_desc& d) {
   return type == LLMP_TYPE_Q4_K && Staged<1>::Bytes(d.ncols_x / 256) <= kLdsMost;
 }
 
-void LaunchSorted(const VecQArgs& a, int workgroups, hipStream_t stream) {
+template <bool kWhole>
+void LaunchShape(const VecQArgs& a, int workgroups, hipStream_t stream) {
   const bool wide = Staged<2>::Bytes(a.d.ncols_x / 256) <= kLdsMost;
   if (a.d.g != nullptr) {
-    wide ? LaunchOne<true, 2>(a, workgroups, stream) : LaunchOne<true, 1>(a, workgroups, stream);
+    wide ? LaunchOne<true, 2, kWhole>(a, workgroups, stream) : LaunchOne<true, 1, kWhole>(a, workgroups, stream);
   } else {
-    wide ? LaunchOne<false, 2>(a, workgroups, stream) : LaunchOne<false, 1>(a, workgroups, stream);
+    wide ? LaunchOne<false, 2, kWhole>(a, workgroups, stream) : LaunchOne<false, 1, kWhole>(a, workgroups, stream);
   }
+}
+
+void LaunchSorted(const VecQArgs& a, int workgroups, hipStream_t stream) {
+  // Up to sixteen tiles, a wave's one or two, the passes may have workgroups of their own (WalkSortedRows); with more that
+  // evens out too little, and to look for it cost every launch 0.7 to 0.9 us.
+  const int tiles = a.d.g != nullptr ? (a.d.nrows + 15) / 16 : (a.d.nrows + 31) / 32;
+  tiles <= 16 ? LaunchShape<true>(a, workgroups, stream) : LaunchShape<false>(a, workgroups, stream);
 }
 
 }  // namespace llmp_hip

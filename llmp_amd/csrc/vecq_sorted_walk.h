@@ -29,7 +29,13 @@ struct SortedSegment {
 // experts, and from the first expert of the lane whose run reaches into the part on, the wave looks at 64 experts at a time,
 // one a lane. So its start is one trip to memory up to 64 experts and few for thousands. (With a load after the other until
 // the part's first expert: 2048 -> 512, 128 rows of 512 experts 37.6 us.)
-template <typename FixedOf, typename CostOf, typename Run>
+// With kWhole every pass has workgroups of its own: a part that ends within an expert is two starts, and with few groups a
+// second start costs more than the groups it evens out (2048 -> 256 of 128 experts, about 1, 4 and 16 rows each, that is 85,
+// 125 and 128 passes: 20.6 / 29.5 / 22.5 us by the line, 16.0 / 17.0 / 18.8 so; 2048 -> 512 29.9 / 33.8 / 27.8 and 21.0 / 22.1 /
+// 23.4). So up to half as many passes as workgroups. Beyond, a pass may have one workgroup alone: still so up to eight groups, a
+// wave's one (2048 -> 256, 160 passes 30.3 -> 21.7 us), and where more than four fifths of the workgroups have work (2048 -> 512,
+// 243 passes 45.0 -> 35.0; with 160 the line takes 33 and this about 38).
+template <bool kWhole, typename FixedOf, typename CostOf, typename Run>
 __device__ __forceinline__ void WalkSortedRows(const int32_t* __restrict__ offsets, int experts, int groups, int pass,
                                                FixedOf fixed_of, CostOf cost_of, Run run) {
   const int lane = threadIdx.x & (kWave - 1);
@@ -39,14 +45,17 @@ __device__ __forceinline__ void WalkSortedRows(const int32_t* __restrict__ offse
     const int passes = (rows + pass - 1) / pass;
     return (passes - 1) * pass_cost(pass) + pass_cost(rows - (passes - 1) * pass);
   };
+  auto passes_of = [&](int rows) { return (max(rows, 0) + pass - 1) / pass; };
   const int per = (experts + kWave - 1) / kWave;
   const int mine = min(lane * per, experts), after = min(mine + per, experts);
   int64_t cost = 0;
+  int passes = 0;
   int my_first = offsets[mine], my_rows = 0, begin = my_first;
   if (per <= 2) {
     const int end = offsets[min(mine + 1, after)], end2 = per == 2 ? offsets[after] : end;
     my_rows = end - begin;
     cost = expert_cost(my_rows) + expert_cost(end2 - end);
+    if constexpr (kWhole) passes = passes_of(my_rows) + passes_of(end2 - end);
   } else {
     constexpr int kAtOnce = 8;  // offsets on their way at a time
     for (int i0 = 0; i0 < per; i0 += kAtOnce) {
@@ -56,8 +65,38 @@ __device__ __forceinline__ void WalkSortedRows(const int32_t* __restrict__ offse
 #pragma unroll
       for (int u = 0; u < kAtOnce; ++u) {  // (past the run's end: no rows)
         cost += expert_cost(end[u] - begin);
+        if constexpr (kWhole) passes += passes_of(end[u] - begin);
         begin = end[u];
       }
+    }
+  }
+  if constexpr (kWhole) {
+    int through = passes;
+#pragma unroll
+    for (int delta = 1; delta < kWave; delta <<= 1) {
+      const int other = __shfl_up(through, delta, kWave);
+      if (lane >= delta) through += other;
+    }
+    const int all = __builtin_amdgcn_readlane(through, kWave - 1), workgroups = gridDim.x;
+    if (all <= workgroups / 2 || (all <= workgroups && (groups <= 8 || all > workgroups / 5 * 4))) {
+      if (all == 0) return;
+      // Pass p has the workgroups w with floor(w all / workgroups) = p.
+      const int p = static_cast<int>(blockIdx.x) * all / workgroups;
+      const int first = (p * workgroups + all - 1) / all, count = ((p + 1) * workgroups + all - 1) / all - first;
+      const int first_lane = __ffsll(__ballot(through > p)) - 1;
+      int rest = p - __builtin_amdgcn_readlane(through - passes, first_lane);  // passes of its experts ahead of p
+      for (int e = first_lane * per; e < experts; ++e) {
+        const int rows_first = __builtin_amdgcn_readfirstlane(offsets[e]);
+        const int rows = __builtin_amdgcn_readfirstlane(offsets[e + 1]) - rows_first;
+        if (rest < passes_of(rows)) {
+          const int at = static_cast<int>(blockIdx.x) - first;
+          const int g_first = groups * at / count, g_end = groups * (at + 1) / count;
+          if (g_first < g_end) run(SortedSegment{e, rows_first, rest * pass, min(pass, rows - rest * pass), g_first, g_end - g_first});
+          return;
+        }
+        rest -= passes_of(rows);
+      }
+      return;
     }
   }
   int64_t inclusive = cost;

@@ -287,11 +287,13 @@ def test_sorted_q4k_rows_at_the_edges_of_passes_and_tiles(device, k, n, glu):
 
 
 @pytest.mark.parametrize("experts,k,n", [(1, 256, 33), (64, 256, 64), (65, 2304, 96), (129, 512, 40), (130, 256, 1041), (130, 2048, 700),
-                                         (513, 512, 40), (4100, 256, 8), (4100, 2304, 8)])
+                                         (513, 512, 40), (4100, 256, 8), (4100, 2304, 8), (200, 2048, 512), (300, 1024, 250),
+                                         (300, 2048, 500), (400, 256, 512)])
 def test_sorted_q4k_rows_of_few_and_of_thousands_of_experts(device, experts, k, n):
     """The workgroups' shares where a lane of the walk has one expert, two, and runs of more than it reads at a time, most
     experts without rows, the first and the last among them; tiles enough for a wave to have several of a segment, whose
-    tokens are then all staged, and too few for that. Against the oracle, within 1e-5 of the RMS (sums of up to 72 F32 terms
+    tokens are then all staged, and too few for that; few tiles and passes below and above the counts where every pass has
+    workgroups of its own. Against the oracle, within 1e-5 of the RMS (sums of up to 72 F32 terms
     that cancel), and a row's values bit for bit whatever rows stand beside it."""
     g = synth.rng(93 + experts)
     counts = g.choice(np.array([0, 0, 0, 1, 3, 9, 17], dtype=np.int32), size=experts)
